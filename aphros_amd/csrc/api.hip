@@ -167,6 +167,12 @@ int aphpois_launch_info(aphpois* h, int* stencil_blocks, int* stream_blocks, int
   return APHPOIS_OK;
 }
 
+int aphpois_set_resident_wait(aphpois* h, long long ticks) {
+  APH_CHECK_H(h);
+  h->eng.set_pers_wait(ticks);
+  return APHPOIS_OK;
+}
+
 int aphpois_set_tile(aphpois* h, int lx, int bz, int vx, int sm) {
   APH_CHECK_H(h);
   if (lx < 0 || lx > 256 || (lx & (lx - 1)) || bz < 0 || vx < 0 || vx > 4 || sm < 0)

@@ -42,6 +42,8 @@ struct Scalars {
                    // last reliable update; 1 stale (that update folded x^ and
                    // alpha p into x64; the next CG operator leaves x^ alone);
                    // 2 stale, the next operator writes x^ = alpha p_in
+  int pers_fail;   // a resident launch gave up waiting (persist.hip); the state
+                   // is that before the launch
   int zero_start;  // PCG: the start's x64 is zero-filled (the start's
                    // residual is b, with no accumulation pass); cleared by it
 };
@@ -103,6 +105,11 @@ struct SysDev {
   // in that order, bit for bit (a zero row sum assembled face by face): the
   // FP64 residual then forms e0 from the neighbour coefficients it loads
   int e0_sum;
+  int pers;  // 1: its iterations run in resident launches (persist.hip); the
+             // iteration kernels pass it by
+  // boundary rows that resident launches exchange: r (CONJUGATE in qq, PCG in
+  // q) or the iterates of even and odd sweeps (JACOBI)
+  void* halo[2];
   // workgroups of this system in the stencil, streaming and residual
   // launches (= number of partials each finalize kernel reads)
   int nblk_st, nblk_sm, nblk_ru;

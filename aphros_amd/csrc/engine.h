@@ -18,6 +18,7 @@
 #include "../../include/aphpois.h"
 #include "common.h"
 #include "kernels.h"
+#include "persist.h"
 
 namespace aph {
 
@@ -49,6 +50,11 @@ struct System {
   bool active = false;  // takes part in the next solve
   bool have_x = false;  // x64/u holds a previous solution (warm start)
   int tune_lx = 0, tune_bz = 0;  // stencil tile of this system (0 = engine default)
+  bool pers_ok = false;          // may run in resident launches, as pers says
+  PersPlan pers{};
+  // their gather slots and, for JACOBI, a second buffer of boundary rows
+  // (outside the budget, as the reduction scratch is)
+  unsigned long long* slots = nullptr;
   // multigrid levels (host copy; device copy in d_lev)
   std::vector<MgLevel> lev;
   MgLevel* d_lev = nullptr;
@@ -146,6 +152,8 @@ class Engine {
   // z = M r with the multigrid preconditioner of the resident system (dense
   // host arrays, x fastest); leaves any solve state of the slot as it was.
   int precond_apply(int slot, const double* r, double* z);
+  // Ticks (100 MHz) that a resident launch's workgroups wait for each other
+  void set_pers_wait(long long ticks) { pers_wait_ = ticks; }
   long long bytes() const;
   int nslots() const { return (int)slots_.size(); }
   System* sys(int slot) {
@@ -194,6 +202,9 @@ class Engine {
   int alloc(System& s, void** p, long long bytes);
   int build_tables();
   int capture();
+  bool use_pers(const System& s) const;
+  int advance_pers(int iters);
+  int pers_fallback(bool* failed);
   int pull_scalars();
   int run_pending_ru();
   void fill_info(int slot, double seconds);
@@ -238,6 +249,19 @@ class Engine {
   LaunchSet L_{};
   std::vector<int> launch_slots_;
   bool dirty_ = true;
+  // resident launches: one per group of systems with the same kernel instance
+  struct PersGroup {
+    int shape, has_m, lds, nblk;
+    const PersRec* recs;
+    const int* b2r;
+  };
+  std::vector<PersGroup> pers_groups_;
+  void* d_pers_ = nullptr;   // their records and workgroup maps
+  unsigned pers_tag_ = 1;    // first tag of the next resident launch
+  bool need_graph_ = false;  // some system of the tables is not resident
+  int pers_cu_ = 0;          // compute units resident launches may count on
+  bool pers_off_ = false;    // a resident launch failed: iteration kernels only
+  long long pers_wait_ = kPersWait;
   hipGraphExec_t gexec_ = nullptr;
   hipGraph_t graph_ = nullptr;
   int graph_k_ = 0;

@@ -60,6 +60,11 @@ constexpr long long kFuseMinCells = 1LL << 24;
 // halos (4.5x the level's bytes) miss L2 and the tiles took 37 + 38 us
 // against 22 + 22 us, so 128^3 keeps the sweeps.
 constexpr long long kTileMaxCells = 1LL << 18;
+// Iterations of one resident launch: a launch costs about 30 us more than its
+// iterations (of 7 to 25 us); the server's steps are shorter, so that a new
+// request waits a few milliseconds at most.
+constexpr int kPersRunIters = 512;
+constexpr int kPersStepIters = 128;
 
 bool make_post_rec(int nx, int ny, int nz, int vx, int ncu, Rec* out) {
   const long long n = (long long)nx * ny * nz;
@@ -159,6 +164,7 @@ Engine::~Engine() {
   if (d_sds_) (void)hipFree(d_sds_);
   if (d_rec_) (void)hipFree(d_rec_);
   if (d_b2r_) (void)hipFree(d_b2r_);
+  if (d_pers_) (void)hipFree(d_pers_);
   if (staging_) (void)hipFree(staging_);
   release(staging_bytes_);
   if (d_flags_) (void)hipFree(d_flags_);
@@ -189,6 +195,7 @@ int Engine::init(int device, int method, int precision, int resmode, double tol,
   device_ = device;
   APH_HIP(hipSetDevice(device_));
   APH_HIP(hipDeviceGetAttribute(&ncu_, hipDeviceAttributeMultiprocessorCount, device_));
+  pers_cu_ = pers_units(device_);
   method_ = method;
   fp32_ = precision == 1;
   if (precond < 0 || precond > 1) return fail(APHPOIS_EINVAL, "unknown preconditioner");
@@ -277,6 +284,8 @@ void Engine::free_system(System& s) {
   if (s.partials) (void)hipFree(s.partials);
   s.partials = nullptr;
   s.partials_cap = 0;
+  if (s.slots) (void)hipFree(s.slots);
+  s.slots = nullptr;
 }
 
 int Engine::add_system(int nx, int ny, int nz, double h3, int* slot) {
@@ -501,6 +510,30 @@ int Engine::add_system(int nx, int ny, int nz, double h3, int* slot) {
     S.dev.qq = (double*)q;
   }
   (void)p;
+  S.pers_ok = !pc_ && pers_plan(method_, fp32_, nx, ny, nz, pers_cu_, &S.pers);
+  if (S.pers_ok) {
+    hipError_t e = hipMalloc((void**)&S.slots,
+                             (size_t)(kPersSlotBytes + (method_ == kJacobi ? 8 * n : 0)));
+    if (e == hipSuccess) {
+      e = launch_fill(S.slots, kPersSlotBytes / 8, 8, st_);
+      if (e == hipSuccess) e = hipStreamSynchronize(st_);
+    } else {
+      S.slots = nullptr;
+    }
+    if (e != hipSuccess) {
+      free_system(S);
+      slots_[id].reset();
+      return hip(e, "gather slots");
+    }
+    if (method_ == kPcg) {
+      S.dev.halo[0] = S.dev.q;
+    } else if (method_ == kConjugate) {
+      S.dev.halo[0] = S.dev.qq;
+    } else {
+      S.dev.halo[0] = S.dev.u[1];
+      S.dev.halo[1] = (char*)S.slots + kPersSlotBytes;
+    }
+  }
   slots_[id] = std::move(s);
   dirty_ = true;
   *slot = id;
@@ -839,6 +872,51 @@ int Engine::prepare(int slot, const double* x0, bool on_device, long long start,
   return APHPOIS_OK;
 }
 
+// Whether a system's iterations run in resident launches: a property of the
+// system and of the measurement hooks (event timing and tile overrides address
+// the iteration kernels), so its results do not depend on its neighbours.
+bool Engine::use_pers(const System& s) const {
+  return s.pers_ok && !pers_off_ && !profile_ && tuning_.lx == 0 && tuning_.bz == 0 && tuning_.vx == 0 &&
+         tuning_.sm == 0 && s.tune_lx == 0 && s.tune_bz == 0;
+}
+
+// Up to `iters` more iterations of every resident system of the tables.
+int Engine::advance_pers(int iters) {
+  for (const PersGroup& g : pers_groups_) {
+    if (pers_tag_ > 0xffffffffu - 2u * (unsigned)iters - 4u) {
+      // the tags start over: no slot may hold one of them
+      for (auto& s : slots_) {
+        if (s && s->slots) APH_HIP(launch_fill(s->slots, kPersSlotBytes / 8, 8, st_));
+      }
+      pers_tag_ = 1;
+    }
+    APH_HIP(launch_pers(method_, fp32_, g.has_m, g.shape, g.lds, L_.sds, g.recs, g.b2r, g.nblk,
+                        iters, pers_tag_, pers_wait_, st_));
+    pers_tag_ += 2u * (unsigned)iters + 2u;
+  }
+  return APHPOIS_OK;
+}
+
+// After the scalars were read: if some resident launch gave up (its systems
+// then hold the state before it), the engine goes on with the iteration
+// kernels, from here on for good.
+int Engine::pers_fallback(bool* failed) {
+  *failed = false;
+  for (int i : launch_slots_) *failed = *failed || h_sc_[i].pers_fail;
+  if (!*failed) return APHPOIS_OK;
+  for (int i : launch_slots_) {
+    if (!h_sc_[i].pers_fail) continue;
+    h_sc_[i].pers_fail = 0;
+    APH_HIP(hipMemcpyAsync(d_sc_ + i, h_sc_ + i, sizeof(Scalars), hipMemcpyHostToDevice, st_));
+  }
+  pers_off_ = true;
+  std::unique_lock<std::mutex> lk;
+  if (api_mu_) lk = std::unique_lock<std::mutex>(*api_mu_);
+  APH_HIP(hipStreamSynchronize(st_));
+  APH_TRY(build_tables());
+  return capture();
+}
+
 int Engine::build_tables() {
   launch_slots_.clear();
   bool all4 = true, all2 = true;
@@ -990,7 +1068,59 @@ int Engine::build_tables() {
     s.dev.nblk_st = a.nblk;
     s.dev.nblk_sm = b.nblk;
     s.dev.nblk_ru = c.nblk;
+    s.dev.pers = use_pers(s) ? 1 : 0;
     sds.push_back(s.dev);
+  }
+  // resident launches: systems of one kernel instance share a launch as long
+  // as every workgroup can have a compute unit
+  pers_groups_.clear();
+  need_graph_ = false;
+  std::vector<std::vector<PersRec>> prec;
+  for (int k = 0; k < ns; ++k) {
+    System& s = *slots_[launch_slots_[k]];
+    if (!s.dev.pers) {
+      need_graph_ = true;
+      continue;
+    }
+    const int has_m = method_ == kPcg && s.dev.has_m ? 1 : 0;
+    size_t gi = 0;
+    for (; gi < pers_groups_.size(); ++gi) {
+      const PersGroup& g = pers_groups_[gi];
+      if (g.shape == s.pers.shape && g.has_m == has_m &&
+          g.nblk + s.pers.nblk <= std::min(pers_cu_, kPersMaxBlocks))
+        break;
+    }
+    if (gi == pers_groups_.size()) {
+      pers_groups_.push_back({s.pers.shape, has_m, 0, 0, nullptr, nullptr});
+      prec.emplace_back();
+    }
+    PersGroup& g = pers_groups_[gi];
+    prec[gi].push_back({k, g.nblk, s.pers.nblk, s.pers.by, s.pers.bz, s.pers.py, s.slots});
+    g.nblk += s.pers.nblk;
+    g.lds = std::max(g.lds, s.pers.lds);
+  }
+  if (d_pers_) APH_HIP(hipFree(d_pers_));
+  d_pers_ = nullptr;
+  if (!pers_groups_.empty()) {
+    std::vector<PersRec> all;
+    std::vector<int> map;
+    std::vector<size_t> r0, m0;
+    for (size_t gi = 0; gi < pers_groups_.size(); ++gi) {
+      r0.push_back(all.size());
+      m0.push_back(map.size());
+      for (size_t i = 0; i < prec[gi].size(); ++i)
+        map.insert(map.end(), prec[gi][i].nblk, (int)i);
+      all.insert(all.end(), prec[gi].begin(), prec[gi].end());
+    }
+    const size_t rbytes = all.size() * sizeof(PersRec);
+    APH_HIP(hipMalloc(&d_pers_, rbytes + map.size() * sizeof(int)));
+    int* dmap = (int*)((char*)d_pers_ + rbytes);
+    APH_HIP(hipMemcpy(d_pers_, all.data(), rbytes, hipMemcpyHostToDevice));
+    APH_HIP(hipMemcpy(dmap, map.data(), map.size() * sizeof(int), hipMemcpyHostToDevice));
+    for (size_t gi = 0; gi < pers_groups_.size(); ++gi) {
+      pers_groups_[gi].recs = (const PersRec*)d_pers_ + r0[gi];
+      pers_groups_[gi].b2r = dmap + m0[gi];
+    }
   }
   // device tables in one buffer each
   long long nrec = (long long)rst.size() + rsm.size() + rru.size();
@@ -1285,7 +1415,7 @@ int Engine::step(int max_replays, std::vector<int>* finished) {
     std::unique_lock<std::mutex> lk;
     if (api_mu_) lk = std::unique_lock<std::mutex>(*api_mu_);
     APH_TRY(build_tables());
-    APH_TRY(capture());
+    if (need_graph_) APH_TRY(capture());
   }
   if (need_start_) {
     // reliable-update kernels: only systems prepared since the last call
@@ -1294,8 +1424,16 @@ int Engine::step(int max_replays, std::vector<int>* finished) {
     need_start_ = false;
   }
   for (int r = 0; r < max_replays && finished->empty(); ++r) {
-    APH_HIP(hipGraphLaunch(gexec_, st_));
+    if (need_graph_) APH_HIP(hipGraphLaunch(gexec_, st_));
+    if (!pers_groups_.empty()) {
+      std::unique_lock<std::mutex> lk;
+      if (api_mu_) lk = std::unique_lock<std::mutex>(*api_mu_);
+      APH_TRY(advance_pers(kPersStepIters));
+    }
     APH_TRY(pull_scalars());
+    bool failed = false;
+    APH_TRY(pers_fallback(&failed));
+    if (failed) continue;
     APH_TRY(run_pending_ru());
     bool alldone = true;
     for (int i : launch_slots_) {
@@ -1320,8 +1458,9 @@ int Engine::run() {
   if (!any) return APHPOIS_OK;
   if (dirty_) {
     APH_TRY(build_tables());
-    APH_TRY(capture());
+    if (need_graph_) APH_TRY(capture());
   }
+  if (!need_graph_) graph_k_ = 1;
   APH_HIP(hipEventRecord(ev0_, st_));
   APH_HIP(launch_start(method_, fp32_, vx_, L_, st_));
   // a replay may end with a system idle until its reliable update (graph
@@ -1378,11 +1517,23 @@ int Engine::run() {
       }
       APH_HIP(hipEventRecord(pev_[(size_t)graph_k_ * nk], st_));
     } else {
-      APH_HIP(hipGraphLaunch(gexec_, st_));
+      if (need_graph_) APH_HIP(hipGraphLaunch(gexec_, st_));
+      APH_TRY(advance_pers(kPersRunIters));
+      if (method_ == kPcg && !pers_groups_.empty()) {
+        // a resident launch ends at a reliable update: apply it and go on
+        // before the host looks at the scalars
+        APH_HIP(launch_start(method_, fp32_, vx_, L_, st_));
+        APH_TRY(advance_pers(kPersRunIters));
+      }
     }
     ++loops;
     APH_TRY(pull_scalars());
-    if (!profile_) APH_TRY(run_pending_ru());
+    if (!profile_) {
+      bool failed = false;
+      APH_TRY(pers_fallback(&failed));
+      if (failed) continue;
+      APH_TRY(run_pending_ru());
+    }
     alldone = true;
     int iters_after = 0;
     for (int i : launch_slots_) {

@@ -275,7 +275,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const SysDev* __restrict__ 
   const Rec rc = recs[b2r[b]];
   const SysDev& s = sds[rc.sys];
   Scalars* sc = s.sc;
-  if (sc->done || sc->ru) return;  // ru: a reliable update is pending
+  if (sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
   const int lb = b - rc.blk0;
   const Tile t = tile_of<VX>(rc, s, lb);
   const int nx = s.nx, ny = s.ny, nz = s.nz;
@@ -428,7 +428,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const SysDev* __restrict__ 
 __global__ __launch_bounds__(kBlock) void k_fin_pcg_spmv(const SysDev* __restrict__ sds) {
   const SysDev& s = sds[blockIdx.x];
   Scalars* sc = s.sc;
-  if (sc->done || sc->ru) return;  // ru: a reliable update is pending
+  if (sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
   double acc[1];
   reduce_partials<1, 0u>(acc, s.partials, s.nblk_st);
   if (threadIdx.x == 0) {
@@ -468,7 +468,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update(const SysDev* __restrict_
   const Rec rc = recs[b2r[b]];
   const SysDev& s = sds[rc.sys];
   Scalars* sc = s.sc;
-  if (sc->done || sc->ru) return;  // ru: a reliable update is pending
+  if (sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
   const int lb = b - rc.blk0;
   const double alpha = sc->alpha;
   const T* __restrict__ q = (const T*)s.q;
@@ -488,7 +488,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update(const SysDev* __restrict_
 __global__ __launch_bounds__(kBlock) void k_fin_pcg_update(const SysDev* __restrict__ sds) {
   const SysDev& s = sds[blockIdx.x];
   Scalars* sc = s.sc;
-  if (sc->done || sc->ru) return;  // ru: a reliable update is pending
+  if (sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
   double acc[1];
   reduce_partials<1, 0u>(acc, s.partials, s.nblk_sm);
   if (threadIdx.x == 0) {

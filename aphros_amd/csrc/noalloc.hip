@@ -4,7 +4,8 @@
 // aphpois_set_system_device + aphpois_solve_device, with every buffer beyond
 // the caller's Expr and solution in one file-scope device array (`scratch`):
 // the system table, the scalars, the launch records, the block -> record map,
-// the reduction partials, the check flags and the work vectors.  The Expr is
+// the reduction partials, the gather slots of the resident launches, the
+// check flags and the work vectors.  The Expr is
 // read in place (component k of cell c at expr[8 c + k]).  No hipMalloc,
 // hipFree, stream, event or graph is created.
 //
@@ -39,6 +40,7 @@ struct NaHeader {
   SysDev sd;
   Scalars sc;
   Rec rec[3];  // stencil, streaming, one-cell-per-thread launches
+  PersRec prec;  // resident launch
   unsigned flags;
 };
 
@@ -46,7 +48,8 @@ constexpr long long al256(long long b) { return (b + 255) & ~255LL; }
 constexpr long long kOfsHdr = 0;
 constexpr long long kOfsB2r = al256(sizeof(NaHeader));
 constexpr long long kOfsPart = kOfsB2r + al256(4 * kNaMaxBlocks);
-constexpr long long kOfsVec = kOfsPart + al256(3 * 8 * kNaMaxBlocks);
+constexpr long long kOfsSlots = kOfsPart + al256(3 * 8 * kNaMaxBlocks);
+constexpr long long kOfsVec = kOfsSlots + al256(kPersSlotBytes);
 constexpr long long kScratchBytes = kOfsVec + kNaVecs * 8 * kNaMaxCells;
 
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
@@ -72,6 +75,17 @@ __global__ __launch_bounds__(kBlock) void k_na_copy(const double* __restrict__ s
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;
 unsigned char* g_ptr[kMaxDevices] = {};
+unsigned g_tag[kMaxDevices] = {};  // last tag the device's gather slots have seen
+
+// The first of `count` tags for the gather slots of a device; *restart: the
+// tags start over and the slots have to be cleared first.
+unsigned take_tags(int device, unsigned count, bool* restart) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  *restart = g_tag[device] > 0xffffffffu - count - 1;
+  const unsigned first = *restart ? 1 : g_tag[device] + 1;
+  g_tag[device] = first + count;
+  return first;
+}
 
 // Address of `scratch` on the current device (taken once per device).
 int scratch_ptr(int device, unsigned char** out) {
@@ -149,6 +163,8 @@ int solve_noalloc(const aphpois_desc* d, const double* expr, const double* x0, d
   s.pp[0] = vec + n;
   s.pp[1] = vec + 2 * n;
   s.qq = vec + 3 * n;
+  s.halo[0] = method == kConjugate ? s.qq : s.u[1];
+  s.halo[1] = vec + n;  // JACOBI
   s.partials = (double*)(base + kOfsPart);
   s.sc = &dh->sc;
   s.nblk_st = rst.nblk;
@@ -166,9 +182,14 @@ int solve_noalloc(const aphpois_desc* d, const double* expr, const double* x0, d
   h.rec[0] = rst;
   h.rec[1] = rsm;
   h.rec[2] = rru;
+  PersPlan plan;
+  bool pers = pers_plan(method, 0, d->nx, d->ny, d->nz, pers_units(d->device), &plan);
+  unsigned long long* slots = (unsigned long long*)(base + kOfsSlots);
+  if (pers) h.prec = {0, 0, plan.nblk, plan.by, plan.bz, plan.py, slots};
 
   const auto t0 = std::chrono::steady_clock::now();
-  hipLaunchKernelGGL(k_na_setup, dim3(grid_of(nb)), dim3(kBlock), 0, st, h, base, nb);
+  const int nmap = std::max(nb, kPersMaxBlocks);
+  hipLaunchKernelGGL(k_na_setup, dim3(grid_of(nmap)), dim3(kBlock), 0, st, h, base, nmap);
   NA_HIP(hipGetLastError());
   NA_HIP(launch_check(expr, 0, d->nx, (long long)d->nx * d->ny, d->nx, d->ny, d->nz,
                       &dh->flags, st));
@@ -204,11 +225,26 @@ int solve_noalloc(const aphpois_desc* d, const double* expr, const double* x0, d
   const int maxloops = (std::max(d->maxiter, d->miniter) + 1) / k + 4;
   Scalars hs;
   for (int loop = 0;; ++loop) {
-    for (int i = 0; i < k; ++i) {
+    if (pers) {
+      const int iters = 512;
+      bool restart = false;
+      const unsigned tag = take_tags(d->device, 2u * iters + 2u, &restart);
+      if (restart) NA_HIP(launch_fill(slots, kPersSlotBytes / 8, 8, st));
+      NA_HIP(launch_pers(method, 0, 0, plan.shape, plan.lds, L.sds, &dh->prec, b2r, plan.nblk, iters,
+                         tag, kPersWait, st));
+    }
+    for (int i = 0; i < k && !pers; ++i) {
       for (int j = 0; j < iter_kernels(method); ++j) NA_HIP(launch_kernel(method, 0, 1, L, st, j));
     }
     NA_HIP(hipMemcpyAsync(&hs, &dh->sc, sizeof(hs), hipMemcpyDeviceToHost, st));
     NA_HIP(hipStreamSynchronize(st));
+    if (hs.pers_fail) {
+      // the resident launch gave up and left the state as it was
+      hs.pers_fail = 0;
+      NA_HIP(hipMemcpyAsync(&dh->sc, &hs, sizeof(hs), hipMemcpyHostToDevice, st));
+      pers = false;
+      continue;
+    }
     if (hs.done) break;
     if (loop > maxloops)
       return set_api_error(APHPOIS_EDEVICE, "solver did not terminate within maxiter");

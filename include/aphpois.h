@@ -286,6 +286,13 @@ int aphpois_launch_info(aphpois* h, int* stencil_blocks, int* stream_blocks, int
  * thread in x (1, 2 or 4; 4 only in MIXED; must divide nx), sm cells per
  * thread of the streaming kernels. */
 int aphpois_set_tile(aphpois* h, int lx, int bz, int vx, int sm);
+/* How long (ticks of a 100 MHz counter; default 2 s) the workgroups of a
+ * resident launch wait for each other before the solve goes on with one
+ * launch per iteration kernel.  Systems of at most 2^21 cells without the
+ * multigrid preconditioner run their iterations in such launches, unless
+ * set_profiling or set_tile address the iteration kernels.  Negative: they
+ * give up at once. */
+int aphpois_set_resident_wait(aphpois* h, long long ticks);
 /* Practical HBM bandwidth of a plain streaming copy kernel on `device`:
  * copies `bytes` (two buffers of that size are allocated and freed) `reps`
  * times after one warm-up copy; *gbps = 2 * bytes * reps / time. */
