@@ -47,11 +47,19 @@ Rec make_stencil_rec(int nx, int ny, int nz, int vx, int blocks_target, const Tu
 // Fused pre-smoothing + restriction (k_mg_pre) and post-smoothing (k_mg_post)
 // of a level: whole-row tiles of lx = nx / vx threads per row and
 // ty = min(kPostBlock / lx, ny + 2) rows of threads (even; ty - 2 output
-// rows), bz planes (even).  Only for the large levels (n >= 2^24 cells: the
-// march is long enough to hide the halo rows and planes it recomputes; such a
-// level coarsens, so its edges are even) whose rows fit 1/8 of the workgroup
-// (ty >= 8 rows).
-constexpr long long kFuseMinCells = 1LL << 24;
+// rows), bz planes (even).  Only for the large levels (the march is long
+// enough to hide the halo rows and planes it recomputes; such a level
+// coarsens, so its edges are even) whose rows fit 1/8 of the workgroup (ty >=
+// 8 rows).
+//
+// From 2^19 cells in FP64 and 3 x 2^20 in FP32 (ms per solve, four launches
+// -> fused): FP64 96^3 4.3 -> 3.8, 128^3 6.5 -> 5.8, 160^3 12.4 -> 10.4, 192^3
+// 19.9 -> 13.4, 224^3 29.3 -> 19.7; mixed 128 x 96 x 160 8.4 -> 8.5 and batched
+// 128^3 5 % slower, 160^3 7.0 -> 6.0, 192^3 9.6 -> 8.6, 224^3 13.9 -> 11.1, 256
+// x 192 x 128 9.2 -> 7.9: below, the level's bytes are in the caches and the
+// march has too few workgroups.  The planes and rows ahead of a march wrap
+// once: at least 8 of each.
+constexpr long long kFuseMinCells64 = 1LL << 19, kFuseMinCells32 = 3LL << 20;
 // Levels below level 0 of FP32 engines with at most this many cells and
 // nx % 4 == 0 smooth in tile launches (k_mg_tile: one launch and one round of
 // global loads per pre- or post-smoothing instead of two z-marching
@@ -68,7 +76,8 @@ constexpr int kPersStepIters = 128;
 
 bool make_post_rec(int nx, int ny, int nz, int vx, int ncu, Rec* out) {
   const long long n = (long long)nx * ny * nz;
-  if (vx <= 0 || nx % vx != 0 || n < kFuseMinCells) return false;
+  if (vx <= 0 || nx % vx != 0 || ny < 8 || nz < 8) return false;
+  if (n < (vx == 4 ? kFuseMinCells32 : kFuseMinCells64)) return false;
   const int lx = nx / vx;
   if (lx > kPostBlock / 8) return false;
   Rec r{};

@@ -1,0 +1,57 @@
+"""One multigrid cycle against the oracle's at the sizes where a level changes
+its kernels: the smallest fused levels (2^19 cells in FP64, 3 * 2^20 in
+mixed precision), short and long rows, partial row tiles, with and without a mass
+term and W levels."""
+import numpy as np
+import pytest
+
+from aphros_amd import _lib as L
+from aphros_amd.solver import Poisson
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+TOL = {L.FP64: 1e-12, L.MIXED: 1e-4}  # rounding; bfloat16 coefficients restated
+
+
+def _system(shape, seed, mass):
+    rng = np.random.default_rng(seed)
+    rho = np.where(rng.random(shape) < 0.2, 100.0, 1.0)
+    f = rng.standard_normal(shape)
+    e = O.assemble(rho, f - f.mean())
+    if mass:
+        e[..., 0] *= 1.0 + 1e-3 * rng.random(shape)
+    return np.ascontiguousarray(e)
+
+
+def _cycle_error(shape, precision, w, mass, seed=1):
+    e = _system(shape, seed, mass)
+    s = Poisson(shape, method=L.PCG, precision=precision, resmode=L.RES_REL_TRUE, tol=1e-8,
+                maxiter=2000, precond=L.PRECOND_MG, mg_w=w)
+    s.set_system(e)
+    r = np.random.default_rng(seed + 1).standard_normal(shape)
+    if not mass:
+        r -= r.mean()
+    z = s.precond_apply(r)
+    x, info = s.solve(None)
+    s.close()
+    assert info["converged"] == 1 and O.true_relres(e, x) <= 1e-8 * (1 + 1e-6)
+    zo, nlev = O.mg_apply(e, r, bf16=precision == L.MIXED, w=w)
+    err = np.abs(z - zo).max() / np.abs(zo).max()
+    print(shape, precision, w, mass, "levels", nlev, "iter", info["iter"], "err", err, flush=True)
+    return err
+
+
+@pytest.mark.parametrize("mass", [False, True])
+@pytest.mark.parametrize("precision,shape,w", [
+    (L.FP64, (128, 64, 64), 0),       # 2^19 cells
+    (L.FP64, (64, 256, 32), 1),       # rows of 16 threads
+    (L.FP64, (64, 96, 96), 2),        # rows of 48 threads, a partial row tile
+    (L.FP64, (8, 256, 256), 1),       # rows of 128 threads, 8 planes
+    (L.MIXED, (192, 128, 128), 0),    # 3 * 2^20 cells
+    (L.MIXED, (768, 128, 32), 1),     # rows of 8 threads
+    (L.MIXED, (128, 160, 160), 2),    # rows of 40 threads, a partial row tile
+    (L.MIXED, (16, 768, 256), 1),     # rows of 64 threads, 16 planes
+])
+def test_smallest_fused_levels(precision, shape, w, mass):
+    assert _cycle_error(shape, precision, w, mass) <= TOL[precision]
