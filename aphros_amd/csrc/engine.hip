@@ -997,15 +997,10 @@ int Engine::build_tables() {
     if (pc_) {
       const int nl = (int)s.lev.size();
       nlev_max = std::max(nlev_max, nl);
-      // LDS of the bottom kernel (same rule as the kernel: everything
-      // resident if it fits, else z and a second buffer per level)
       const int es = fp32_ ? 4 : 8;
-      long long zbytes = 0, fbytes = 0;
-      for (int l = s.dev.mg_lb; l < nl; ++l) {
-        zbytes += bottom_z_bytes(s.lev[l].n, es);
-        fbytes += bottom_full_bytes(s.lev[l].n, es, s.dev.has_m);
-      }
-      coarse_max = std::max(coarse_max, fbytes <= kBottomLdsMax ? fbytes : zbytes);
+      long long zbytes = 0;
+      for (int l = s.dev.mg_lb; l < nl; ++l) zbytes += bottom_z_bytes(s.lev[l].n, es);
+      coarse_max = std::max(coarse_max, zbytes);
       bottom_at[s.dev.mg_lb] = 1;
       deep = std::max(deep, s.dev.mg_lb);
       for (int l = 0; l < s.dev.mg_lb; ++l) {

@@ -893,46 +893,36 @@ struct LevelView {
   }
 };
 
-// Explicit address spaces for the bottom kernel: its level data sit in LDS
-// (or, for levels too large for it, in global memory) behind generic
-// pointers, which would otherwise compile to flat loads with 64-bit
-// addresses.
+// Explicit address spaces for the bottom kernel, whose pointers into LDS are
+// generic and would otherwise compile to flat accesses with 64-bit addresses.
 template <typename T>
 using lds_cp = const __attribute__((address_space(3))) T*;
 template <typename T>
 using lds_p = __attribute__((address_space(3))) T*;
-template <typename T>
-using glb_cp = const __attribute__((address_space(1))) T*;
-template <typename T>
-using glb_p = __attribute__((address_space(1))) T*;
 
-// A level of the bottom kernel with 32-bit indices: the operator and
-// operation order of LevelView, periodic neighbours from the flat index.
-// CL: coefficients, mass and right-hand side in LDS (else global memory).
-template <typename T, bool CL>
-struct LdsView {
-  template <typename U>
-  using CP = std::conditional_t<CL, lds_cp<U>, glb_cp<U>>;
-  template <typename U>
-  using P = std::conditional_t<CL, lds_p<U>, glb_p<U>>;
+// A coarsest level in global memory with 32-bit indices: the operator and
+// operation order of LevelView, periodic neighbours from the flat index, u in
+// LDS.
+template <typename T>
+struct GlobalView {
   using E = std::conditional_t<sizeof(T) == 4, unsigned short, T>;
   int nx, ny, nz, pl, n;
-  CP<E> a[4];
-  CP<T> m;
+  gcp<E> a[4];
+  gcp<T> m;
   bool hasm;
-  P<T> r;
-  __device__ explicit LdsView(const MgLevel& L)
+  gcp<T> r;
+  __device__ explicit GlobalView(const MgLevel& L)
       : nx(L.nx), ny(L.ny), nz(L.nz), pl(L.nx * L.ny), n((int)L.n), hasm(L.m != nullptr) {
     if constexpr (sizeof(T) == 4) {
-      a[0] = a[1] = a[2] = a[3] = (CP<E>)(const E*)L.kc;
+      a[0] = a[1] = a[2] = a[3] = (gcp<E>)(const E*)L.kc;
     } else {
-      a[0] = (CP<E>)(const E*)L.kx;
-      a[1] = (CP<E>)(const E*)L.ky;
-      a[2] = (CP<E>)(const E*)L.kz;
-      a[3] = (CP<E>)(const E*)L.dinv;
+      a[0] = (gcp<E>)(const E*)L.kx;
+      a[1] = (gcp<E>)(const E*)L.ky;
+      a[2] = (gcp<E>)(const E*)L.kz;
+      a[3] = (gcp<E>)(const E*)L.dinv;
     }
-    m = hasm ? (CP<T>)(const T*)L.m : CP<T>{};
-    r = (P<T>)(T*)L.r;
+    m = hasm ? (gcp<T>)(const T*)L.m : gcp<T>{};
+    r = (gcp<T>)(const T*)L.r;
   }
   __device__ T k(int c, int i) const {
     if constexpr (sizeof(T) == 4) {
@@ -2286,7 +2276,8 @@ struct WaveLevel {
   int n;
   int nb[6];  // lanes of the xm, xp, ym, yp, zm, zp neighbours
   T kx, kxm, ky, kym, kz, kzm, d, m;
-  __device__ void load(const MgLevel& L, int lane) {
+  // k: kx, ky, kz, D^-1 and mass term of the level's cells (LDS)
+  __device__ void load(const MgLevel& L, const T (*k)[64], int lane) {
     n = (int)L.n;
     const bool on = lane < n;
     const int c = on ? lane : 0;
@@ -2298,15 +2289,14 @@ struct WaveLevel {
     nb[3] = on ? c + (wrapp(y, L.ny) - y) * L.nx : lane;
     nb[4] = on ? c + (wrapm(z, L.nz) - z) * pl : lane;
     nb[5] = on ? c + (wrapp(z, L.nz) - z) * pl : lane;
-    const MgCoefs<T> co(L);
-    kx = on ? co.comp1(0, c) : (T)0;
-    kxm = on ? co.comp1(0, nb[0]) : (T)0;
-    ky = on ? co.comp1(1, c) : (T)0;
-    kym = on ? co.comp1(1, nb[2]) : (T)0;
-    kz = on ? co.comp1(2, c) : (T)0;
-    kzm = on ? co.comp1(2, nb[4]) : (T)0;
-    d = on ? co.comp1(3, c) : (T)0;
-    m = (on && L.m) ? ((const T*)L.m)[c] : (T)0;
+    kx = on ? k[0][c] : (T)0;
+    kxm = on ? k[0][nb[0]] : (T)0;
+    ky = on ? k[1][c] : (T)0;
+    kym = on ? k[1][nb[2]] : (T)0;
+    kz = on ? k[2][c] : (T)0;
+    kzm = on ? k[2][nb[4]] : (T)0;
+    d = on ? k[3][c] : (T)0;
+    m = on ? k[4][c] : (T)0;
   }
   // (L u) of this lane's cell; every lane of the wavefront must call it
   __device__ T lap(T u) const {
@@ -2319,351 +2309,443 @@ struct WaveLevel {
   }
 };
 
-// The bottom of the cycle: levels lb..top of a system (its cycle from level
-// lb down; lb > every W level) in one workgroup.  Levels of more than 64
-// cells: z and a second buffer of every level in LDS and, when they fit
-// (bottom_full_bytes), the levels' coefficients, mass and right-hand sides
-// too (copied in once; the restriction then writes the coarse right-hand
-// sides to LDS), barriers between the steps; the last one or two levels of at
-// most 64 cells: one wavefront, a cell per lane.  The same operations as the
-// per-level launches: zero-guess sweep + sweep, restriction, `sweeps` damped
-// Jacobi sweeps from zero on the coarsest level, prolongation + sweep + sweep;
-// the correction of level lb goes to its z[1] (z[0] when lb is the coarsest).
-// Each system takes part only in the launch for its own lb (s.mg_lb == l0).
-// The engine chooses lb so that the levels fit in LDS.
-constexpr int kBottomThreads = 1024;
+constexpr int kBottomThreads = 512;
 
+// The cells of a bottom level that one thread of the workgroup owns, NV at
+// most: operator, right-hand side and iterate in registers for the whole
+// visit; the stencil's neighbours come from a copy of the iterate in LDS.
+// VEC (FP32, nx % 4 == 0): groups of four consecutive cells of a row (the
+// packed coefficients of a group in two 16-byte loads, neighbouring rows in
+// 16-byte LDS reads), the groups tid + 512 j; otherwise the cells tid + 512 v.
+template <typename T, int NV, bool VEC>
+struct BottomCells {
+  static_assert(!VEC || (sizeof(T) == 4 && NV % 4 == 0), "groups of packed coefficients");
+  using V4 = vec_t<float, 4>;
+  using U4 = vec_t<unsigned, 4>;
+  using U2 = vec_t<unsigned, 2>;
+  int n, nx, ny, nz, pl;
+  int c[NV];    // cell (cell 0 for a slot without one)
+  int edge[NV]; // bits 0..5: it lies on the x-, x+, y-, y+, z-, z+ side of the
+                // level; < 0: no cell
+  int par[NV];  // the coarse cell it belongs to
+  int kid[NV];  // its first child on the finer level
+  T kx[NV], kw[NV], ky[NV], ks[NV], kz[NV], kb[NV];  // plus and minus faces
+  T d[NV], m[NV], r[NV], z[NV];
+
+  __device__ __forceinline__ int xm(int v) const {
+    return c[v] + ((edge[v] & 1) ? nx - 1 : -1);
+  }
+  __device__ __forceinline__ int xp(int v) const {
+    return c[v] + ((edge[v] & 2) ? 1 - nx : 1);
+  }
+  __device__ __forceinline__ int ym(int v) const {
+    return c[v] + ((edge[v] & 4) ? pl - nx : -nx);
+  }
+  __device__ __forceinline__ int yp(int v) const {
+    return c[v] + ((edge[v] & 8) ? nx - pl : nx);
+  }
+  __device__ __forceinline__ int zm(int v) const {
+    return c[v] + ((edge[v] & 16) ? n - pl : -pl);
+  }
+  __device__ __forceinline__ int zp(int v) const {
+    return c[v] + ((edge[v] & 32) ? pl - n : pl);
+  }
+  __device__ __forceinline__ bool on(int v) const { return edge[v] >= 0; }
+
+  // issues the loads of the level's coefficients (and right-hand side)
+  __device__ __forceinline__ void load(const MgLevel& L, bool with_r) {
+    nx = L.nx;
+    ny = L.ny;
+    nz = L.nz;
+    pl = nx * ny;
+    n = (int)L.n;
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int i = VEC ? 4 * (tid + v / 4 * kBottomThreads) + v % 4 : tid + v * kBottomThreads;
+      const bool in = i < n;
+      c[v] = in ? i : 0;
+      const int t = c[v] / nx, x = c[v] - t * nx, zz = t / ny, y = t - zz * ny;
+      edge[v] = (x == 0 ? 1 : 0) | (x == nx - 1 ? 2 : 0) | (y == 0 ? 4 : 0) |
+                (y == ny - 1 ? 8 : 0) | (zz == 0 ? 16 : 0) | (zz == nz - 1 ? 32 : 0) |
+                (in ? 0 : (int)0x80000000);
+      par[v] = ((zz >> 1) * (ny >> 1) + (y >> 1)) * (nx >> 1) + (x >> 1);
+      kid[v] = ((2 * zz) * (2 * ny) + 2 * y) * (2 * nx) + 2 * x;
+      kx[v] = kw[v] = ky[v] = ks[v] = kz[v] = kb[v] = d[v] = m[v] = r[v] = z[v] = (T)0;
+    }
+    const T* mp = (const T*)L.m;
+    const T* rp = (const T*)L.r;
+    if constexpr (VEC) {
+      const gcp<unsigned short> kc = (gcp<unsigned short>)L.kc;
+      constexpr int G = NV / 4;
+      U4 c0[G], c1[G];
+      U2 y2[G], z2[G];
+      unsigned short w0[G];
+      V4 rv[G], mv[G];
+#pragma unroll
+      for (int j = 0; j < G; ++j) {
+        const int i = c[4 * j], ixm = xm(4 * j);
+        const gcp<U4> g = (gcp<U4>)(kc + 4 * i);
+        c0[j] = g[0];
+        c1[j] = g[1];
+        y2[j] = *(gcp<U2>)(kc + 4 * ym(4 * j) + 4);
+        z2[j] = *(gcp<U2>)(kc + 4 * zm(4 * j) + 8);
+        w0[j] = *(gcp<unsigned short>)(kc + 16 * (ixm >> 2) + (ixm & 3));
+        rv[j] = with_r ? *(gcp<V4>)((gcp<float>)rp + i) : (V4)(0.0f);
+        mv[j] = mp ? *(gcp<V4>)((gcp<float>)mp + i) : (V4)(0.0f);
+      }
+#pragma unroll
+      for (int j = 0; j < G; ++j) {
+        const V4 x4 = bf4(c0[j].x, c0[j].y), y4 = bf4(c0[j].z, c0[j].w),
+                 zz4 = bf4(c1[j].x, c1[j].y), d4 = bf4(c1[j].z, c1[j].w),
+                 s4 = bf4(y2[j].x, y2[j].y), b4 = bf4(z2[j].x, z2[j].y);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          kx[4 * j + v] = x4[v];
+          kw[4 * j + v] = v > 0 ? x4[v > 0 ? v - 1 : 0] : bf2f(w0[j]);
+          ky[4 * j + v] = y4[v];
+          ks[4 * j + v] = s4[v];
+          kz[4 * j + v] = zz4[v];
+          kb[4 * j + v] = b4[v];
+          d[4 * j + v] = d4[v];
+          m[4 * j + v] = mv[j][v];
+          r[4 * j + v] = rv[j][v];
+        }
+      }
+    } else {
+      const MgCoefs<T> co(L);
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        if (on(v)) {
+          kx[v] = co.comp1g(0, c[v]);
+          kw[v] = co.comp1g(0, xm(v));
+          ky[v] = co.comp1g(1, c[v]);
+          ks[v] = co.comp1g(1, ym(v));
+          kz[v] = co.comp1g(2, c[v]);
+          kb[v] = co.comp1g(2, zm(v));
+          d[v] = co.comp1g(3, c[v]);
+          if (mp) m[v] = ld1(mp, c[v]);
+          if (with_r) r[v] = ld1(rp, c[v]);
+        }
+      }
+    }
+  }
+  // LDS <- w (the thread's cells)
+  __device__ __forceinline__ void put(T* u_, const T (&w)[NV]) const {
+    const lds_p<T> u = (lds_p<T>)u_;
+    if constexpr (VEC) {
+#pragma unroll
+      for (int j = 0; j < NV; j += 4) {
+        if (on(j)) *(lds_p<V4>)(u + c[j]) = V4{w[j], w[j + 1], w[j + 2], w[j + 3]};
+      }
+    } else {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        if (on(v)) u[c[v]] = w[v];
+      }
+    }
+  }
+  // (L w) of the thread's cells, w in registers and in LDS
+  __device__ __forceinline__ void lap(const T* u_, const T (&w)[NV], T (&l)[NV]) const {
+    const lds_cp<T> u = (lds_cp<T>)u_;
+    if constexpr (VEC) {
+#pragma unroll
+      for (int j = 0; j < NV; j += 4) {
+        if (j > 0 && j * kBottomThreads >= n) break;  // (uniform)
+        const V4 a = *(lds_cp<V4>)(u + ym(j)), b = *(lds_cp<V4>)(u + yp(j));
+        const V4 e = *(lds_cp<V4>)(u + zm(j)), f = *(lds_cp<V4>)(u + zp(j));
+        const float uw = u[xm(j)], ue = u[c[j] + ((edge[j + 3] & 2) ? 4 - nx : 4)];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int i = j + v;
+          const float up = v < 3 ? w[v < 3 ? i + 1 : i] : ue, um = v > 0 ? w[v > 0 ? i - 1 : i] : uw;
+          l[i] = kx[i] * (w[i] - up) + kw[i] * (w[i] - um) + ky[i] * (w[i] - b[v]) +
+                 ks[i] * (w[i] - a[v]) + kz[i] * (w[i] - f[v]) + kb[i] * (w[i] - e[v]);
+          l[i] += m[i] * w[i];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        if (v > 0 && v * kBottomThreads >= n) break;  // (uniform)
+        l[v] = kx[v] * (w[v] - u[xp(v)]) + kw[v] * (w[v] - u[xm(v)]) +
+               ky[v] * (w[v] - u[yp(v)]) + ks[v] * (w[v] - u[ym(v)]) +
+               kz[v] * (w[v] - u[zp(v)]) + kb[v] * (w[v] - u[zm(v)]);
+        l[v] += m[v] * w[v];
+      }
+    }
+  }
+  // z += om D^-1 (r - L z), z put into u first
+  __device__ __forceinline__ void sweep(T* u, T om) {
+    T l[NV] = {};
+    put(u, z);
+    __syncthreads();
+    lap(u, z, l);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) z[v] = z[v] + om * d[v] * (r[v] - l[v]);
+  }
+  // pre-smoothing from zero; the residual is left in u0
+  __device__ __forceinline__ void down(T* u0, T* u1) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) z[v] = (T)kOmegaA * d[v] * r[v];
+    sweep(u0, (T)kOmegaB);
+    T l[NV] = {};
+    put(u1, z);
+    __syncthreads();
+    lap(u1, z, l);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) l[v] = r[v] - l[v];
+    put(u0, l);
+    __syncthreads();
+  }
+  // right-hand side: the residual res of the finer level summed over the
+  // 2x2x2 children in a fixed order
+  __device__ __forceinline__ void restrict_from(const T* res_) {
+    const lds_cp<T> res = (lds_cp<T>)res_;
+    const int fnx = 2 * nx, fny = 2 * ny;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      if (on(v)) {
+        T sum = 0;
+#pragma unroll
+        for (int dz = 0; dz < 2; ++dz)
+#pragma unroll
+          for (int dy = 0; dy < 2; ++dy)
+#pragma unroll
+            for (int dx = 0; dx < 2; ++dx) sum += res[kid[v] + (dz * fny + dy) * fnx + dx];
+        r[v] = sum;
+      }
+    }
+  }
+  // prolongation of the coarse correction zc and both post-sweeps
+  __device__ __forceinline__ void up(const T* zc_, T* u0, T* u1) {
+    const lds_cp<T> zc = (lds_cp<T>)zc_;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) z[v] = z[v] + (T)kProlong * zc[par[v]];
+    sweep(u0, (T)kOmegaB);
+    sweep(u1, (T)kOmegaA);
+  }
+  // `sweeps` damped Jacobi sweeps from zero (the coarsest level); returns the
+  // buffer that is free afterwards
+  __device__ __forceinline__ T* solve(T* u0, T* u1, int sweeps) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) z[v] = (T)kOmega * d[v] * r[v];
+    for (int k = 1; k < sweeps; ++k) {
+      sweep(u0, (T)kOmega);
+      T* t = u0;
+      u0 = u1;
+      u1 = t;
+    }
+    return u0;
+  }
+};
+
+// Levels l0 .. top of a system whose level l0 has at most NV cells per thread;
+// smem: bottom_z_bytes of every level; out: the correction of level l0.
+template <typename T, int NV, bool VEC>
+__device__ __forceinline__ void bottom_levels(const SysDev& s, int l0, int sweeps, T* smem,
+                                              T* out) {
+  __shared__ T wk[2][5][64];  // operators of the wavefront's levels
+  const int top = s.nlev - 1;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const MgLevel& La = s.lev[l0];
+  // the first level of at most 64 cells; `two` levels above it (a level below
+  // one of 4096 cells has 512, the next 64)
+  int lw = l0;
+  while (lw <= top && s.lev[lw].n > 64) ++lw;
+  const bool two = lw > l0 + 1;
+  const MgLevel& Lb = s.lev[two ? l0 + 1 : l0];
+  T* const a0 = smem;
+  T* const a1 = a0 + lds_al16(La.n * (int)sizeof(T)) / (int)sizeof(T);
+  T* const b0 = a1 + lds_al16(La.n * (int)sizeof(T)) / (int)sizeof(T);
+  T* const b1 = b0 + (two ? lds_al16(Lb.n * (int)sizeof(T)) / (int)sizeof(T) : 0);
+  T* const w0 = b1 + (two ? lds_al16(Lb.n * (int)sizeof(T)) / (int)sizeof(T) : 0);
+  // all loads of all levels in flight together
+  BottomCells<T, NV, VEC> A;
+  BottomCells<T, 1, false> B;
+  if (lw > l0) A.load(La, true);
+  if (two) B.load(Lb, false);
+  T ra = (T)0;
+  if (tid < 128 && lw + (tid >> 6) <= top) {
+    const MgLevel& L = s.lev[lw + (tid >> 6)];
+    if (lane < (int)L.n) {
+      const MgCoefs<T> co(L);
+      T k[5];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) k[c] = co.comp1g(c, lane);
+      k[4] = L.m ? ld1((const T*)L.m, lane) : (T)0;
+      if (lw == l0 && tid < 64) ra = ld1((const T*)L.r, lane);
+#pragma unroll
+      for (int c = 0; c < 5; ++c) wk[tid >> 6][c][lane] = k[c];
+    }
+  }
+  const T* zc = w0;  // the correction that level l0 takes
+  if (lw > l0) {
+    if (!two && lw > top) A.solve(a0, a1, sweeps);
+    else A.down(a0, a1);
+  }
+  if (two) {
+    B.restrict_from(a0);
+    if (lw > top) {
+      T* const f = B.solve(b0, b1, sweeps);
+      B.put(f, B.z);
+      __syncthreads();
+      zc = f;
+    } else {
+      B.down(b0, b1);
+    }
+  }
+  if (lw <= top) {
+    if (lw == l0) __syncthreads();  // wk (the steps above have barriers)
+    if (tid < 64) {
+      const MgLevel& Lf = s.lev[lw];
+      WaveLevel<T> W;
+      W.load(Lf, wk[0], lane);
+      const T w = (T)kOmega, wa = (T)kOmegaA, wb = (T)kOmegaB;
+      const int fx = Lf.nx, fy = Lf.ny;
+      const int cl = lane < W.n ? lane : 0;
+      const int x = cl % fx, y = (cl / fx) % fy, zz = cl / (fx * fy);
+      if (lw > l0) {
+        // right-hand side from the residual of the level above
+        const lds_cp<T> res = (lds_cp<T>)(two ? b0 : a0);
+        const int unx = 2 * fx, uny = 2 * fy;
+        const int f0 = (2 * zz * uny + 2 * y) * unx + 2 * x;
+        T sum = 0;
+#pragma unroll
+        for (int dz = 0; dz < 2; ++dz)
+#pragma unroll
+          for (int dy = 0; dy < 2; ++dy)
+#pragma unroll
+            for (int dx = 0; dx < 2; ++dx) sum += res[f0 + (dz * uny + dy) * unx + dx];
+        ra = lane < W.n ? sum : (T)0;
+      }
+      T z;
+      if (lw == top) {
+        z = w * W.d * ra;
+        for (int k = 1; k < sweeps; ++k) z = z + w * W.d * (ra - W.lap(z));
+      } else {
+        const MgLevel& Lc = s.lev[lw + 1];
+        WaveLevel<T> C;
+        C.load(Lc, wk[1], lane);
+        z = wa * W.d * ra;
+        z = z + wb * W.d * (ra - W.lap(z));
+        const T res = ra - W.lap(z);
+        const bool con = lane < C.n;
+        const int cc = con ? lane : 0;
+        const int X = cc % Lc.nx, Y = (cc / Lc.nx) % Lc.ny, Z = cc / (Lc.nx * Lc.ny);
+        T rb = 0;
+#pragma unroll
+        for (int dz = 0; dz < 2; ++dz)
+#pragma unroll
+          for (int dy = 0; dy < 2; ++dy)
+#pragma unroll
+            for (int dx = 0; dx < 2; ++dx) {
+              const int f = ((2 * Z + dz) * fy + 2 * Y + dy) * fx + 2 * X + dx;
+              rb += __shfl(res, f, 64);
+            }
+        if (!con) rb = (T)0;
+        T q = w * C.d * rb;
+        for (int k = 1; k < sweeps; ++k) q = q + w * C.d * (rb - C.lap(q));
+        // prolongation of the coarsest correction, two sweeps
+        const T u =
+            z + (T)kProlong * __shfl(q, ((zz >> 1) * Lc.ny + (y >> 1)) * Lc.nx + (x >> 1), 64);
+        z = u + wb * W.d * (ra - W.lap(u));
+        z = z + wa * W.d * (ra - W.lap(z));
+      }
+      if (lane < W.n) {
+        if (lw == l0) st1(out, (long long)lane, z);
+        else ((lds_p<T>)w0)[lane] = z;
+      }
+    }
+    if (lw == l0) return;
+    __syncthreads();
+    if (two) {
+      B.up(w0, b0, b1);
+      B.put(b0, B.z);
+      __syncthreads();
+      zc = b0;
+    }
+  }
+  if (two || lw <= top) A.up(zc, a0, a1);
+  if constexpr (VEC) {
+#pragma unroll
+    for (int j = 0; j < NV; j += 4) {
+      if (A.on(j))
+        *(gmp<vec_t<float, 4>>)(out + A.c[j]) =
+            vec_t<float, 4>{A.z[j], A.z[j + 1], A.z[j + 2], A.z[j + 3]};
+    }
+  } else {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      if (A.on(v)) st1(out, (long long)A.c[v], A.z[v]);
+    }
+  }
+}
+
+// The bottom of the cycle: levels lb..top of a system (its cycle from level
+// lb down; lb > every W level) in one workgroup.  A level of more than 64
+// cells is held by all threads (BottomCells: at most two such levels, of at
+// most 4096 (FP32) / 2048 (FP64) and 512 cells), the last one or two levels
+// of at most 64 cells by one wavefront, a cell per lane; only iterates and
+// residuals go through LDS.  The same operations as the per-level launches:
+// zero-guess sweep + sweep, restriction, `sweeps` damped Jacobi sweeps from
+// zero on the coarsest level, prolongation + sweep + sweep; the correction of
+// level lb goes to its z[1] (z[0] when lb is the coarsest).  A coarsest level
+// alone may have more cells than the threads hold (8192 / 4096): its
+// coefficients then come from memory.  Each system takes part only in the
+// launch for its own lb (s.mg_lb == l0).
+//
+// What bounds it is latency: one round of loads for all levels, then a dozen
+// barriers and the wavefront's shuffles.  Per visit (16^3 .. 2^3, FP32) 22.7
+// -> 11.2 us against a form that copied all levels into LDS and re-read
+// coefficients and indices in every step; FP64 25.6 -> 12 us.  512 threads: at
+// 1024 the 128 registers a thread may have spill.
 template <typename T>
 __global__ __launch_bounds__(kBottomThreads) void k_mg_bottom(const SysDev* __restrict__ sds,
                                                               int sweeps, int l0, int wl,
                                                               int so) {
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ MgLevel lv[kMaxLevels];  // the levels, with LDS pointers if resident
   const SysDev& s = sds[blockIdx.x];
   if (s.nlev <= 0 || s.sc->done || s.mg_lb != l0) return;
   if (wl >= 0 && wl >= s.mg_w) return;
   if (so && !s.sc->first) return;
+  constexpr int NV = sizeof(T) == 4 ? 8 : 4;
   const int top = s.nlev - 1;
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const T w = (T)kOmega, wa = (T)kOmegaA, wb = (T)kOmegaB;
-  constexpr int es = sizeof(T);
-  long long full_bytes = 0;
-  for (int l = l0; l <= top; ++l) full_bytes += bottom_full_bytes(s.lev[l].n, es, s.has_m);
-  const bool full = full_bytes <= kBottomLdsMax;
-  // z and the second buffer of each level (pointer tables in LDS: indexed
-  // by level at run time, they would otherwise live in scratch)
-  __shared__ T* za[kMaxLevels];
-  __shared__ T* zb[kMaxLevels];
-  unsigned char* p = smem;
-  for (int l = l0; l <= top; ++l) {
-    if (tid == 0) za[l] = (T*)p;
-    p += lds_al16(s.lev[l].n * es);
-    if (tid == 0) zb[l] = (T*)p;
-    p += lds_al16(s.lev[l].n * es);
-  }
-  if (tid == 0) {
-    for (int l = l0; l <= top; ++l) lv[l] = s.lev[l];
-  }
-  // the copies into LDS as one table of segments (16-byte units; a tail of
-  // 4-byte words per segment), so that every thread issues all of its loads
-  // before it waits for any
-  constexpr int kSeg = 6 * kMaxLevels;
-  __shared__ const uint4* cs_src[kSeg];
-  __shared__ uint4* cs_dst[kSeg];
-  __shared__ int cs_beg[kSeg + 1];
-  __shared__ int cs_tail[kSeg];
-  int nseg = 0;
-  if (full) {
-    // record a copy of `bytes` (a multiple of 4) from global memory to LDS
-    auto copy = [&](void* dst, const void* src, long long bytes) {
-      if (tid == 0) {
-        cs_src[nseg] = (const uint4*)src;
-        cs_dst[nseg] = (uint4*)dst;
-        cs_beg[nseg + 1] = cs_beg[nseg] + (int)(bytes >> 4);
-        cs_tail[nseg] = (int)((bytes & 15) >> 2);
-      }
-      ++nseg;
-    };
-    if (tid == 0) cs_beg[0] = 0;
-    for (int l = l0; l <= top; ++l) {
-      const MgLevel& G = s.lev[l];
-      const long long n = G.n;
-      if constexpr (es == 4) {
-        copy(p, G.kc, bottom_coef_bytes(n, es));
-        if (tid == 0) lv[l].kc = p;
-        p += lds_al16(bottom_coef_bytes(n, es));
-      } else {
-        const void* src[4] = {G.kx, G.ky, G.kz, G.dinv};
-        for (int c = 0; c < 4; ++c) {
-          copy(p, src[c], 8 * n);
-          if (tid == 0) {
-            if (c == 0) lv[l].kx = p;
-            if (c == 1) lv[l].ky = p;
-            if (c == 2) lv[l].kz = p;
-            if (c == 3) lv[l].dinv = p;
-          }
-          p += lds_al16(8 * n);
-        }
-      }
-      if (s.has_m) {
-        copy(p, G.m, n * es);
-        if (tid == 0) lv[l].m = p;
-        p += lds_al16(n * es);
-      }
-      // right-hand side: level l0's from memory, the coarser ones restricted here
-      if (l == l0) copy(p, G.r, n * es);
-      if (tid == 0) lv[l].r = p;
-      p += lds_al16(n * es);
-    }
-    __syncthreads();
-    const int total = cs_beg[nseg];
-    using W4 = vec_t<unsigned, 4>;
-    for (int b0 = tid; b0 < total; b0 += 4 * nt) {
-      W4 v0 = 0u, v1 = 0u, v2 = 0u, v3 = 0u;
-      int s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-      auto load = [&](int u, int& sg, W4& v) {
-        if (u < total) {
-          while (cs_beg[sg + 1] <= u) ++sg;
-          v = *(glb_cp<W4>)((const W4*)cs_src[sg] + (u - cs_beg[sg]));
-        }
-      };
-      auto store = [&](int u, int sg, W4 v) {
-        if (u < total) *(lds_p<W4>)((W4*)cs_dst[sg] + (u - cs_beg[sg])) = v;
-      };
-      load(b0, s0, v0);
-      load(b0 + nt, s1, v1);
-      load(b0 + 2 * nt, s2, v2);
-      load(b0 + 3 * nt, s3, v3);
-      store(b0, s0, v0);
-      store(b0 + nt, s1, v1);
-      store(b0 + 2 * nt, s2, v2);
-      store(b0 + 3 * nt, s3, v3);
-    }
-    for (int k = 0; k < nseg; ++k) {
-      const int n16 = cs_beg[k + 1] - cs_beg[k];
-      if (tid < cs_tail[k])
-        ((unsigned*)(cs_dst[k] + n16))[tid] = ((const unsigned*)(cs_src[k] + n16))[tid];
-    }
-  }
-  __syncthreads();
-  // levels lw..top go to one wavefront (a level below one of <= 64 cells has
-  // <= 8, and a coarser one would have < 8: at most two such levels)
-  int lw = l0;
-  while (lw <= top && lv[lw].n > 64) ++lw;
-  // out = u + om D^-1 (r - L u) on level l, u and out in LDS
-  // f(view) with the level's data in LDS or in global memory
-  auto with_view = [&](int l, auto f) {
-    if (full) {
-      f(LdsView<T, true>(lv[l]));
-    } else {
-      f(LdsView<T, false>(lv[l]));
-    }
-  };
-  auto sweep = [&](int l, const T* u_, T* out_, T om) {
-    const lds_cp<T> u = (lds_cp<T>)u_;
-    const lds_p<T> out = (lds_p<T>)out_;
-    with_view(l, [&](const auto& V) {
-      for_cells(V.n, V.nx, V.ny, [&](int i, int x, int y, int z) {
-        out[i] = u[i] + om * V.dinv(i) * (V.r[i] - V.lap(i, x, y, z, u));
-      });
-    });
-    __syncthreads();
-  };
-  // FP32 levels resident in LDS with nx % 4 == 0: groups of 4 cells per
-  // thread (the packed coefficients of a group in two 16-byte reads, the
-  // neighbouring rows and planes in 16-byte reads), the operation order of
-  // LdsView::lap per cell
-  using V4 = vec_t<float, 4>;
-  using U4 = vec_t<unsigned, 4>;
-  using U2 = vec_t<unsigned, 2>;
-  auto vec_ok = [&](int l) { return sizeof(T) == 4 && full && lv[l].nx % 4 == 0; };
-  // f(g, i, x0, y, z) for the groups g = i / 4 of level l
-  auto for_groups = [&](int l, auto f) {
-    const int nx = lv[l].nx, ny = lv[l].ny, ng = (int)lv[l].n / 4;
-    for (int g = tid; g < ng; g += nt) {
-      const int i = 4 * g;
-      const int x0 = i % nx, t = i / nx;
-      f(g, i, x0, t % ny, t / ny);
-    }
-  };
-  // (L u) of the 4 cells from i = 4 g (x0, y, z) of level l, u in LDS
-  auto lap4 = [&](int l, const float* u_, int g, int i, int x0, int y, int z) -> V4 {
-    const lds_cp<float> u = (lds_cp<float>)u_;
-    const lds_cp<unsigned short> kc = (lds_cp<unsigned short>)(const unsigned short*)lv[l].kc;
-    const int nx = lv[l].nx, ny = lv[l].ny, nz = lv[l].nz, pl = nx * ny, n = (int)lv[l].n;
-    const U4 c0 = *(lds_cp<U4>)(kc + 16 * g), c1 = *(lds_cp<U4>)(kc + 16 * g + 8);
-    const int ixm = x0 == 0 ? i + nx - 1 : i - 1, ixp = x0 + 4 == nx ? i - nx + 4 : i + 4;
-    const int iym = y == 0 ? i + pl - nx : i - nx, iyp = y == ny - 1 ? i - pl + nx : i + nx;
-    const int izm = z == 0 ? i + n - pl : i - pl, izp = z == nz - 1 ? i - n + pl : i + pl;
-    const V4 w = *(lds_cp<V4>)(u + i);
-    const V4 wym = *(lds_cp<V4>)(u + iym), wyp = *(lds_cp<V4>)(u + iyp);
-    const V4 wzm = *(lds_cp<V4>)(u + izm), wzp = *(lds_cp<V4>)(u + izp);
-    const float wxm = u[ixm], wxp = u[ixp];
-    const U2 ym2 = *(lds_cp<U2>)(kc + 16 * (iym >> 2) + 4);
-    const U2 zm2 = *(lds_cp<U2>)(kc + 16 * (izm >> 2) + 8);
-    const float kxm = bflo(kc[16 * (ixm >> 2) + (ixm & 3)]);
-    const V4 kx = bf4(c0.x, c0.y), ky = bf4(c0.z, c0.w), kz = bf4(c1.x, c1.y);
-    const V4 kym = bf4(ym2.x, ym2.y), kzm = bf4(zm2.x, zm2.y);
-    V4 s4;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const float up = v < 3 ? w[v + 1] : wxp, uw = v > 0 ? w[v - 1] : wxm;
-      const float kw = v > 0 ? kx[v - 1] : kxm;
-      s4[v] = kx[v] * (w[v] - up) + kw * (w[v] - uw) + ky[v] * (w[v] - wyp[v]) +
-              kym[v] * (w[v] - wym[v]) + kz[v] * (w[v] - wzp[v]) + kzm[v] * (w[v] - wzm[v]);
-    }
-    if (lv[l].m) s4 += *(lds_cp<V4>)((const float*)lv[l].m + i) * w;
-    return s4;
-  };
-  auto dinv4 = [&](int l, int g) {
-    const U2 d = *(lds_cp<U2>)((lds_cp<unsigned short>)(const unsigned short*)lv[l].kc +
-                               16 * g + 12);
-    return bf4(d.x, d.y);
-  };
-  // out = u + om D^-1 (r - L u) on level l by groups, then a barrier
-  auto sweep4 = [&](int l, const T* u, T* out, T om) {
-    for_groups(l, [&](int g, int i, int x0, int y, int z) {
-      const V4 uc = *(lds_cp<V4>)((const float*)u + i);
-      const V4 rr = *(lds_cp<V4>)((const float*)lv[l].r + i);
-      *(lds_p<V4>)((float*)out + i) =
-          uc + (float)om * dinv4(l, g) * (rr - lap4(l, (const float*)u, g, i, x0, y, z));
-    });
-    __syncthreads();
-  };
-  for (int l = l0; l < lw && l < top; ++l) {
-    const lds_p<T> zal = (lds_p<T>)za[l];
-    const lds_p<T> zbl = (lds_p<T>)zb[l];
-    if (vec_ok(l)) {
-      for_groups(l, [&](int g, int i, int, int, int) {
-        *(lds_p<V4>)((float*)zb[l] + i) =
-            (float)wa * dinv4(l, g) * *(lds_cp<V4>)((const float*)lv[l].r + i);
-      });
-      __syncthreads();
-      sweep4(l, zb[l], za[l], wb);
-      for_groups(l, [&](int g, int i, int x0, int y, int z) {
-        *(lds_p<V4>)((float*)zb[l] + i) = *(lds_cp<V4>)((const float*)lv[l].r + i) -
-                                          lap4(l, (const float*)za[l], g, i, x0, y, z);
-      });
-      __syncthreads();
-    } else {
-    with_view(l, [&](const auto& V) {
-      for (int i = tid; i < V.n; i += nt) zbl[i] = wa * V.dinv(i) * V.r[i];
-    });
-    __syncthreads();
-    sweep(l, zb[l], za[l], wb);
-    // restriction of r - L z into r of level l + 1: the residual of every
-    // cell into the free second buffer, then the sums over the 2x2x2
-    // children in a fixed order
-    with_view(l, [&](const auto& V) {
-      for_cells(V.n, V.nx, V.ny, [&](int i, int x, int y, int z) {
-        zbl[i] = V.r[i] - V.lap(i, x, y, z, (lds_cp<T>)zal);
-      });
-    });
-    __syncthreads();
-    }
-    const MgLevel& Lf = lv[l];
-    with_view(l + 1, [&](const auto& C) {
-      const int fnx = Lf.nx, fpl = Lf.nx * Lf.ny;
-      for_cells(C.n, C.nx, C.ny, [&](int c, int X, int Y, int Z) {
-        const int f0 = 2 * Z * fpl + 2 * Y * fnx + 2 * X;
-        T sum = 0;
-        for (int dz = 0; dz < 2; ++dz)
-          for (int dy = 0; dy < 2; ++dy)
-            for (int dx = 0; dx < 2; ++dx) sum += zbl[f0 + dz * fpl + dy * fnx + dx];
-        C.r[c] = sum;
-      });
-    });
-    __syncthreads();
-  }
-  if (lw <= top) {
-    if (tid < 64) {
-      const int lane = tid;
-      WaveLevel<T> A;
-      A.load(lv[lw], lane);
-      const T ra = lane < A.n ? ((const T*)lv[lw].r)[lane] : (T)0;
-      T z;
-      if (lw == top) {
-        z = w * A.d * ra;
-        for (int k = 1; k < sweeps; ++k) z = z + w * A.d * (ra - A.lap(z));
-      } else {
-        const MgLevel& Lf = lv[lw];
-        const MgLevel& Lc = lv[lw + 1];
-        z = wa * A.d * ra;
-        z = z + wb * A.d * (ra - A.lap(z));
-        const T res = ra - A.lap(z);
-        WaveLevel<T> B;
-        B.load(Lc, lane);
-        const bool con = lane < B.n;
-        const int C = con ? lane : 0;
-        const int X = C % Lc.nx, Y = (C / Lc.nx) % Lc.ny, Z = C / (Lc.nx * Lc.ny);
-        T rb = 0;
-        for (int dz = 0; dz < 2; ++dz)
-          for (int dy = 0; dy < 2; ++dy)
-            for (int dx = 0; dx < 2; ++dx) {
-              const int f = ((2 * Z + dz) * Lf.ny + 2 * Y + dy) * Lf.nx + 2 * X + dx;
-              rb += __shfl(res, f, 64);
-            }
-        if (!con) rb = (T)0;
-        T zc = w * B.d * rb;
-        for (int k = 1; k < sweeps; ++k) zc = zc + w * B.d * (rb - B.lap(zc));
-        // prolongation of the coarsest correction, two sweeps
-        const int c = lane < A.n ? lane : 0;
-        const int x = c % Lf.nx, y = (c / Lf.nx) % Lf.ny, zz = c / (Lf.nx * Lf.ny);
-        const T u =
-            z + (T)kProlong * __shfl(zc, ((zz >> 1) * Lc.ny + (y >> 1)) * Lc.nx + (x >> 1), 64);
-        z = u + wb * A.d * (ra - A.lap(u));
-        z = z + wa * A.d * (ra - A.lap(z));
-      }
-      if (lane < A.n) za[lw][lane] = z;
-    }
-    __syncthreads();
-  } else {
-    // a coarsest level of more than 64 cells: block-wide sweeps
-    const int n = (int)lv[top].n;
-    T* a = za[top];
-    T* b = zb[top];
-    with_view(top, [&](const auto& V) {
-      const lds_p<T> al = (lds_p<T>)a;
-      for (int i = tid; i < n; i += nt) al[i] = w * V.dinv(i) * V.r[i];
+  const int tid = threadIdx.x;
+  const MgLevel& La = s.lev[l0];
+  const int na = (int)La.n;
+  T* const out = (T*)La.z[l0 == top ? 0 : 1];
+  T* const a0 = (T*)smem;
+  T* const a1 = a0 + lds_al16(na * (int)sizeof(T)) / (int)sizeof(T);
+  if (na > NV * kBottomThreads) {
+    // (l0 == top)
+    const GlobalView<T> V(La);
+    const T w = (T)kOmega;
+    T *a = a0, *b = a1;
+    for_cells(na, V.nx, V.ny, [&](int i, int, int, int) {
+      ((lds_p<T>)a)[i] = w * V.dinv(i) * V.r[i];
     });
     __syncthreads();
     for (int k = 1; k < sweeps; ++k) {
-      sweep(top, a, b, w);
+      const lds_cp<T> u = (lds_cp<T>)a;
+      for_cells(na, V.nx, V.ny, [&](int i, int x, int y, int z) {
+        ((lds_p<T>)b)[i] = u[i] + w * V.dinv(i) * (V.r[i] - V.lap(i, x, y, z, u));
+      });
+      __syncthreads();
       T* t = a;
       a = b;
       b = t;
     }
-    if (a != za[top]) {
-      for (int i = tid; i < n; i += nt) za[top][i] = a[i];
-      __syncthreads();
+    for (int i = tid; i < na; i += kBottomThreads) out[i] = ((lds_cp<T>)a)[i];
+    return;
+  }
+  if constexpr (sizeof(T) == 4) {
+    if (na > 2 * kBottomThreads && La.nx % 4 == 0) {
+      bottom_levels<T, NV, true>(s, l0, sweeps, a0, out);
+      return;
     }
   }
-  // the post-smoothed correction of level l ends in zb[l] (bit l of inb;
-  // the levels solved above end in za)
-  unsigned inb = 0;
-  for (int l = (lw <= top ? lw : top) - 1; l >= l0; --l) {
-    const MgLevel& Lf = lv[l];
-    const MgLevel& Lc = lv[l + 1];
-    const int n = (int)Lf.n;
-    const lds_cp<T> zc = (lds_cp<T>)(((inb >> (l + 1)) & 1u) ? zb[l + 1] : za[l + 1]);
-    const lds_cp<T> zf = (lds_cp<T>)za[l];
-    const lds_p<T> u = (lds_p<T>)zb[l];
-    for_cells(n, Lf.nx, Lf.ny, [&](int i, int x, int y, int z) {
-      u[i] = zf[i] + (T)kProlong * zc[((z >> 1) * Lc.ny + (y >> 1)) * Lc.nx + (x >> 1)];
-    });
-    __syncthreads();
-    if (vec_ok(l)) {
-      sweep4(l, zb[l], za[l], wb);
-      sweep4(l, za[l], zb[l], wa);
-    } else {
-      sweep(l, zb[l], za[l], wb);
-      sweep(l, za[l], zb[l], wa);
-    }
-    inb |= 1u << l;
-  }
-  const T* __restrict__ res = ((inb >> l0) & 1u) ? zb[l0] : za[l0];
-  T* out = (T*)s.lev[l0].z[l0 == top ? 0 : 1];  // global
-  for (int i = tid; i < (int)lv[l0].n; i += nt) out[i] = res[i];
+  bottom_levels<T, NV, false>(s, l0, sweeps, a0, out);
 }
 
 // (r, z) of the preconditioned CG: beta = (r,z) / (r,z)_old (0 after a start)

@@ -55,3 +55,34 @@ def _cycle_error(shape, precision, w, mass, seed=1):
 ])
 def test_smallest_fused_levels(precision, shape, w, mass):
     assert _cycle_error(shape, precision, w, mass) <= TOL[precision]
+
+
+@pytest.mark.parametrize("mass", [False, True])
+@pytest.mark.parametrize("precision", [L.FP64, L.MIXED])
+@pytest.mark.parametrize("shape", [
+    (8, 8, 8),        # the bottom is one wavefront's (4^3, 2^3)
+    (6, 6, 6),        # one coarsest level of 27 cells
+    (10, 10, 10),     # one coarsest level of 125 cells, all threads
+    (20, 20, 20),     # 10^3 above a coarsest level of 5^3
+    (24, 24, 24),     # 12^3, 6^3 and a wavefront's 3^3
+    (28, 28, 28),     # 14^3 (rows of 14), coarsest 7^3
+    (32, 24, 40),     # 3840, 480 and 60 cells
+    (32, 32, 32),     # 4096, 512, 64 and 8 cells
+    (4, 4, 2048),     # 2 x 2 x 1024 cells above 1 x 1 x 512
+    (30, 30, 30),     # a coarsest level of 3375 cells
+])
+def test_bottom_levels(shape, precision, mass):
+    assert _cycle_error(shape, precision, 0, mass) <= TOL[precision]
+
+
+def test_largest_coarsest_level():
+    """19^3 cells on the coarsest of two levels, more than the threads hold:
+    FP32 engines only, beyond what the oracle's cycle takes."""
+    shape = (38, 38, 38)
+    e = _system(shape, 3, False)
+    s = Poisson(shape, method=L.PCG, precision=L.MIXED, resmode=L.RES_REL_TRUE, tol=1e-8,
+                maxiter=2000, precond=L.PRECOND_MG)
+    s.set_system(e)
+    x, info = s.solve(None)
+    s.close()
+    assert info["converged"] == 1 and O.true_relres(e, x) <= 1e-8 * (1 + 1e-6)
