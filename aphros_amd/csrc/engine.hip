@@ -60,14 +60,13 @@ Rec make_stencil_rec(int nx, int ny, int nz, int vx, int blocks_target, const Tu
 // march has too few workgroups.  The planes and rows ahead of a march wrap
 // once: at least 8 of each.
 constexpr long long kFuseMinCells64 = 1LL << 19, kFuseMinCells32 = 3LL << 20;
-// Levels below level 0 of FP32 engines with at most this many cells and
-// nx % 4 == 0 smooth in tile launches (k_mg_tile: one launch and one round of
-// global loads per pre- or post-smoothing instead of two z-marching
-// launches).  Per visit at 64^3: 8.1 + 8.6 us against 12 + 11 us for the
-// sweep pairs; at 32^3 6 + 6 us against 11.5 + 11.5 us; at 128^3 the tiles'
-// halos (4.5x the level's bytes) miss L2 and the tiles took 37 + 38 us
-// against 22 + 22 us, so 128^3 keeps the sweeps.
-constexpr long long kTileMaxCells = 1LL << 18;
+// Levels of FP32 engines with at most this many cells and nx % 4 == 0 smooth in
+// tile launches (k_mg_tile: one launch and one round of global loads per pre-
+// or post-smoothing instead of two z-marching launches).  Microseconds per
+// iteration of a whole solve, level 0 swept -> tiled: 32^3 65 -> 56, 48^3 81 ->
+// 73, 64^3 84 -> 80, 80^3 112 -> 108, but 96^3 113 -> 117 and 128^3 135 -> 160:
+// the tiles' halos (4.5x the level's bytes) then miss L2.
+constexpr long long kTileMaxCells = 1LL << 19;
 // Iterations of one resident launch: a launch costs about 30 us more than its
 // iterations (of 7 to 25 us); the server's steps are shorter, so that a new
 // request waits a few milliseconds at most.
@@ -466,7 +465,7 @@ int Engine::add_system(int nx, int ny, int nz, double h3, int* slot) {
         MgLevel& L = S.lev[l];
         L.post = make_post_rec(L.nx, L.ny, L.nz, fp32_ ? 4 : 2, ncu_, &t)
                      ? 1
-                     : (fp32_ && l >= 1 && L.n <= kTileMaxCells && L.nx % 4 == 0 ? 2 : 0);
+                     : (fp32_ && L.n <= kTileMaxCells && L.nx % 4 == 0 ? 2 : 0);
       }
       for (int l = 1; l <= w && rc == APHPOIS_OK; ++l) {
         // a fused or tile level's second cycle leaves z[1] (the first
@@ -1052,6 +1051,7 @@ int Engine::build_tables() {
           t.blk0 = (int)blt[l].size();
           for (int i = 0; i < t.nblk; ++i) blt[l].push_back((int)rlt[l].size());
           rlt[l].push_back(t);
+          if (l == 0) nblk_pc = t.nblk;
         } else {
           post_plain[l] = 1;
         }

@@ -66,7 +66,7 @@ struct LaunchSet {
 constexpr int kPostBlock = 1024;
 // k_mg_tile: output cells per tile edge and threads per workgroup
 constexpr int kTile = 8;
-constexpr int kTileBlock = 256;
+constexpr int kTileBlock = 512;
 
 // LDS of the bottom-levels kernel, per level of n cells (element size es): two
 // buffers for iterates and residuals.

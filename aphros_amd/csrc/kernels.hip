@@ -1266,13 +1266,16 @@ __global__ __launch_bounds__(kBlock) void k_mg_sweep(const SysDev* __restrict__ 
 //   POST: u = z[0] + kProlong P z_c (12^3 box); v = u + wB D^-1 (r - L u)
 //         (10^3 box); z[1] = v + wA D^-1 (r - L v) (+ zs: the last sweep of
 //         a second coarse correction) on the tile
+// 512 threads: 256 took 1-4 % longer per iteration of a solve (48^3 .. 256^3),
+// 1024 as long; what bounds a tile is its chain of loads and LDS phases.
 // The box is staged in LDS by rows of 16 cells (x0-4 .. x0+11, four aligned
 // groups of 4 cells: r as float4, the packed bfloat16 coefficients as two
 // 16-byte halves, u formed as the row is loaded), y and z from -2 to +9
 // around the tile.  Rows and groups wrap periodically (a level edge shorter
 // than the box repeats cells); tile cells past the level's edge are neither
 // stored nor restricted (edges are even, tiles start at multiples of 8).
-template <bool PRE>
+// DOT (POST on level 0): partials of (r, z[1]).
+template <bool PRE, bool DOT>
 __global__ __launch_bounds__(kTileBlock) void k_mg_tile(const SysDev* __restrict__ sds,
                                                         const Rec* __restrict__ recs,
                                                         const int* __restrict__ b2r, int l,
@@ -1374,6 +1377,7 @@ __global__ __launch_bounds__(kTileBlock) void k_mg_tile(const SysDev* __restrict
   }
   __syncthreads();
   gmp<float> zout = (gmp<float>)(PRE ? Lv.z[0] : Lv.z[1]);
+  double dot = 0.0;
   for (int c = threadIdx.x; c < NT; c += kTileBlock) {
     const int a = c % kTile, bb = (c / kTile) % kTile, cz = c / (kTile * kTile);
     const int xi = 4 + a, ri = (2 + bb) + (2 + cz) * B;
@@ -1386,8 +1390,15 @@ __global__ __launch_bounds__(kTileBlock) void k_mg_tile(const SysDev* __restrict
     } else {
       float out = sV[j] + (float)kOmegaA * kf(ri, xi, 3) * (sR[j] - lap(sV, ri, xi));
       if (addzs && in) out += ((gcp<float>)Lv.zs)[g];
-      if (in) zout[g] = out;
+      if (in) {
+        zout[g] = out;
+        if constexpr (DOT) dot += (double)sR[j] * (double)out;
+      }
     }
+  }
+  if constexpr (DOT) {
+    double acc[1] = {dot};
+    block_partial<1, 0u, kTileBlock>(acc, s.partials, rc.nblk, lb);
   }
   if constexpr (PRE) {
     __syncthreads();
@@ -3521,9 +3532,9 @@ static void launch_cycle(const LaunchSet& L, hipStream_t st, int l, int wl, bool
     launch_sweep<T, 3, false>(L, st, l, -1, -1, wl);
   }
   if (L.post_tile[l]) {
-    mark(2);
+    mark(l == 0 ? 0 : 2);
     if constexpr (sizeof(T) == 4) {
-      hipLaunchKernelGGL(k_mg_tile<true>, dim3(L.nlt[l]), dim3(kTileBlock), 0, st, L.sds,
+      hipLaunchKernelGGL((k_mg_tile<true, false>), dim3(L.nlt[l]), dim3(kTileBlock), 0, st, L.sds,
                          L.rec_lt[l], L.b2r_lt[l], l, wl, L.start_only, 0);
     }
   }
@@ -3545,10 +3556,16 @@ static void launch_cycle(const LaunchSet& L, hipStream_t st, int l, int wl, bool
     else launch_post_l<T, false, false>(L, st, l, wl, second ? 1 : 0);
   }
   if (L.post_tile[l]) {
-    mark(2);
+    mark(l == 0 ? 5 : 2);
     if constexpr (sizeof(T) == 4) {
-      hipLaunchKernelGGL(k_mg_tile<false>, dim3(L.nlt[l]), dim3(kTileBlock), 0, st, L.sds,
-                         L.rec_lt[l], L.b2r_lt[l], l, wl, L.start_only, second ? 1 : 0);
+      if (l == 0) {
+        hipLaunchKernelGGL((k_mg_tile<false, true>), dim3(L.nlt[l]), dim3(kTileBlock), 0, st,
+                           L.sds, L.rec_lt[l], L.b2r_lt[l], l, wl, L.start_only, 0);
+      } else {
+        hipLaunchKernelGGL((k_mg_tile<false, false>), dim3(L.nlt[l]), dim3(kTileBlock), 0, st,
+                           L.sds, L.rec_lt[l], L.b2r_lt[l], l, wl, L.start_only,
+                           second ? 1 : 0);
+      }
     }
   }
   if (L.post_plain[l]) {

@@ -70,6 +70,8 @@ def test_smallest_fused_levels(precision, shape, w, mass):
     (32, 32, 32),     # 4096, 512, 64 and 8 cells
     (4, 4, 2048),     # 2 x 2 x 1024 cells above 1 x 1 x 512
     (30, 30, 30),     # a coarsest level of 3375 cells
+    (64, 64, 128),    # 2^19 cells: the largest level in tiles
+    (36, 44, 52),     # partial tiles on every side
 ])
 def test_bottom_levels(shape, precision, mass):
     assert _cycle_error(shape, precision, 0, mass) <= TOL[precision]
