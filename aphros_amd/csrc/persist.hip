@@ -82,10 +82,13 @@ struct Shared {
 // over the nblk workgroups of a system; the result is valid in every thread of
 // every workgroup, summed in workgroup order.  Every global store this thread
 // issued before the call is complete before the workgroup's values appear.
+// meanwhile(): run by every wavefront once the workgroup's values are on their
+// way, before it waits for the others'.
 // Returns false if some workgroup's values did not appear in time.
-template <int NV, unsigned MaxMask>
+template <int NV, unsigned MaxMask, class F>
 __device__ __forceinline__ bool gather(double (&v)[NV], u64* slots, int nblk, int me,
-                                       unsigned tag, long long wait, Shared& sh) {
+                                       unsigned tag, long long wait, Shared& sh,
+                                       F meanwhile) {
   wave_reduce<NV, MaxMask>(v);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) {
@@ -108,6 +111,7 @@ __device__ __forceinline__ bool gather(double (&v)[NV], u64* slots, int nblk, in
     st_agent(slots + (long long)me * kPersWords + lane,
              ((lane & 1) ? (b & 0xffffffff00000000ull) : (b << 32)) | tag);
   }
+  meanwhile();
   if (wave < ngrp) {
     // wave w reads the slots 64 w .. 64 w + 63, one per lane
     const int i = lane + 64 * wave;
@@ -225,12 +229,13 @@ __device__ __forceinline__ void halo_table(const Box& b, int2* tab) {
   }
 }
 
-// f(h, value(g), lds offset) over this thread's halo cells, four loads of
-// value(g) in flight
+// f(h, value(g), lds offset) over this thread's halo cells from the skip-th on,
+// four loads of value(g) in flight
 template <class V, class F>
-__device__ __forceinline__ void for_halo(const Box& b, const int2* tab, V value, F f) {
+__device__ __forceinline__ void for_halo(const Box& b, const int2* tab, V value, F f,
+                                         int skip = 0) {
   constexpr int U = 4;
-  for (int h0 = threadIdx.x; h0 < b.nhalo; h0 += U * kT) {
+  for (int h0 = threadIdx.x + skip * kT; h0 < b.nhalo; h0 += U * kT) {
     decltype(value(0)) v[U];
     int o[U];
 #pragma unroll
@@ -250,6 +255,60 @@ __device__ __forceinline__ void for_halo(const Box& b, const int2* tab, V value,
     }
   }
 }
+
+// Halo values a thread loads early, by the bytes of one vector of its cells:
+// what the registers left over hold.
+constexpr int early_halo(int bytes) { return bytes >= 128 ? 0 : (bytes >= 64 ? 2 : 4); }
+
+// The first HR halo values of a thread, loaded while the gather that follows
+// their stores is under way: a neighbour's values in that gather say that its
+// rows are in memory.
+template <typename T, int HR>
+struct EarlyHalo {
+  T v[HR > 0 ? HR : 1];
+  int nb;  // slot of the neighbour in y-, y+, z-, z+ (lane % 4)
+  __device__ EarlyHalo(const PersRec& rc, int lb) {
+    const int pz = rc.nblk / rc.py, jy = lb % rc.py, jz = lb / rc.py;
+    const int q = threadIdx.x & 3;
+    const int y = q == 0 ? (jy == 0 ? rc.py - 1 : jy - 1)
+                         : (q == 1 ? (jy == rc.py - 1 ? 0 : jy + 1) : jy);
+    const int z = q == 2 ? (jz == 0 ? pz - 1 : jz - 1)
+                         : (q == 3 ? (jz == pz - 1 ? 0 : jz + 1) : jz);
+    nb = (z * rc.py + y) * kPersWords;
+  }
+  // waits for the neighbours' values of gather `tag` in `slots` (as long as the
+  // gather itself would), then starts the loads of rows of src
+  __device__ __forceinline__ void load(const Box& b, const int2* tab, const T* src,
+                                       const u64* slots, unsigned tag, long long wait) {
+    if (HR == 0) return;
+    const long long t0 = wall_clock64();
+    for (int n = 1;; ++n) {
+      if (!__any((unsigned)ld_agent(slots + nb) != tag)) break;
+      if (((n & 255) == 0 && wall_clock64() - t0 > wait) || wait < 0) break;
+    }
+#pragma unroll
+    for (int k = 0; k < HR; ++k) {
+      const int h = (int)threadIdx.x + k * kT;
+      if (h < b.nhalo) {
+        const int row = b.row_of(h);
+        v[k] = ld_agent(src + tab[row].x + (h - row * b.nx));
+      }
+    }
+  }
+  // f(h, global index, value, lds offset) of the cells loaded
+  template <class F>
+  __device__ __forceinline__ void use(const Box& b, const int2* tab, F f) const {
+#pragma unroll
+    for (int k = 0; k < HR; ++k) {
+      const int h = (int)threadIdx.x + k * kT;
+      if (h < b.nhalo) {
+        const int row = b.row_of(h), x = h - row * b.nx;
+        const int2 t = tab[row];
+        f(h, t.x + x, v[k], t.y + x);
+      }
+    }
+  }
+};
 
 // distance in LDS to a column's x neighbours
 __device__ __forceinline__ int step_xm(int d, int nx) { return (d & kXm) ? nx - 1 : -1; }
@@ -309,6 +368,8 @@ __global__ __launch_bounds__(kT) void k_pers_cg(const SysDev* __restrict__ sds,
   __syncthreads();
   u64* const sl0 = rc.slots;
   u64* const sl1 = rc.slots + kPersMaxBlocks * kPersWords;
+  constexpr int HR = early_halo(8 * CC * ZC);
+  EarlyHalo<double, HR> eh(rc, lb);
   bool ok = true;
   for (int it = 0; it < iters && !done; ++it) {
 #pragma unroll
@@ -318,8 +379,10 @@ __global__ __launch_bounds__(kT) void k_pers_cg(const SysDev* __restrict__ sds,
     }
     if (!first) {
       const double* hs = it == 0 ? rg : hg;
+      if (it > 0)
+        eh.use(b, tab, [&](int, int, double v, int o) { sp[o] = v + beta * sp[o]; });
       for_halo(b, tab, [&](int gi) { return ld_agent(hs + gi); },
-               [&](int, double v, int o) { sp[o] = v + beta * sp[o]; });
+               [&](int, double v, int o) { sp[o] = v + beta * sp[o]; }, it > 0 ? HR : 0);
 #pragma unroll
       for (int c = 0; c < CC; ++c) {
         if (d[c] & kOn) {
@@ -361,7 +424,7 @@ __global__ __launch_bounds__(kT) void k_pers_cg(const SysDev* __restrict__ sds,
         }
       }
     }
-    ok = gather<1, 0u>(acc, sl0, rc.nblk, lb, tag + 2 * it, wait, sh);
+    ok = gather<1, 0u>(acc, sl0, rc.nblk, lb, tag + 2 * it, wait, sh, [] {});
     if (!ok) break;
     const double alpha = rho / (acc[0] + 1e-100);
     double ac2[2] = {0.0, 0.0};
@@ -380,7 +443,8 @@ __global__ __launch_bounds__(kT) void k_pers_cg(const SysDev* __restrict__ sds,
         }
       }
     }
-    ok = gather<2, 2u>(ac2, sl1, rc.nblk, lb, tag + 2 * it + 1, wait, sh);
+    ok = gather<2, 2u>(ac2, sl1, rc.nblk, lb, tag + 2 * it + 1, wait, sh,
+                       [&] { eh.load(b, tab, hg, sl1, tag + 2 * it + 1, wait); });
     if (!ok) break;
     const double dot_r = ac2[0];
     res = rmode == 1 ? ac2[1] / h3 : sqrt(dot_r / h3);
@@ -468,6 +532,8 @@ __global__ __launch_bounds__(kT) void k_pers_jacobi(const SysDev* __restrict__ s
   const int miniter = sc->miniter, maxiter = sc->maxiter;
   u64* const sl0 = rc.slots;
   u64* const sl1 = rc.slots + kPersMaxBlocks * kPersWords;
+  constexpr int HR = early_halo(8 * CC * ZC);
+  EarlyHalo<double, HR> eh(rc, lb);
   bool ok = true;
   __syncthreads();
   for (int it = 0; it < iters && !done; ++it) {
@@ -509,7 +575,9 @@ __global__ __launch_bounds__(kT) void k_pers_jacobi(const SysDev* __restrict__ s
       }
     }
     // (the gather's barriers separate these reads of LDS from the writes below)
-    ok = gather<1, 1u>(acc, (it & 1) ? sl1 : sl0, rc.nblk, lb, tag + it, wait, sh);
+    u64* const sl = (it & 1) ? sl1 : sl0;
+    ok = gather<1, 1u>(acc, sl, rc.nblk, lb, tag + it, wait, sh,
+                       [&] { eh.load(b, tab, ub, sl, tag + it, wait); });
     if (!ok) break;
     res = acc[0];
     iter += 1;
@@ -517,8 +585,9 @@ __global__ __launch_bounds__(kT) void k_pers_jacobi(const SysDev* __restrict__ s
       conv = res < tol ? 1 : 0;
       done = 1;
     }
+    eh.use(b, tab, [&](int, int, double w, int o) { sp[o] = w; });
     for_halo(b, tab, [&](int gi) { return ld_agent(ub + gi); },
-             [&](int, double w, int o) { sp[o] = w; });
+             [&](int, double w, int o) { sp[o] = w; }, HR);
 #pragma unroll
     for (int c = 0; c < CC; ++c) {
 #pragma unroll
@@ -630,6 +699,8 @@ __global__ __launch_bounds__(kT) void k_pers_pcg(const SysDev* __restrict__ sds,
   const int maxiter = sc->maxiter;
   u64* const sl0 = rc.slots;
   u64* const sl1 = rc.slots + kPersMaxBlocks * kPersWords;
+  constexpr int HR = early_halo((int)sizeof(T) * CC * ZC);
+  EarlyHalo<T, HR> eh(rc, lb);
   bool ok = true;
   struct RS {
     T r, S;
@@ -656,13 +727,16 @@ __global__ __launch_bounds__(kT) void k_pers_pcg(const SysDev* __restrict__ sds,
     }
     // p = r + beta p; x^ += alpha p_old as in k_pcg_spmv (fold 0 and 2)
     const T* hs = it == 0 ? rg : hg;
+    auto halo_p = [&](int h, T rh, T Sh, int o) {
+      const T pn = (T)((double)rh + beta * (double)ph[h]);
+      ph[h] = pn;
+      sp[o] = (double)Sh * (double)pn;
+    };
+    if (it > 0)
+      eh.use(b, tab, [&](int h, int gi, T rh, int o) { halo_p(h, rh, Sg[gi], o); });
     for_halo(
         b, tab, [&](int gi) { return RS{ld_agent(hs + gi), Sg[gi]}; },
-        [&](int h, RS v, int o) {
-          const T pn = (T)((double)v.r + beta * (double)ph[h]);
-          ph[h] = pn;
-          sp[o] = (double)v.S * (double)pn;
-        });
+        [&](int h, RS v, int o) { halo_p(h, v.r, v.S, o); }, it > 0 ? HR : 0);
 #pragma unroll
     for (int c = 0; c < CC; ++c) {
       if (!(d[c] & kOn)) continue;
@@ -711,7 +785,7 @@ __global__ __launch_bounds__(kT) void k_pers_pcg(const SysDev* __restrict__ sds,
         }
       }
     }
-    ok = gather<1, 0u>(acc, sl0, rc.nblk, lb, tag + 2 * it, wait, sh);
+    ok = gather<1, 0u>(acc, sl0, rc.nblk, lb, tag + 2 * it, wait, sh, [] {});
     if (!ok) break;
     const double pq = acc[0];
     fold = fold == 1 ? 2 : 0;
@@ -735,7 +809,8 @@ __global__ __launch_bounds__(kT) void k_pers_pcg(const SysDev* __restrict__ sds,
         }
       }
     }
-    ok = gather<1, 0u>(ac2, sl1, rc.nblk, lb, tag + 2 * it + 1, wait, sh);
+    ok = gather<1, 0u>(ac2, sl1, rc.nblk, lb, tag + 2 * it + 1, wait, sh,
+                       [&] { eh.load(b, tab, hg, sl1, tag + 2 * it + 1, wait); });
     if (!ok) break;
     const double rn = ac2[0];
     iter += 1;

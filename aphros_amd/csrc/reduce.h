@@ -13,17 +13,38 @@
 
 namespace aph {
 
+// x of another lane by a DPP control (within rows of 16 lanes)
+template <int Ctrl>
+__device__ __forceinline__ double dpp_of(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, Ctrl, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), Ctrl, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// x of a given lane, uniform
+__device__ __forceinline__ double lane_of(double x, int lane) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_readlane((int)b, lane);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// Sum (or max) over the wavefront, the same in every lane: within rows of 16
+// lanes by DPP moves (neighbour, pair, half-row mirror, row mirror), then over
+// the four rows.  Every lane must take part.  (A butterfly of __shfl_xor goes
+// through LDS twelve times: ~0.25 us against ~0.05 us.)
 template <int NV, unsigned MaxMask>
 __device__ __forceinline__ void wave_reduce(double (&v)[NV]) {
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
+    const bool mx = (MaxMask >> k) & 1u;
+    auto op = [mx](double a, double b) { return mx ? fmax(a, b) : a + b; };
     double x = v[k];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const double y = __shfl_xor(x, off, 64);
-      x = ((MaxMask >> k) & 1u) ? fmax(x, y) : x + y;
-    }
-    v[k] = x;
+    x = op(x, dpp_of<0xB1>(x));   // quad_perm 1 0 3 2
+    x = op(x, dpp_of<0x4E>(x));   // quad_perm 2 3 0 1
+    x = op(x, dpp_of<0x141>(x));  // row_half_mirror
+    x = op(x, dpp_of<0x140>(x));  // row_mirror
+    v[k] = op(op(lane_of(x, 0), lane_of(x, 16)), op(lane_of(x, 32), lane_of(x, 48)));
   }
 }
 
