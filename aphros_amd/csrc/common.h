@@ -135,6 +135,21 @@ struct Rec {
   int ty;  // rows of threads of a whole-row tile (k_mg_post: output rows + 2 halo rows)
 };
 
+// One system in a launch of the PCG kernels: its record with copies of the
+// system's and (cycle launches) the level's table entries, the coarser level's
+// beside it.  A workgroup then finds all it needs one dependent load away
+// (two in a launch of several systems, through the workgroup map) instead of
+// four (map, record, system, level), each of which may miss the L2, emptied
+// between launches of what other XCDs wrote; uniform 64-byte aligned loads into
+// SGPRs free 10-15 VGPRs of the sweeps.  Mixed multigrid solves 64^3 2.58 ->
+// 2.51 ms, 96^3 6.15 -> 5.89, 128^3 8.58 -> 8.30, 256^3 25.1 -> 24.7, 512^3
+// 178.9 -> 177.9.
+struct alignas(64) Ent {
+  Rec rc;
+  SysDev s;
+  MgLevel lv, lc;
+};
+
 // Physical workgroup id -> logical id such that the workgroups that run on
 // one XCD (ids x, x+8, x+16, ...) get a contiguous range of logical tiles and
 // share halo rows in that XCD's L2.

@@ -243,7 +243,8 @@ class Engine {
   Scalars* h_sc_ = nullptr;  // pinned mirror
   unsigned* d_counter_ = nullptr;
   SysDev* d_sds_ = nullptr;
-  Rec* d_rec_ = nullptr;
+  Rec* d_rec_ = nullptr;  // reference modes
+  Ent* d_ent_ = nullptr;  // PCG
   int* d_b2r_ = nullptr;
   long long rec_cap_ = 0, b2r_cap_ = 0;
   LaunchSet L_{};

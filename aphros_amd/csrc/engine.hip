@@ -171,6 +171,7 @@ Engine::~Engine() {
   if (d_counter_) (void)hipFree(d_counter_);
   if (d_sds_) (void)hipFree(d_sds_);
   if (d_rec_) (void)hipFree(d_rec_);
+  if (d_ent_) (void)hipFree(d_ent_);
   if (d_b2r_) (void)hipFree(d_b2r_);
   if (d_pers_) (void)hipFree(d_pers_);
   if (staging_) (void)hipFree(staging_);
@@ -1135,7 +1136,12 @@ int Engine::build_tables() {
   }
   if (nrec > rec_cap_) {
     if (d_rec_) APH_HIP(hipFree(d_rec_));
-    APH_HIP(hipMalloc(&d_rec_, sizeof(Rec) * std::max(1LL, nrec)));
+    if (d_ent_) APH_HIP(hipFree(d_ent_));
+    d_rec_ = nullptr;
+    d_ent_ = nullptr;
+    rec_cap_ = 0;
+    if (method_ == kPcg) APH_HIP(hipMalloc(&d_ent_, sizeof(Ent) * std::max(1LL, nrec)));
+    else APH_HIP(hipMalloc(&d_rec_, sizeof(Rec) * std::max(1LL, nrec)));
     rec_cap_ = nrec;
   }
   if (nb2r > b2r_cap_) {
@@ -1147,6 +1153,7 @@ int Engine::build_tables() {
   d_sds_ = nullptr;
   APH_HIP(hipMalloc(&d_sds_, sizeof(SysDev) * std::max(1, ns)));
   std::vector<Rec> recs;
+  std::vector<int> rlev;  // level of a record's entry (-1: none)
   recs.insert(recs.end(), rst.begin(), rst.end());
   recs.insert(recs.end(), rsm.begin(), rsm.end());
   recs.insert(recs.end(), rru.begin(), rru.end());
@@ -1154,6 +1161,7 @@ int Engine::build_tables() {
   b2r.insert(b2r.end(), bst.begin(), bst.end());
   for (int v : bsm) b2r.push_back(v);
   for (int v : bru) b2r.push_back(v);
+  rlev.assign(recs.size(), -1);
   size_t rec_lf_ofs[kMaxLevels], rec_lc_ofs[kMaxLevels], b2r_lf_ofs[kMaxLevels],
       b2r_lc_ofs[kMaxLevels], rec_lp_ofs[kMaxLevels], b2r_lp_ofs[kMaxLevels],
       rec_lt_ofs[kMaxLevels], b2r_lt_ofs[kMaxLevels];
@@ -1166,6 +1174,7 @@ int Engine::build_tables() {
     recs.insert(recs.end(), rlp[l].begin(), rlp[l].end());
     rec_lt_ofs[l] = recs.size();
     recs.insert(recs.end(), rlt[l].begin(), rlt[l].end());
+    rlev.resize(recs.size(), l);
     b2r_lf_ofs[l] = b2r.size();
     b2r.insert(b2r.end(), blf[l].begin(), blf[l].end());
     b2r_lc_ofs[l] = b2r.size();
@@ -1177,16 +1186,39 @@ int Engine::build_tables() {
   }
   if (ns > 0) {
     APH_HIP(hipMemcpy(d_sds_, sds.data(), sizeof(SysDev) * ns, hipMemcpyHostToDevice));
-    APH_HIP(hipMemcpy(d_rec_, recs.data(), sizeof(Rec) * nrec, hipMemcpyHostToDevice));
+    if (method_ == kPcg) {
+      std::vector<Ent> ents(nrec);
+      for (long long i = 0; i < nrec; ++i) {
+        const System& s = *slots_[launch_slots_[recs[i].sys]];
+        ents[i].rc = recs[i];
+        ents[i].s = sds[recs[i].sys];
+        const int l = rlev[i];
+        ents[i].lv = l >= 0 ? s.lev[l] : MgLevel{};
+        ents[i].lc = l >= 0 ? s.lev[l + 1] : MgLevel{};
+      }
+      APH_HIP(hipMemcpy(d_ent_, ents.data(), sizeof(Ent) * nrec, hipMemcpyHostToDevice));
+    } else {
+      APH_HIP(hipMemcpy(d_rec_, recs.data(), sizeof(Rec) * nrec, hipMemcpyHostToDevice));
+    }
     APH_HIP(hipMemcpy(d_b2r_, b2r.data(), sizeof(int) * nb2r, hipMemcpyHostToDevice));
   }
   L_.sds = d_sds_;
-  L_.rec_st = d_rec_;
-  L_.rec_sm = d_rec_ + rst.size();
-  L_.rec_ru = d_rec_ + rst.size() + rsm.size();
-  L_.b2r_st = d_b2r_;
-  L_.b2r_sm = d_b2r_ + bst.size();
-  L_.b2r_ru = d_b2r_ + bst.size() + bsm.size();
+  // PCG launches of one system need no workgroup map
+  auto map_of = [&](size_t ofs, size_t nsys) -> const int* {
+    return method_ == kPcg && nsys <= 1 ? nullptr : d_b2r_ + ofs;
+  };
+  if (method_ == kPcg) {
+    L_.ent_st = d_ent_;
+    L_.ent_sm = d_ent_ + rst.size();
+    L_.ent_ru = d_ent_ + rst.size() + rsm.size();
+  } else {
+    L_.rec_st = d_rec_;
+    L_.rec_sm = d_rec_ + rst.size();
+    L_.rec_ru = d_rec_ + rst.size() + rsm.size();
+  }
+  L_.b2r_st = map_of(0, rst.size());
+  L_.b2r_sm = map_of(bst.size(), rsm.size());
+  L_.b2r_ru = map_of(bst.size() + bsm.size(), rru.size());
   L_.nst = (int)bst.size();
   L_.nsm = (int)bsm.size();
   L_.nru = (int)bru.size();
@@ -1202,21 +1234,21 @@ int Engine::build_tables() {
   for (int l = 0; l < kMaxLevels; ++l) L_.bottom_at[l] = bottom_at[l];
   L_.deep = deep;
   for (int l = 0; l < kMaxLevels; ++l) {
-    L_.rec_lf[l] = d_rec_ + rec_lf_ofs[l];
-    L_.rec_lc[l] = d_rec_ + rec_lc_ofs[l];
-    L_.b2r_lf[l] = d_b2r_ + b2r_lf_ofs[l];
-    L_.b2r_lc[l] = d_b2r_ + b2r_lc_ofs[l];
+    L_.ent_lf[l] = d_ent_ + rec_lf_ofs[l];
+    L_.ent_lc[l] = d_ent_ + rec_lc_ofs[l];
+    L_.b2r_lf[l] = map_of(b2r_lf_ofs[l], rlf[l].size());
+    L_.b2r_lc[l] = map_of(b2r_lc_ofs[l], rlc[l].size());
     L_.nlf[l] = (int)blf[l].size();
     L_.nlc[l] = (int)blc[l].size();
     L_.post_fused[l] = post_fused[l];
     L_.post_plain[l] = post_plain[l];
     L_.vx_p[l] = fp32_ ? 4 : 2;
-    L_.rec_lp[l] = d_rec_ + rec_lp_ofs[l];
-    L_.b2r_lp[l] = d_b2r_ + b2r_lp_ofs[l];
+    L_.ent_lp[l] = d_ent_ + rec_lp_ofs[l];
+    L_.b2r_lp[l] = map_of(b2r_lp_ofs[l], rlp[l].size());
     L_.nlp[l] = (int)blp[l].size();
     L_.post_tile[l] = post_tile[l];
-    L_.rec_lt[l] = d_rec_ + rec_lt_ofs[l];
-    L_.b2r_lt[l] = d_b2r_ + b2r_lt_ofs[l];
+    L_.ent_lt[l] = d_ent_ + rec_lt_ofs[l];
+    L_.b2r_lt[l] = map_of(b2r_lt_ofs[l], rlt[l].size());
     L_.nlt[l] = (int)blt[l].size();
   }
   dirty_ = false;

@@ -21,11 +21,15 @@ struct LaunchSet {
   const int* b2r_sm = nullptr;
   const Rec* rec_ru = nullptr;  // one-cell-per-thread stencil launches (FP64 residuals)
   const int* b2r_ru = nullptr;
+  // the same for the PCG kernels (b2r null: one system)
+  const Ent* ent_st = nullptr;
+  const Ent* ent_sm = nullptr;
+  const Ent* ent_ru = nullptr;
   int nst = 0, nsm = 0, nru = 0;
   int vx_ru = 1;  // cells per thread of the PCG FP64 residual launch (rec_ru)
   int ns = 0;  // systems (one workgroup each in the finalize kernels)
   // multigrid preconditioner (pc = 1): per level l < nlev_max - 1, the
-  // one-cell-per-thread tiling of level l (rec_lf) and of level l+1 (rec_lc)
+  // one-cell-per-thread tiling of level l (ent_lf) and of level l+1 (ent_lc)
   // over the systems that coarsen below l
   int pc = 0;
   int nlev_max = 0;
@@ -36,25 +40,25 @@ struct LaunchSet {
   int coarse_sweeps = kCoarseSweeps;
   int coarse_lds = 0;  // dynamic LDS bytes of the bottom-levels kernel
   int vx_l[kMaxLevels] = {};  // cells per thread in x of the level-l sweeps
-  const Rec* rec_lf[kMaxLevels] = {};
+  const Ent* ent_lf[kMaxLevels] = {};
   const int* b2r_lf[kMaxLevels] = {};
   int nlf[kMaxLevels] = {};
-  const Rec* rec_lc[kMaxLevels] = {};
+  const Ent* ent_lc[kMaxLevels] = {};
   const int* b2r_lc[kMaxLevels] = {};
   int nlc[kMaxLevels] = {};
   // post-smoothing of level l: some systems fused (k_mg_post over the
-  // whole-row tiles rec_lp, cells per thread vx_p), some with two sweeps
+  // whole-row tiles ent_lp, cells per thread vx_p), some with two sweeps
   // (the sweep launches skip the systems whose level has post = 1)
   int post_fused[kMaxLevels] = {};
   int post_plain[kMaxLevels] = {};
   int vx_p[kMaxLevels] = {};
-  const Rec* rec_lp[kMaxLevels] = {};
+  const Ent* ent_lp[kMaxLevels] = {};
   const int* b2r_lp[kMaxLevels] = {};
   int nlp[kMaxLevels] = {};
   // small levels whose pre- and post-smoothing run as one tile launch each
   // (k_mg_tile, MgLevel::post == 2; 8^3 cells per workgroup, tiles_x/y/z)
   int post_tile[kMaxLevels] = {};
-  const Rec* rec_lt[kMaxLevels] = {};
+  const Ent* ent_lt[kMaxLevels] = {};
   const int* b2r_lt[kMaxLevels] = {};
   int nlt[kMaxLevels] = {};
   // event-profiled cycles only: the launches below level 0 as one replay of

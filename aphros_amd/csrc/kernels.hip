@@ -263,17 +263,16 @@ __device__ __forceinline__ Tile tile_of(const Rec& rc, const SysDev& s, int lb) 
 // x64, and x^ = alpha p_in (no read) in the iteration after, x^ being stale
 // since that update (xh_fold 1, 2).
 template <typename T, int VX, bool SC, bool XH>
-__global__ __launch_bounds__(kBlock) void k_pcg_spmv(const SysDev* __restrict__ sds,
-                                                     const Rec* __restrict__ recs,
-                                                     const int* __restrict__ b2r) {
+__global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ents, const int* __restrict__ b2r) {
   // arithmetic of the operator: FP64 for the Jacobi-scaled form, T with the
   // multigrid preconditioner (whose V-cycle absorbs FP32 rounding anyway)
   using A = typename std::conditional<SC, double, T>::type;
   using D = vec_t<A, VX>;
   __shared__ A su[2][kBlock * VX];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
-  const Rec rc = recs[b2r[b]];
-  const SysDev& s = sds[rc.sys];
+  const Ent& en = ents[b2r ? b2r[b] : 0];
+  const Rec rc = en.rc;
+  const SysDev& s = en.s;
   Scalars* sc = s.sc;
   if (sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
   const int lb = b - rc.blk0;
@@ -460,13 +459,12 @@ __device__ __forceinline__ void stream_range(long long n, int nblk, int lb, long
 // residual) follows.  x^ += alpha p is left to the CG operator of the next
 // iteration, which reads p anyway (k_pcg_spmv, XH).
 template <typename T, int VX>
-__global__ __launch_bounds__(kBlock) void k_pcg_update(const SysDev* __restrict__ sds,
-                                                       const Rec* __restrict__ recs,
-                                                       const int* __restrict__ b2r) {
+__global__ __launch_bounds__(kBlock) void k_pcg_update(const Ent* __restrict__ ents, const int* __restrict__ b2r) {
   using D = vec_t<double, VX>;
   const int b = blockIdx.x;
-  const Rec rc = recs[b2r[b]];
-  const SysDev& s = sds[rc.sys];
+  const Ent& en = ents[b2r ? b2r[b] : 0];
+  const Rec rc = en.rc;
+  const SysDev& s = en.s;
   Scalars* sc = s.sc;
   if (sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
   const int lb = b - rc.blk0;
@@ -515,13 +513,12 @@ __global__ __launch_bounds__(kBlock) void k_fin_pcg_update(const SysDev* __restr
 // the operator skips it; x^ counts as zero from here on (xh_fold 1: not read
 // again before the operator after next overwrites it).
 template <typename T, int VX>
-__global__ __launch_bounds__(kBlock) void k_ru_accum(const SysDev* __restrict__ sds,
-                                                     const Rec* __restrict__ recs,
-                                                     const int* __restrict__ b2r) {
+__global__ __launch_bounds__(kBlock) void k_ru_accum(const Ent* __restrict__ ents, const int* __restrict__ b2r) {
   using D = vec_t<double, VX>;
   const int b = blockIdx.x;
-  const Rec rc = recs[b2r[b]];
-  const SysDev& s = sds[rc.sys];
+  const Ent& en = ents[b2r ? b2r[b] : 0];
+  const Rec rc = en.rc;
+  const SysDev& s = en.s;
   Scalars* sc = s.sc;
   // a zero start: x64 and x^ are zero already, and so is their mean
   if (sc->done || !sc->ru || sc->zero_start) return;
@@ -566,14 +563,13 @@ __global__ __launch_bounds__(kBlock) void k_fin_ru_accum(const SysDev* __restric
 // x of planes z-1, z, z+1 and e_z of plane z-1 in registers, the x plane of
 // the tile in LDS for the x and y neighbours.
 template <typename T, int VX>
-__global__ __launch_bounds__(kBlock) void k_ru_resid(const SysDev* __restrict__ sds,
-                                                     const Rec* __restrict__ recs,
-                                                     const int* __restrict__ b2r) {
+__global__ __launch_bounds__(kBlock) void k_ru_resid(const Ent* __restrict__ ents, const int* __restrict__ b2r) {
   static_assert(VX == 1, "one cell per thread");
   __shared__ double su[2][kBlock];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
-  const Rec rc = recs[b2r[b]];
-  const SysDev& s = sds[rc.sys];
+  const Ent& en = ents[b2r ? b2r[b] : 0];
+  const Rec rc = en.rc;
+  const SysDev& s = en.s;
   Scalars* sc = s.sc;
   if (sc->done || !sc->ru) return;
   const int lb = b - rc.blk0;
@@ -664,14 +660,13 @@ __global__ __launch_bounds__(kBlock) void k_ru_resid(const SysDev* __restrict__ 
 // k_ru_resid with 2 cells per thread (even nx): 16-byte FP64 loads of x, b
 // and the coefficients; the same per-cell operation order and partials.
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_ru_resid2(const SysDev* __restrict__ sds,
-                                                      const Rec* __restrict__ recs,
-                                                      const int* __restrict__ b2r) {
+__global__ __launch_bounds__(kBlock) void k_ru_resid2(const Ent* __restrict__ ents, const int* __restrict__ b2r) {
   using D2 = vec_t<double, 2>;
   __shared__ double su[2][kBlock * 2];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
-  const Rec rc = recs[b2r[b]];
-  const SysDev& s = sds[rc.sys];
+  const Ent& en = ents[b2r ? b2r[b] : 0];
+  const Rec rc = en.rc;
+  const SysDev& s = en.s;
   Scalars* sc = s.sc;
   if (sc->done || !sc->ru) return;
   const int lb = b - rc.blk0;
@@ -1015,9 +1010,7 @@ __device__ __forceinline__ Cell cell_of(const Rec& rc, int lb, int nx, int ny, i
 // L0: the launch on level 0 (a separate instance, so that profiles keep the
 // bandwidth-bound fine-grid sweeps apart from the coarse levels).
 template <typename T, int VX, int MODE, bool DOT, bool L0>
-__global__ __launch_bounds__(kBlock) void k_mg_sweep(const SysDev* __restrict__ sds,
-                                                     const Rec* __restrict__ recs,
-                                                     const int* __restrict__ b2r, int l_arg,
+__global__ __launch_bounds__(kBlock) void k_mg_sweep(const Ent* __restrict__ ents, const int* __restrict__ b2r, int l_arg,
                                                      int zin, int zout, int wl, int so,
                                                      int addzs) {
   const int l = L0 ? 0 : l_arg;
@@ -1027,15 +1020,16 @@ __global__ __launch_bounds__(kBlock) void k_mg_sweep(const SysDev* __restrict__ 
   __shared__ T su[2][kBlock * VX];
   __shared__ T sacc[MODE == 3 ? kBlock * NP : 1];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
-  const Rec rc = recs[b2r[b]];
-  const SysDev& s = sds[rc.sys];
+  const Ent& en = ents[b2r ? b2r[b] : 0];
+  const Rec rc = en.rc;
+  const SysDev& s = en.s;
   if (s.sc->done) return;
   // a launch of the second coarse correction below W level wl: only the
   // systems with more than wl W levels take part
   if (wl >= 0 && wl >= s.mg_w) return;
   // so: the start of newly prepared systems (first == 1); running ones skip
   if (so && !s.sc->first) return;
-  const MgLevel& Lv = s.lev[l];
+  const MgLevel& Lv = en.lv;
   // this system's level runs fused kernels (k_mg_pre, k_mg_post) instead
   if ((MODE == 0 || MODE == 1 || MODE == 2 || MODE == 3) && Lv.post) return;
   // zin / zout < 0: the level's pre-smoothed iterate (z[0] if fused, else z[1])
@@ -1070,7 +1064,7 @@ __global__ __launch_bounds__(kBlock) void k_mg_sweep(const SysDev* __restrict__ 
   gmp<T> __restrict__ rco = nullptr;
   int cnx = 0, cny = 0;
   if constexpr (MODE == 2 || MODE == 3) {
-    const MgLevel& Lc = s.lev[l + 1];
+    const MgLevel& Lc = en.lc;
     if constexpr (MODE == 2) {
       zc = (gcp<T>)Lc.z[l + 1 == s.nlev - 1 ? 0 : 1];
     } else {
@@ -1276,9 +1270,7 @@ __global__ __launch_bounds__(kBlock) void k_mg_sweep(const SysDev* __restrict__ 
 // stored nor restricted (edges are even, tiles start at multiples of 8).
 // DOT (POST on level 0): partials of (r, z[1]).
 template <bool PRE, bool DOT>
-__global__ __launch_bounds__(kTileBlock) void k_mg_tile(const SysDev* __restrict__ sds,
-                                                        const Rec* __restrict__ recs,
-                                                        const int* __restrict__ b2r, int l,
+__global__ __launch_bounds__(kTileBlock) void k_mg_tile(const Ent* __restrict__ ents, const int* __restrict__ b2r, int l,
                                                         int wl, int so, int addzs) {
   constexpr int B = kTile + 4;            // box rows per edge (y, z)
   constexpr int W = kTile + 8;            // cells per staged row (x)
@@ -1291,13 +1283,14 @@ __global__ __launch_bounds__(kTileBlock) void k_mg_tile(const SysDev* __restrict
   __shared__ __align__(16) unsigned short sK[NR * NG * 16];  // kx[4] ky[4] kz[4] dinv[4] per group
   __shared__ float sres[PRE ? NT : 1];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
-  const Rec rc = recs[b2r[b]];
-  const SysDev& s = sds[rc.sys];
+  const Ent& en = ents[b2r ? b2r[b] : 0];
+  const Rec rc = en.rc;
+  const SysDev& s = en.s;
   if (s.sc->done) return;
   if (wl >= 0 && wl >= s.mg_w) return;
   if (so && !s.sc->first) return;
-  const MgLevel& Lv = s.lev[l];
-  const MgLevel& Lc = s.lev[l + 1];
+  const MgLevel& Lv = en.lv;
+  const MgLevel& Lc = en.lc;
   const int nx = Lv.nx, ny = Lv.ny, nz = Lv.nz;
   const int lb = b - rc.blk0;
   const int x0 = (lb % rc.tiles_x) * kTile;
@@ -1421,20 +1414,19 @@ __global__ __launch_bounds__(kTileBlock) void k_mg_tile(const SysDev* __restrict
 // Residual of level l restricted to level l+1: r_{l+1}[C] = sum over the
 // 2x2x2 children c of (r - L z)_c.  One thread per coarse cell.
 template <typename T, bool L0>
-__global__ __launch_bounds__(kBlock) void k_mg_restrict(const SysDev* __restrict__ sds,
-                                                        const Rec* __restrict__ recs,
-                                                        const int* __restrict__ b2r, int l_arg,
+__global__ __launch_bounds__(kBlock) void k_mg_restrict(const Ent* __restrict__ ents, const int* __restrict__ b2r, int l_arg,
                                                         int zin, int wl, int so) {
   const int l = L0 ? 0 : l_arg;
   const int b = xcd_remap(blockIdx.x, gridDim.x);
-  const Rec rc = recs[b2r[b]];
-  const SysDev& s = sds[rc.sys];
+  const Ent& en = ents[b2r ? b2r[b] : 0];
+  const Rec rc = en.rc;
+  const SysDev& s = en.s;
   if (s.sc->done) return;
   if (wl >= 0 && wl >= s.mg_w) return;
   if (so && !s.sc->first) return;
-  const MgLevel& Lf = s.lev[l];
+  const MgLevel& Lf = en.lv;
   if (Lf.post) return;  // restricted by k_mg_pre
-  const MgLevel& Lc = s.lev[l + 1];
+  const MgLevel& Lc = en.lc;
   const LevelView<T> F(Lf);
   const int lb = b - rc.blk0;
   const Cell c = cell_of(rc, lb, Lc.nx, Lc.ny, Lc.nz);
@@ -1475,24 +1467,22 @@ __global__ __launch_bounds__(kBlock) void k_mg_restrict(const SysDev* __restrict
 // hits).  The u rows just outside the tile (for the halo rows' v) and the u
 // planes before and after the tile come from memory.
 template <typename T, int VX, bool DOT, bool L0>
-__global__ __launch_bounds__(kPostBlock) void k_mg_post(const SysDev* __restrict__ sds,
-                                                        const Rec* __restrict__ recs,
-                                                        const int* __restrict__ b2r, int l_arg,
+__global__ __launch_bounds__(kPostBlock) void k_mg_post(const Ent* __restrict__ ents, const int* __restrict__ b2r, int l_arg,
                                                         int wl, int so, int addzs) {
   const int l = L0 ? 0 : l_arg;
   using V = vec_t<T, VX>;
   __shared__ T su[2][kPostBlock * VX];
   __shared__ T sv[2][kPostBlock * VX];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
-  // launch tables (recs, b2r, sds) and level tables (s.lev) are device
-  // arrays written by the host between launches only
-  const Rec rc = cload(gtab(recs + cload(gtab(b2r + b))));
-  const SysDev s = cload(gtab(sds + rc.sys));
+  // launch tables (ents, b2r) are device arrays written by the host between launches only
+  const gcp<Ent> en = gtab(ents + (b2r ? cload(gtab(b2r + b)) : 0));
+  const Rec rc = cload(&en->rc);
+  const SysDev s = cload(&en->s);
   if (s.sc->done) return;
   if (wl >= 0 && wl >= s.mg_w) return;
   if (so && !s.sc->first) return;
-  const MgLevel Lv = cload(gtab(s.lev + l));
-  const MgLevel Lc = cload(gtab(s.lev + l + 1));
+  const MgLevel Lv = cload(&en->lv);
+  const MgLevel Lc = cload(&en->lc);
   const int nx = Lv.nx, ny = Lv.ny, nz = Lv.nz;
   const int lb = b - rc.blk0;
   const int lx = rc.lx, ty = rc.ty;  // lx * VX == nx, ty <= kPostBlock / lx
@@ -1661,9 +1651,7 @@ __device__ __forceinline__ vec_t<float, 4> bf4(unsigned a, unsigned b) {
 // ky and kx of the neighbouring cells instead of loading them again.  Same
 // arithmetic as k_mg_post.
 template <bool DOT, bool L0>
-__global__ __launch_bounds__(kPostBlock) void k_mg_post4(const SysDev* __restrict__ sds,
-                                                         const Rec* __restrict__ recs,
-                                                         const int* __restrict__ b2r,
+__global__ __launch_bounds__(kPostBlock) void k_mg_post4(const Ent* __restrict__ ents, const int* __restrict__ b2r,
                                                          int l_arg, int wl, int so, int addzs) {
   using V = vec_t<float, 4>;
   using U4 = vec_t<unsigned, 4>;
@@ -1674,13 +1662,14 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_post4(const SysDev* __restric
   __shared__ float su[2][kPostBlock * VX];
   __shared__ float sv[2][kPostBlock * VX];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
-  const Rec rc = cload(gtab(recs + cload(gtab(b2r + b))));
-  const SysDev s = cload(gtab(sds + rc.sys));
+  const gcp<Ent> en = gtab(ents + (b2r ? cload(gtab(b2r + b)) : 0));
+  const Rec rc = cload(&en->rc);
+  const SysDev s = cload(&en->s);
   if (s.sc->done) return;
   if (wl >= 0 && wl >= s.mg_w) return;
   if (so && !s.sc->first) return;
-  const MgLevel Lv = cload(gtab(s.lev + l));
-  const MgLevel Lc = cload(gtab(s.lev + l + 1));
+  const MgLevel Lv = cload(&en->lv);
+  const MgLevel Lc = cload(&en->lc);
   const int nx = Lv.nx, ny = Lv.ny, nz = Lv.nz;
   const int lb = b - rc.blk0;
   const int lx = rc.lx, ty = rc.ty;
@@ -1868,9 +1857,7 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_post4(const SysDev* __restric
 // rows hand their sums to the even row above).  One barrier per step; u and z
 // planes double-buffered in LDS.
 template <typename T, int VX, bool L0>
-__global__ __launch_bounds__(kPostBlock) void k_mg_pre(const SysDev* __restrict__ sds,
-                                                       const Rec* __restrict__ recs,
-                                                       const int* __restrict__ b2r, int l_arg,
+__global__ __launch_bounds__(kPostBlock) void k_mg_pre(const Ent* __restrict__ ents, const int* __restrict__ b2r, int l_arg,
                                                        int wl, int so) {
   static_assert(VX >= 2, "x pairs of the restriction are summed in the thread");
   constexpr int NP = VX / 2;
@@ -1880,15 +1867,15 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_pre(const SysDev* __restrict_
   __shared__ T sz[2][kPostBlock * VX];
   __shared__ T sacc[kPostBlock * NP];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
-  // launch tables (recs, b2r, sds) and level tables (s.lev) are device
-  // arrays written by the host between launches only
-  const Rec rc = cload(gtab(recs + cload(gtab(b2r + b))));
-  const SysDev s = cload(gtab(sds + rc.sys));
+  // launch tables (ents, b2r) are device arrays written by the host between launches only
+  const gcp<Ent> en = gtab(ents + (b2r ? cload(gtab(b2r + b)) : 0));
+  const Rec rc = cload(&en->rc);
+  const SysDev s = cload(&en->s);
   if (s.sc->done) return;
   if (wl >= 0 && wl >= s.mg_w) return;
   if (so && !s.sc->first) return;
-  const MgLevel Lv = cload(gtab(s.lev + l));
-  const MgLevel Lc = cload(gtab(s.lev + l + 1));
+  const MgLevel Lv = cload(&en->lv);
+  const MgLevel Lc = cload(&en->lc);
   const int nx = Lv.nx, ny = Lv.ny, nz = Lv.nz;
   const int lb = b - rc.blk0;
   const int lx = rc.lx, ty = rc.ty;  // lx * VX == nx, ty even, <= kPostBlock / lx
@@ -2056,9 +2043,7 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_pre(const SysDev* __restrict_
 // k + 1; plane k-1's packed coefficients, r, ky and kx wait in LDS slots for
 // the residual.  Same arithmetic as k_mg_pre.
 template <bool L0>
-__global__ __launch_bounds__(kPostBlock) void k_mg_pre4(const SysDev* __restrict__ sds,
-                                                        const Rec* __restrict__ recs,
-                                                        const int* __restrict__ b2r, int l_arg,
+__global__ __launch_bounds__(kPostBlock) void k_mg_pre4(const Ent* __restrict__ ents, const int* __restrict__ b2r, int l_arg,
                                                         int wl, int so) {
   using V = vec_t<float, 4>;
   using U4 = vec_t<unsigned, 4>;
@@ -2077,13 +2062,14 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_pre4(const SysDev* __restrict
   __shared__ unsigned skx[kPostBlock];               // kx of cell xm, plane k-1
   __shared__ vec_t<float, NP> spend[kPostBlock];     // even rows' pending sums
   const int b = xcd_remap(blockIdx.x, gridDim.x);
-  const Rec rc = cload(gtab(recs + cload(gtab(b2r + b))));
-  const SysDev s = cload(gtab(sds + rc.sys));
+  const gcp<Ent> en = gtab(ents + (b2r ? cload(gtab(b2r + b)) : 0));
+  const Rec rc = cload(&en->rc);
+  const SysDev s = cload(&en->s);
   if (s.sc->done) return;
   if (wl >= 0 && wl >= s.mg_w) return;
   if (so && !s.sc->first) return;
-  const MgLevel Lv = cload(gtab(s.lev + l));
-  const MgLevel Lc = cload(gtab(s.lev + l + 1));
+  const MgLevel Lv = cload(&en->lv);
+  const MgLevel Lc = cload(&en->lc);
   const int nx = Lv.nx, ny = Lv.ny, nz = Lv.nz;
   const int lb = b - rc.blk0;
   const int lx = rc.lx, ty = rc.ty;
@@ -3426,41 +3412,41 @@ static void launch_sweep_l(const LaunchSet& L, hipStream_t st, int l, int zin, i
                            int wl, int addzs) {
   switch (L.vx_l[l]) {
     case 4:
-      APH_LAUNCH((k_mg_sweep<T, 4, MODE, DOT, L0>), L.nlf[l], st, L.sds, L.rec_lf[l],
+      APH_LAUNCH((k_mg_sweep<T, 4, MODE, DOT, L0>), L.nlf[l], st, L.ent_lf[l],
                  L.b2r_lf[l], l, zin, zout, wl, L.start_only, addzs);
       break;
     case 2:
-      APH_LAUNCH((k_mg_sweep<T, 2, MODE, DOT, L0>), L.nlf[l], st, L.sds, L.rec_lf[l],
+      APH_LAUNCH((k_mg_sweep<T, 2, MODE, DOT, L0>), L.nlf[l], st, L.ent_lf[l],
                  L.b2r_lf[l], l, zin, zout, wl, L.start_only, addzs);
       break;
     default:
       if constexpr (MODE == 3) {
-        APH_LAUNCH((k_mg_restrict<T, L0>), L.nlc[l], st, L.sds, L.rec_lc[l], L.b2r_lc[l], l,
+        APH_LAUNCH((k_mg_restrict<T, L0>), L.nlc[l], st, L.ent_lc[l], L.b2r_lc[l], l,
                    zin, wl, L.start_only);
       } else {
-        APH_LAUNCH((k_mg_sweep<T, 1, MODE, DOT, L0>), L.nlf[l], st, L.sds, L.rec_lf[l],
-                   L.b2r_lf[l], l, zin, zout, wl, L.start_only, addzs);
+        APH_LAUNCH((k_mg_sweep<T, 1, MODE, DOT, L0>), L.nlf[l], st, L.ent_lf[l],
+                 L.b2r_lf[l], l, zin, zout, wl, L.start_only, addzs);
       }
       break;
   }
 }
 
-// pre-smoothing + restriction of level l, fused, for the systems in rec_lp[l]
+// pre-smoothing + restriction of level l, fused, for the systems in ent_lp[l]
 template <typename T, bool L0>
 static void launch_pre_l(const LaunchSet& L, hipStream_t st, int l, int wl) {
   const dim3 g(L.nlp[l]), t(kPostBlock);
   if (L.vx_p[l] == 4) {
     if constexpr (sizeof(T) == 4) {
-      hipLaunchKernelGGL((k_mg_pre4<L0>), g, t, 0, st, L.sds, L.rec_lp[l], L.b2r_lp[l], l, wl,
+      hipLaunchKernelGGL((k_mg_pre4<L0>), g, t, 0, st, L.ent_lp[l], L.b2r_lp[l], l, wl,
                          L.start_only);
     }
   } else {
-    hipLaunchKernelGGL((k_mg_pre<T, 2, L0>), g, t, 0, st, L.sds, L.rec_lp[l], L.b2r_lp[l], l, wl,
+    hipLaunchKernelGGL((k_mg_pre<T, 2, L0>), g, t, 0, st, L.ent_lp[l], L.b2r_lp[l], l, wl,
                        L.start_only);
   }
 }
 
-// both post-smoothing sweeps of level l, fused, for the systems in rec_lp[l]
+// both post-smoothing sweeps of level l, fused, for the systems in ent_lp[l]
 template <typename T, bool DOT, bool L0>
 static void launch_post_l(const LaunchSet& L, hipStream_t st, int l, int wl, int addzs) {
   const dim3 g(L.nlp[l]), t(kPostBlock);
@@ -3469,16 +3455,16 @@ static void launch_post_l(const LaunchSet& L, hipStream_t st, int l, int wl, int
   switch (L.vx_p[l]) {
     case 4:
       if constexpr (sizeof(T) == 4) {
-        hipLaunchKernelGGL((k_mg_post4<DOT, L0>), g, t, 0, st, L.sds, L.rec_lp[l],
-                           L.b2r_lp[l], l, wl, L.start_only, addzs);
+        hipLaunchKernelGGL((k_mg_post4<DOT, L0>), g, t, 0, st, L.ent_lp[l], L.b2r_lp[l], l,
+                           wl, L.start_only, addzs);
       }
       break;
     case 2:
-      hipLaunchKernelGGL((k_mg_post<T, 2, DOT, L0>), g, t, 0, st, L.sds, L.rec_lp[l], L.b2r_lp[l],
+      hipLaunchKernelGGL((k_mg_post<T, 2, DOT, L0>), g, t, 0, st, L.ent_lp[l], L.b2r_lp[l],
                          l, wl, L.start_only, addzs);
       break;
     default:
-      hipLaunchKernelGGL((k_mg_post<T, 1, DOT, L0>), g, t, 0, st, L.sds, L.rec_lp[l], L.b2r_lp[l],
+      hipLaunchKernelGGL((k_mg_post<T, 1, DOT, L0>), g, t, 0, st, L.ent_lp[l], L.b2r_lp[l],
                          l, wl, L.start_only, addzs);
       break;
   }
@@ -3534,8 +3520,8 @@ static void launch_cycle(const LaunchSet& L, hipStream_t st, int l, int wl, bool
   if (L.post_tile[l]) {
     mark(l == 0 ? 0 : 2);
     if constexpr (sizeof(T) == 4) {
-      hipLaunchKernelGGL((k_mg_tile<true, false>), dim3(L.nlt[l]), dim3(kTileBlock), 0, st, L.sds,
-                         L.rec_lt[l], L.b2r_lt[l], l, wl, L.start_only, 0);
+      hipLaunchKernelGGL((k_mg_tile<true, false>), dim3(L.nlt[l]), dim3(kTileBlock), 0, st,
+                         L.ent_lt[l], L.b2r_lt[l], l, wl, L.start_only, 0);
     }
   }
   if (l == 0 && L.below0) {
@@ -3560,10 +3546,10 @@ static void launch_cycle(const LaunchSet& L, hipStream_t st, int l, int wl, bool
     if constexpr (sizeof(T) == 4) {
       if (l == 0) {
         hipLaunchKernelGGL((k_mg_tile<false, true>), dim3(L.nlt[l]), dim3(kTileBlock), 0, st,
-                           L.sds, L.rec_lt[l], L.b2r_lt[l], l, wl, L.start_only, 0);
+                           L.ent_lt[l], L.b2r_lt[l], l, wl, L.start_only, 0);
       } else {
         hipLaunchKernelGGL((k_mg_tile<false, false>), dim3(L.nlt[l]), dim3(kTileBlock), 0, st,
-                           L.sds, L.rec_lt[l], L.b2r_lt[l], l, wl, L.start_only,
+                           L.ent_lt[l], L.b2r_lt[l], l, wl, L.start_only,
                            second ? 1 : 0);
       }
     }
@@ -3642,22 +3628,22 @@ template <typename T, int VX>
 static void launch_pcg_kernel(const LaunchSet& L, hipStream_t st, int j) {
   switch (j) {
     case 0:
-      if (L.pc) APH_LAUNCH((k_pcg_spmv<T, VX, false, true>), L.nst, st, L.sds, L.rec_st, L.b2r_st);
-      else APH_LAUNCH((k_pcg_spmv<T, VX, true, true>), L.nst, st, L.sds, L.rec_st, L.b2r_st);
+      if (L.pc) APH_LAUNCH((k_pcg_spmv<T, VX, false, true>), L.nst, st, L.ent_st, L.b2r_st);
+      else APH_LAUNCH((k_pcg_spmv<T, VX, true, true>), L.nst, st, L.ent_st, L.b2r_st);
       break;
     case 8: launch_vcycle<T>(L, st); break;
     case 1: APH_LAUNCH(k_fin_pcg_spmv, L.ns, st, L.sds); break;
     case 2:
-      APH_LAUNCH((k_pcg_update<T, VX>), L.nsm, st, L.sds, L.rec_sm, L.b2r_sm);
+      APH_LAUNCH((k_pcg_update<T, VX>), L.nsm, st, L.ent_sm, L.b2r_sm);
       break;
     case 3: APH_LAUNCH(k_fin_pcg_update, L.ns, st, L.sds); break;
     case 4:
-      APH_LAUNCH((k_ru_accum<T, VX>), L.nsm, st, L.sds, L.rec_sm, L.b2r_sm);
+      APH_LAUNCH((k_ru_accum<T, VX>), L.nsm, st, L.ent_sm, L.b2r_sm);
       break;
     case 5: APH_LAUNCH(k_fin_ru_accum, L.ns, st, L.sds); break;
     case 6:
-      if (L.vx_ru == 2) APH_LAUNCH(k_ru_resid2<T>, L.nru, st, L.sds, L.rec_ru, L.b2r_ru);
-      else APH_LAUNCH((k_ru_resid<T, 1>), L.nru, st, L.sds, L.rec_ru, L.b2r_ru);
+      if (L.vx_ru == 2) APH_LAUNCH(k_ru_resid2<T>, L.nru, st, L.ent_ru, L.b2r_ru);
+      else APH_LAUNCH((k_ru_resid<T, 1>), L.nru, st, L.ent_ru, L.b2r_ru);
       break;
     default: APH_LAUNCH(k_fin_ru_resid, L.ns, st, L.sds); break;
   }
