@@ -44,6 +44,9 @@ struct Scalars {
                    // 2 stale, the next operator writes x^ = alpha p_in
   int pers_fail;   // a resident launch gave up waiting (persist.hip); the state
                    // is that before the launch
+  // what the CG operator of a lean system (SysDev::lean) leaves for its update,
+  // and rz is (r, z) itself rather than a sum over its partials
+  int cur_next, iter_next, xf_next, rz_ok;
   int zero_start;  // PCG: the start's x64 is zero-filled (the start's
                    // residual is b, with no accumulation pass); cleared by it
 };
@@ -97,7 +100,15 @@ struct SysDev {
   double* pp[2];
   double* qq;
   // reductions
-  double* partials;  // 4 * nblk_max doubles
+  double* partials;
+  // partials of x64's sum, the FP64 residual and (r, z): regions of their own
+  // in lean systems, else `partials` too
+  double* pacc;
+  double* pres;
+  double* ppc;
+  // 1: a multigrid system whose reductions are finished by every workgroup of
+  // the kernel that needs the result (kernels.hip), not by finalize kernels
+  int lean;
   unsigned* counter;
   Scalars* sc;
   int neg;  // 1 if the diagonal is negative (A = -L): r^ = -S r64

@@ -67,6 +67,13 @@ constexpr long long kFuseMinCells64 = 1LL << 19, kFuseMinCells32 = 3LL << 20;
 // 73, 64^3 84 -> 80, 80^3 112 -> 108, but 96^3 113 -> 117 and 128^3 135 -> 160:
 // the tiles' halos (4.5x the level's bytes) then miss L2.
 constexpr long long kTileMaxCells = 1LL << 19;
+// Multigrid systems of at most this many cells finish their reductions in the
+// kernels that need them (SysDev::lean).  ms per solve, finalize kernels ->
+// lean: mixed 16^3 2.80 -> 2.48, 32^3 3.03 -> 2.53, 64^3 2.52 -> 2.18, 96^3 5.89
+// -> 5.57, 128^3 8.17 -> 7.79, 192^3 15.6 -> 15.4; FP64 64^3 5.96 -> 5.35, 128^3
+// 12.2 -> 11.7, 192^3 the same; above, the operator's reads of r cost more than
+// the launches: 224 x 192 x 256 23.5 -> 24.2, 320^3 42.9 -> 44.3 (256^3 the same).
+constexpr long long kLeanCells = 1LL << 23;
 // Iterations of one resident launch: a launch costs about 30 us more than its
 // iterations (of 7 to 25 us); the server's steps are shorter, so that a new
 // request waits a few milliseconds at most.
@@ -971,6 +978,7 @@ int Engine::build_tables() {
     }
   }
   // post-smoothing per level: fused for the systems whose level says so
+  L_.any_lean = L_.any_plain = 0;
   int post_fused[kMaxLevels] = {}, post_plain[kMaxLevels] = {}, post_tile[kMaxLevels] = {};
   std::vector<std::vector<Rec>> rlp(kMaxLevels), rlt(kMaxLevels);
   std::vector<std::vector<int>> blp(kMaxLevels), blt(kMaxLevels);
@@ -1059,9 +1067,11 @@ int Engine::build_tables() {
       }
     }
     s.dev.nblk_pc = nblk_pc;
-    // partials: 3 values per block of the largest reducing launch of this system
-    const int nmax = std::max(std::max(a.nblk, nblk_pc), std::max(b.nblk, c.nblk));
-    const long long need = 3LL * nmax * 8;
+    // partials: 3 values per block of the largest reducing launch of this
+    // system; lean: 4 (operator) + 1 (x64) + 3 (residual) + 1 ((r, z)), apart
+    const long long nmax = std::max(std::max(a.nblk, nblk_pc), std::max(b.nblk, c.nblk));
+    s.dev.lean = pc_ && s.dev.mg_lb > 0 && s.n <= kLeanCells ? 1 : 0;
+    const long long need = (s.dev.lean ? 9 : 3) * nmax * 8;
     if (need > s.partials_cap) {
       if (s.partials) APH_HIP(hipFree(s.partials));
       s.partials = nullptr;
@@ -1070,6 +1080,10 @@ int Engine::build_tables() {
       s.partials_cap = need;
     }
     s.dev.partials = (double*)s.partials;
+    s.dev.pacc = s.dev.partials + (s.dev.lean ? 4 * nmax : 0);
+    s.dev.pres = s.dev.partials + (s.dev.lean ? 5 * nmax : 0);
+    s.dev.ppc = s.dev.partials + (s.dev.lean ? 8 * nmax : 0);
+    (s.dev.lean ? L_.any_lean : L_.any_plain) = 1;
     s.dev.nblk_st = a.nblk;
     s.dev.nblk_sm = b.nblk;
     s.dev.nblk_ru = c.nblk;
@@ -1275,7 +1289,7 @@ int Engine::capture() {
   const int nk = iter_kernels(method_, pc_ ? 1 : 0);
   const int ng = graph_kernels(method_, pc_ ? 1 : 0);  // of them in the graph
   // launches per iteration (the multigrid cycle counts as one kernel in nk)
-  const int nl = ng + (pc_ ? vcycle_launches(L_) - 1 : 0);
+  const int nl = (L_.any_plain ? ng + (pc_ ? 1 : 0) : 4) + (pc_ ? vcycle_launches(L_) - 2 : 0);
   int k = check_every_;
   if (k <= 0) {
     // about 4 ms of work per replay (iterations past convergence cost a
@@ -1306,9 +1320,11 @@ int Engine::capture() {
     }
   }
   APH_HIP(hipStreamBeginCapture(st_, hipStreamCaptureModeThreadLocal));
+  LaunchSet Lc = L_;
   for (int i = 0; i < k; ++i) {
+    Lc.close = i + 1 == k ? 1 : 0;
     for (int j = 0; j < ng; ++j) {
-      const hipError_t e = launch_kernel(method_, fp32_, vx_, L_, st_, j);
+      const hipError_t e = launch_kernel(method_, fp32_, vx_, Lc, st_, j);
       if (e != hipSuccess) {
         hipGraph_t g = nullptr;
         (void)hipStreamEndCapture(st_, &g);

@@ -239,6 +239,151 @@ __device__ __forceinline__ Tile tile_of(const Rec& rc, const SysDev& s, int lb) 
 }
 
 // ===========================================================================
+// Lean systems (SysDev::lean: multigrid, at most kLeanCells cells).  The kernel
+// after a reducing one sums its partials itself, every workgroup the same way,
+// and workgroup 0 stores what the iteration keeps; no field is stored by a
+// kernel whose other workgroups still read it.  The operator also forms (r, r),
+// (r, q) and (q, q), so the update knows |r - alpha q|^2, and with it whether a
+// reliable update follows, before it touches r.  Six of an iteration's launches
+// fall away (four finalize kernels, an accumulation pass, (r, z)), which cost
+// ~4 us each while the kernels of a small system take 5 to 10 us: 64^3 63 -> 54
+// us per iteration of a solve, 32^3 46 -> 38.
+// ===========================================================================
+
+// Before the operator: beta from (r, z).  False: the solve ends.
+__device__ __forceinline__ bool lean_beta(const SysDev& s, Scalars* sc, int lb, double& beta) {
+  const bool ok = sc->rz_ok;
+  double acc[1] = {sc->rz};
+  if (!ok) reduce_partials<1, 0u>(acc, s.ppc, s.nblk_pc);
+  const double rz = acc[0];
+  beta = sc->first ? 0.0 : rz / sc->rho;
+  if (lb == 0 && threadIdx.x == 0) {
+    if (!isfinite(rz)) {
+      sc->status = 6;
+      sc->done = 1;
+    }
+    if (!ok) sc->rz = rz;
+    sc->cur_next = sc->cur ^ 1;
+    sc->iter_next = sc->iter + 1;
+    sc->xf_next = sc->xh_fold == 1 ? 2 : 0;
+  }
+  return isfinite(rz);
+}
+
+// Before the update: alpha, and whether a reliable update follows (1), not (0),
+// or the solve ends (-1).
+__device__ __forceinline__ int lean_step(const SysDev& s, Scalars* sc, int lb, double& alpha) {
+  double d[4];  // (p, q), (r, r), (r, q), (q, q)
+  reduce_partials<4, 0u>(d, s.partials, s.nblk_st);
+  const bool bad = !(d[0] != 0.0) || !isfinite(d[0]);
+  const double rz = sc->rz;
+  const int iter = sc->iter_next;
+  alpha = rz / d[0];
+  const double rn = d[1] - alpha * (2.0 * d[2] - alpha * d[3]);
+  const double rs = sqrt(fmax(rn, 0.0));
+  const bool trig = !isfinite(rn) || rs < sc->delta * sqrt(sc->rmax2) ||
+                    sc->gamma * rs <= 0.9 * sc->tol || iter > sc->maxiter;
+  if (lb == 0 && threadIdx.x == 0) {
+    if (bad) {
+      sc->status = 6;
+      sc->done = 1;
+    } else {
+      sc->alpha = alpha;
+      sc->cur = sc->cur_next;
+      sc->iter = iter;
+      sc->xh_fold = trig ? 1 : sc->xf_next;
+      sc->rho = rz;
+      sc->first = 0;
+      sc->rz_ok = 0;
+      sc->ru = trig ? 1 : 0;
+      sc->rho_pend = rn;
+    }
+  }
+  return bad ? -1 : (trig ? 1 : 0);
+}
+
+// Before the FP64 residual: the mean of x64.
+__device__ __forceinline__ double lean_mean(const SysDev& s, Scalars* sc, int lb) {
+  double acc[1] = {0.0};  // a zero start's sum
+  if (!sc->zero_start) reduce_partials<1, 0u>(acc, s.pacc, s.nblk_sm);
+  const double mean = sc->singular ? acc[0] / (double)s.n : 0.0;
+  if (lb == 0 && threadIdx.x == 0) {
+    sc->mean_pending = mean;
+    sc->xh_fold = 1;
+  }
+  return mean;
+}
+
+// What a reliable update's true residual (acc: |r^|^2, |r|^2, max |r|) says:
+// true if the solve ends.  `store`: by one thread of one workgroup.
+__device__ __forceinline__ bool ru_verdict(Scalars* sc, const double (&acc)[3], bool store) {
+  const double rh2 = acc[0], rr = acc[1], mx = acc[2];
+  const double relres = sc->bnorm2 > 0 ? sqrt(rr / sc->bnorm2) : sqrt(rr);
+  const double l2 = sqrt(rr / sc->h3), lmax = mx / sc->h3;
+  const double metric = sc->resmode == 2 ? relres : (sc->resmode == 1 ? lmax : l2);
+  const bool conv = sc->resmode == 2 ? metric <= sc->tol : metric < sc->tol;
+  const bool bad = !isfinite(rr) || !isfinite(rh2);
+  // the reference's rule (src/linear/linear.ipp:109-110): at most
+  // maxiter + 1 iterations, never fewer than miniter
+  const bool stop = sc->iter >= sc->miniter && (conv || sc->iter > sc->maxiter);
+  if (store) {
+    sc->relres = relres;
+    sc->res_l2 = l2;
+    sc->res_max = lmax;
+    sc->residual = metric;
+    sc->nru += 1;
+    if (bad) {
+      sc->status = 6;
+      sc->done = 1;
+    } else if (stop) {
+      sc->converged = conv ? 1 : 0;
+      sc->done = 1;
+    } else {
+      if (!sc->pc) {
+        sc->beta = sc->first ? 0.0 : rh2 / sc->rho;
+        sc->rho = rh2;
+        sc->first = 0;
+      }
+      sc->rmax2 = rh2;
+      sc->gamma = rh2 > 0 ? metric / sqrt(rh2) : 1.0;
+    }
+    sc->zero_start = 0;
+  }
+  return bad || stop;
+}
+
+// Before the cycle, after a reliable update: its verdict.
+template <int NT>
+__device__ __forceinline__ bool lean_verdict(const SysDev& s, Scalars* sc, int lb) {
+  double acc[3];
+  reduce_partials<3, 4u, NT>(acc, s.pres, s.nblk_ru);
+  return ru_verdict(sc, acc, lb == 0 && threadIdx.x == 0);
+}
+
+// x64 = (x64 - mp) + S * (x^ + fa p) on cells [beg, end) (stale: x^ counts as
+// zero); this thread's part of the new x64's sum.
+template <typename T, int VX>
+__device__ __forceinline__ double ru_accum_cells(const SysDev& s, long long beg, long long end,
+                                                 double mp, double fa, bool stale,
+                                                 const T* __restrict__ p) {
+  using D = vec_t<double, VX>;
+  const T* __restrict__ S = (const T*)s.S;
+  const T* __restrict__ xh = (const T*)s.xh;
+  double* __restrict__ x = s.x64;
+  double sum = 0.0;
+  for (long long i = beg + (long long)threadIdx.x * VX; i < end; i += (long long)kBlock * VX) {
+    const D sv = S ? ldd<T, VX>(S, i) : (D)(1.0);
+    D h = stale ? (D)(0.0) : ldd<T, VX>(xh, i);
+    if (fa != 0.0) h += fa * ldd<T, VX>(p, i);
+    const D xv = (*reinterpret_cast<const D*>(x + i) - mp) + sv * h;
+    *reinterpret_cast<D*>(x + i) = xv;
+#pragma unroll
+    for (int v = 0; v < VX; ++v) sum += xv[v];
+  }
+  return sum;
+}
+
+// ===========================================================================
 // PCG (scaled, structure-preserving): q = S * L(k) * (S p) with
 //   (L u)_c = sum_faces k_f (u_c - u_nb) + m_c u_c,
 // where k are the plus-face conductances of each cell.  The p update
@@ -263,7 +408,8 @@ __device__ __forceinline__ Tile tile_of(const Rec& rc, const SysDev& s, int lb) 
 // x64, and x^ = alpha p_in (no read) in the iteration after, x^ being stale
 // since that update (xh_fold 1, 2).
 template <typename T, int VX, bool SC, bool XH>
-__global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ents, const int* __restrict__ b2r) {
+__global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ents,
+                                                     const int* __restrict__ b2r) {
   // arithmetic of the operator: FP64 for the Jacobi-scaled form, T with the
   // multigrid preconditioner (whose V-cycle absorbs FP32 rounding anyway)
   using A = typename std::conditional<SC, double, T>::type;
@@ -274,12 +420,17 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
   const Rec rc = en.rc;
   const SysDev& s = en.s;
   Scalars* sc = s.sc;
-  if (sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
+  const bool lean = !SC && s.lean;
+  // ru: a reliable update is pending (lean: the last one, done by now)
+  if (sc->done || (!lean && sc->ru) || s.pers) return;
   const int lb = b - rc.blk0;
   const Tile t = tile_of<VX>(rc, s, lb);
   const int nx = s.nx, ny = s.ny, nz = s.nz;
   const int cur = sc->cur;
-  const double beta = sc->beta;
+  double beta = sc->beta;
+  if constexpr (!SC) {
+    if (lean && !lean_beta(s, sc, lb, beta)) return;
+  }
   const gcp<T> __restrict__ r = (gcp<T>)s.z;  // r (Jacobi-scaled) or z = M^-1 r
   const gcp<T> __restrict__ pin = (gcp<T>)s.p[cur];
   const gmp<T> __restrict__ pout = (gmp<T>)s.p[cur ^ 1];
@@ -289,6 +440,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
   const gcp<T> __restrict__ kz = (gcp<T>)s.kz;
   const gcp<T> __restrict__ S = (gcp<T>)s.S;
   const gcp<T> __restrict__ mm = (gcp<T>)s.m;
+  const gcp<T> __restrict__ rr = (gcp<T>)s.r;  // lean: also (r, r), (r, q), (q, q)
   const int has_m = s.has_m;
   const int lx = rc.lx;
   const int tx = lx * VX;                 // tile width in cells (LDS row)
@@ -357,12 +509,17 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
   }
   __syncthreads();
   double dot = 0.0;
+  double dr[3] = {0.0, 0.0, 0.0};
   for (int z = t.za; z < t.zb; ++z) {
     const int buf = (z - t.za) & 1;
     if (t.active) {
       const long long base = (long long)z * pl;
       const long long ic = base + row + t.x0;
       const long long in = (long long)wrapp(z, nz) * pl + row + t.x0;
+      V rv = (T)0;
+      if constexpr (!SC) {
+        if (lean) rv = ldv<T, VX>(rr, ic);
+      }
       const V pn = z + 1 < t.zb ? pnew_own(in) : pnew_st(in);
       const V Sn = sld(in);
       const D un = cva<A, VX>(Sn) * cva<A, VX>(pn);
@@ -411,6 +568,17 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
       const vec_t<double, VX> pcd = cvt<VX>(pc), qd = cvt<VX>(qv);
 #pragma unroll
       for (int v = 0; v < VX; ++v) dot += pcd[v] * qd[v];
+      if constexpr (!SC) {
+        if (lean) {
+          const vec_t<double, VX> rd = cvt<VX>(rv);
+#pragma unroll
+          for (int v = 0; v < VX; ++v) {
+            dr[0] += rd[v] * rd[v];
+            dr[1] += rd[v] * qd[v];
+            dr[2] += qd[v] * qd[v];
+          }
+        }
+      }
       um = uc;
       uc = un;
       pc = pn;
@@ -418,16 +586,23 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
     }
     __syncthreads();
   }
+  if constexpr (!SC) {
+    if (lean) {
+      double acc[4] = {dot, dr[0], dr[1], dr[2]};
+      block_partial<4, 0u>(acc, s.partials, rc.nblk, lb);
+      return;
+    }
+  }
   double acc[1] = {dot};
   block_partial<1, 0u>(acc, s.partials, rc.nblk, lb);
 }
 
 // Finalize kernels: one workgroup per system, launched after the reducing
-// kernel of the same name.
+// kernel of the same name (systems with SysDev::lean do without).
 __global__ __launch_bounds__(kBlock) void k_fin_pcg_spmv(const SysDev* __restrict__ sds) {
   const SysDev& s = sds[blockIdx.x];
   Scalars* sc = s.sc;
-  if (sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
+  if (s.lean || sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
   double acc[1];
   reduce_partials<1, 0u>(acc, s.partials, s.nblk_st);
   if (threadIdx.x == 0) {
@@ -459,21 +634,40 @@ __device__ __forceinline__ void stream_range(long long n, int nblk, int lb, long
 // residual) follows.  x^ += alpha p is left to the CG operator of the next
 // iteration, which reads p anyway (k_pcg_spmv, XH).
 template <typename T, int VX>
-__global__ __launch_bounds__(kBlock) void k_pcg_update(const Ent* __restrict__ ents, const int* __restrict__ b2r) {
+__global__ __launch_bounds__(kBlock) void k_pcg_update(const Ent* __restrict__ ents,
+                                                       const int* __restrict__ b2r) {
   using D = vec_t<double, VX>;
   const int b = blockIdx.x;
   const Ent& en = ents[b2r ? b2r[b] : 0];
   const Rec rc = en.rc;
   const SysDev& s = en.s;
   Scalars* sc = s.sc;
-  if (sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
+  const bool lean = s.lean;
+  // ru: a reliable update is pending (lean: the last one, done by now)
+  if (sc->done || (!lean && sc->ru) || s.pers) return;
   const int lb = b - rc.blk0;
-  const double alpha = sc->alpha;
+  double alpha = sc->alpha;
   const T* __restrict__ q = (const T*)s.q;
   T* __restrict__ r = (T*)s.r;
   double acc[1] = {0.0};
   long long beg, end;
   stream_range<VX>(s.n, rc.nblk, lb, beg, end);
+  if (lean) {
+    const int what = lean_step(s, sc, lb, alpha);
+    if (what < 0) return;
+    if (what > 0) {
+      // a reliable update replaces r by the FP64 residual: no update of r, but
+      // its first part at once
+      acc[0] = ru_accum_cells<T, VX>(s, beg, end, sc->mean_pending, alpha, sc->xf_next != 0,
+                                     (const T*)s.p[sc->cur_next]);
+      block_partial<1, 0u>(acc, s.pacc, rc.nblk, lb);
+      return;
+    }
+    for (long long i = beg + (long long)threadIdx.x * VX; i < end;
+         i += (long long)kBlock * VX)
+      std_<T, VX>(r, i, rnd<T, VX>(ldd<T, VX>(r, i) - alpha * ldd<T, VX>(q, i)));
+    return;
+  }
   for (long long i = beg + (long long)threadIdx.x * VX; i < end; i += (long long)kBlock * VX) {
     const D rv = rnd<T, VX>(ldd<T, VX>(r, i) - alpha * ldd<T, VX>(q, i));
     std_<T, VX>(r, i, rv);
@@ -486,7 +680,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update(const Ent* __restrict__ e
 __global__ __launch_bounds__(kBlock) void k_fin_pcg_update(const SysDev* __restrict__ sds) {
   const SysDev& s = sds[blockIdx.x];
   Scalars* sc = s.sc;
-  if (sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
+  if (s.lean || sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
   double acc[1];
   reduce_partials<1, 0u>(acc, s.partials, s.nblk_sm);
   if (threadIdx.x == 0) {
@@ -512,9 +706,12 @@ __global__ __launch_bounds__(kBlock) void k_fin_pcg_update(const SysDev* __restr
 // next iteration's CG operator would add it), so alpha p is added here and
 // the operator skips it; x^ counts as zero from here on (xh_fold 1: not read
 // again before the operator after next overwrites it).
+// so: the start of newly prepared systems; of the multigrid systems only those
+// (first == 1) take part.  In lean systems the update kernel does this part of
+// every later one.
 template <typename T, int VX>
-__global__ __launch_bounds__(kBlock) void k_ru_accum(const Ent* __restrict__ ents, const int* __restrict__ b2r) {
-  using D = vec_t<double, VX>;
+__global__ __launch_bounds__(kBlock) void k_ru_accum(const Ent* __restrict__ ents,
+                                                     const int* __restrict__ b2r, int so) {
   const int b = blockIdx.x;
   const Ent& en = ents[b2r ? b2r[b] : 0];
   const Rec rc = en.rc;
@@ -522,35 +719,24 @@ __global__ __launch_bounds__(kBlock) void k_ru_accum(const Ent* __restrict__ ent
   Scalars* sc = s.sc;
   // a zero start: x64 and x^ are zero already, and so is their mean
   if (sc->done || !sc->ru || sc->zero_start) return;
+  if (s.lean && !so) return;
+  if (so && sc->pc && !sc->first) return;
   const int lb = b - rc.blk0;
-  const double mp = sc->mean_pending;
-  const T* __restrict__ S = (const T*)s.S;
-  T* __restrict__ xh = (T*)s.xh;
-  double* __restrict__ x = s.x64;
-  const double fa = sc->alpha;  // 0 at a start
-  const bool stale = sc->xh_fold != 0;  // x^ counts as zero
-  const T* __restrict__ p = (const T*)s.p[sc->cur];
-  double acc[1] = {0.0};
   long long beg, end;
   stream_range<VX>(s.n, rc.nblk, lb, beg, end);
-  for (long long i = beg + (long long)threadIdx.x * VX; i < end; i += (long long)kBlock * VX) {
-    const D sv = S ? ldd<T, VX>(S, i) : (D)(1.0);
-    D h = stale ? (D)(0.0) : ldd<T, VX>(xh, i);
-    if (fa != 0.0) h += fa * ldd<T, VX>(p, i);
-    const D xv = (*reinterpret_cast<const D*>(x + i) - mp) + sv * h;
-    *reinterpret_cast<D*>(x + i) = xv;
-#pragma unroll
-    for (int v = 0; v < VX; ++v) acc[0] += xv[v];
-  }
-  block_partial<1, 0u>(acc, s.partials, rc.nblk, lb);
+  // alpha is 0 at a start
+  double acc[1] = {ru_accum_cells<T, VX>(s, beg, end, sc->mean_pending, sc->alpha,
+                                         sc->xh_fold != 0, (const T*)s.p[sc->cur])};
+  block_partial<1, 0u>(acc, s.pacc, rc.nblk, lb);
 }
 
-__global__ __launch_bounds__(kBlock) void k_fin_ru_accum(const SysDev* __restrict__ sds) {
+__global__ __launch_bounds__(kBlock) void k_fin_ru_accum(const SysDev* __restrict__ sds, int so) {
   const SysDev& s = sds[blockIdx.x];
   Scalars* sc = s.sc;
-  if (sc->done || !sc->ru) return;
+  if (s.lean || sc->done || !sc->ru) return;
+  if (so && sc->pc && !sc->first) return;
   double acc[1] = {0.0};  // a zero start's sum (k_ru_accum wrote no partials)
-  if (!sc->zero_start) reduce_partials<1, 0u>(acc, s.partials, s.nblk_sm);
+  if (!sc->zero_start) reduce_partials<1, 0u>(acc, s.pacc, s.nblk_sm);
   if (threadIdx.x == 0) {
     sc->mean_pending = sc->singular ? acc[0] / (double)s.n : 0.0;
     sc->xh_fold = 1;
@@ -563,7 +749,8 @@ __global__ __launch_bounds__(kBlock) void k_fin_ru_accum(const SysDev* __restric
 // x of planes z-1, z, z+1 and e_z of plane z-1 in registers, the x plane of
 // the tile in LDS for the x and y neighbours.
 template <typename T, int VX>
-__global__ __launch_bounds__(kBlock) void k_ru_resid(const Ent* __restrict__ ents, const int* __restrict__ b2r) {
+__global__ __launch_bounds__(kBlock) void k_ru_resid(const Ent* __restrict__ ents,
+                                                     const int* __restrict__ b2r, int so) {
   static_assert(VX == 1, "one cell per thread");
   __shared__ double su[2][kBlock];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
@@ -572,10 +759,11 @@ __global__ __launch_bounds__(kBlock) void k_ru_resid(const Ent* __restrict__ ent
   const SysDev& s = en.s;
   Scalars* sc = s.sc;
   if (sc->done || !sc->ru) return;
+  if (so && sc->pc && !sc->first) return;
   const int lb = b - rc.blk0;
   const Tile t = tile_of<1>(rc, s, lb);
   const int nx = s.nx, ny = s.ny, nz = s.nz;
-  const double mp = sc->mean_pending;
+  const double mp = s.lean ? lean_mean(s, sc, lb) : sc->mean_pending;
   const double sgn = s.neg ? -1.0 : 1.0;
   const gcp<double> __restrict__ x = (gcp<double>)s.x64;
   const gcp<double> __restrict__ bb = (gcp<double>)s.b64;
@@ -654,13 +842,14 @@ __global__ __launch_bounds__(kBlock) void k_ru_resid(const Ent* __restrict__ ent
     }
     if (!zs) __syncthreads();
   }
-  block_partial<3, 4u>(acc, s.partials, rc.nblk, lb);
+  block_partial<3, 4u>(acc, s.pres, rc.nblk, lb);
 }
 
 // k_ru_resid with 2 cells per thread (even nx): 16-byte FP64 loads of x, b
 // and the coefficients; the same per-cell operation order and partials.
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_ru_resid2(const Ent* __restrict__ ents, const int* __restrict__ b2r) {
+__global__ __launch_bounds__(kBlock) void k_ru_resid2(const Ent* __restrict__ ents,
+                                                     const int* __restrict__ b2r, int so) {
   using D2 = vec_t<double, 2>;
   __shared__ double su[2][kBlock * 2];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
@@ -669,10 +858,11 @@ __global__ __launch_bounds__(kBlock) void k_ru_resid2(const Ent* __restrict__ en
   const SysDev& s = en.s;
   Scalars* sc = s.sc;
   if (sc->done || !sc->ru) return;
+  if (so && sc->pc && !sc->first) return;
   const int lb = b - rc.blk0;
   const Tile t = tile_of<2>(rc, s, lb);
   const int nx = s.nx, ny = s.ny, nz = s.nz;
-  const double mp = sc->mean_pending;
+  const double mp = s.lean ? lean_mean(s, sc, lb) : sc->mean_pending;
   const double sgn = s.neg ? -1.0 : 1.0;
   const gcp<double> __restrict__ x = (gcp<double>)s.x64;
   const gcp<double> __restrict__ bb = (gcp<double>)s.b64;
@@ -789,45 +979,19 @@ __global__ __launch_bounds__(kBlock) void k_ru_resid2(const Ent* __restrict__ en
     }
     if (!zs) __syncthreads();
   }
-  block_partial<3, 4u>(acc, s.partials, rc.nblk, lb);
+  block_partial<3, 4u>(acc, s.pres, rc.nblk, lb);
 }
 
-__global__ __launch_bounds__(kBlock) void k_fin_ru_resid(const SysDev* __restrict__ sds) {
+__global__ __launch_bounds__(kBlock) void k_fin_ru_resid(const SysDev* __restrict__ sds, int so) {
   const SysDev& s = sds[blockIdx.x];
   Scalars* sc = s.sc;
-  if (sc->done || !sc->ru) return;
+  if (s.lean || sc->done || !sc->ru) return;
+  if (so && sc->pc && !sc->first) return;
   double acc[3];
-  reduce_partials<3, 4u>(acc, s.partials, s.nblk_ru);
+  reduce_partials<3, 4u>(acc, s.pres, s.nblk_ru);
   if (threadIdx.x == 0) {
-    const double rh2 = acc[0], rr = acc[1], mx = acc[2];
-    const double relres = sc->bnorm2 > 0 ? sqrt(rr / sc->bnorm2) : sqrt(rr);
-    const double l2 = sqrt(rr / sc->h3), lmax = mx / sc->h3;
-    const double metric = sc->resmode == 2 ? relres : (sc->resmode == 1 ? lmax : l2);
-    const bool conv = sc->resmode == 2 ? metric <= sc->tol : metric < sc->tol;
-    sc->relres = relres;
-    sc->res_l2 = l2;
-    sc->res_max = lmax;
-    sc->residual = metric;
-    sc->nru += 1;
-    if (!isfinite(rr) || !isfinite(rh2)) {
-      sc->status = 6;
-      sc->done = 1;
-    } else if (sc->iter >= sc->miniter && (conv || sc->iter > sc->maxiter)) {
-      // the reference's rule (src/linear/linear.ipp:109-110): at most
-      // maxiter + 1 iterations, never fewer than miniter
-      sc->converged = conv ? 1 : 0;
-      sc->done = 1;
-    } else {
-      if (!sc->pc) {
-        sc->beta = sc->first ? 0.0 : rh2 / sc->rho;
-        sc->rho = rh2;
-      }
-      sc->rmax2 = rh2;
-      sc->gamma = rh2 > 0 ? metric / sqrt(rh2) : 1.0;
-      if (!sc->pc) sc->first = 0;
-    }
+    ru_verdict(sc, acc, true);
     sc->ru = 0;
-    sc->zero_start = 0;
   }
 }
 
@@ -1010,7 +1174,8 @@ __device__ __forceinline__ Cell cell_of(const Rec& rc, int lb, int nx, int ny, i
 // L0: the launch on level 0 (a separate instance, so that profiles keep the
 // bandwidth-bound fine-grid sweeps apart from the coarse levels).
 template <typename T, int VX, int MODE, bool DOT, bool L0>
-__global__ __launch_bounds__(kBlock) void k_mg_sweep(const Ent* __restrict__ ents, const int* __restrict__ b2r, int l_arg,
+__global__ __launch_bounds__(kBlock) void k_mg_sweep(const Ent* __restrict__ ents,
+                                                     const int* __restrict__ b2r, int l_arg,
                                                      int zin, int zout, int wl, int so,
                                                      int addzs) {
   const int l = L0 ? 0 : l_arg;
@@ -1029,6 +1194,9 @@ __global__ __launch_bounds__(kBlock) void k_mg_sweep(const Ent* __restrict__ ent
   if (wl >= 0 && wl >= s.mg_w) return;
   // so: the start of newly prepared systems (first == 1); running ones skip
   if (so && !s.sc->first) return;
+  if constexpr (MODE == 1 && L0) {
+    if (en.lv.post == 0 && s.lean && s.sc->ru && lean_verdict<kBlock>(s, s.sc, b - rc.blk0)) return;
+  }
   const MgLevel& Lv = en.lv;
   // this system's level runs fused kernels (k_mg_pre, k_mg_post) instead
   if ((MODE == 0 || MODE == 1 || MODE == 2 || MODE == 3) && Lv.post) return;
@@ -1245,7 +1413,7 @@ __global__ __launch_bounds__(kBlock) void k_mg_sweep(const Ent* __restrict__ ent
   }
   if constexpr (DOT) {
     double acc[1] = {dot};
-    block_partial<1, 0u>(acc, s.partials, rc.nblk, lb);
+    block_partial<1, 0u>(acc, s.ppc, rc.nblk, lb);
   }
 }
 
@@ -1270,7 +1438,8 @@ __global__ __launch_bounds__(kBlock) void k_mg_sweep(const Ent* __restrict__ ent
 // stored nor restricted (edges are even, tiles start at multiples of 8).
 // DOT (POST on level 0): partials of (r, z[1]).
 template <bool PRE, bool DOT>
-__global__ __launch_bounds__(kTileBlock) void k_mg_tile(const Ent* __restrict__ ents, const int* __restrict__ b2r, int l,
+__global__ __launch_bounds__(kTileBlock) void k_mg_tile(const Ent* __restrict__ ents,
+                                                        const int* __restrict__ b2r, int l,
                                                         int wl, int so, int addzs) {
   constexpr int B = kTile + 4;            // box rows per edge (y, z)
   constexpr int W = kTile + 8;            // cells per staged row (x)
@@ -1289,6 +1458,9 @@ __global__ __launch_bounds__(kTileBlock) void k_mg_tile(const Ent* __restrict__ 
   if (s.sc->done) return;
   if (wl >= 0 && wl >= s.mg_w) return;
   if (so && !s.sc->first) return;
+  if constexpr (PRE) {
+    if (l == 0 && s.lean && s.sc->ru && lean_verdict<kTileBlock>(s, s.sc, b - rc.blk0)) return;
+  }
   const MgLevel& Lv = en.lv;
   const MgLevel& Lc = en.lc;
   const int nx = Lv.nx, ny = Lv.ny, nz = Lv.nz;
@@ -1391,7 +1563,7 @@ __global__ __launch_bounds__(kTileBlock) void k_mg_tile(const Ent* __restrict__ 
   }
   if constexpr (DOT) {
     double acc[1] = {dot};
-    block_partial<1, 0u, kTileBlock>(acc, s.partials, rc.nblk, lb);
+    block_partial<1, 0u, kTileBlock>(acc, s.ppc, rc.nblk, lb);
   }
   if constexpr (PRE) {
     __syncthreads();
@@ -1414,7 +1586,8 @@ __global__ __launch_bounds__(kTileBlock) void k_mg_tile(const Ent* __restrict__ 
 // Residual of level l restricted to level l+1: r_{l+1}[C] = sum over the
 // 2x2x2 children c of (r - L z)_c.  One thread per coarse cell.
 template <typename T, bool L0>
-__global__ __launch_bounds__(kBlock) void k_mg_restrict(const Ent* __restrict__ ents, const int* __restrict__ b2r, int l_arg,
+__global__ __launch_bounds__(kBlock) void k_mg_restrict(const Ent* __restrict__ ents,
+                                                        const int* __restrict__ b2r, int l_arg,
                                                         int zin, int wl, int so) {
   const int l = L0 ? 0 : l_arg;
   const int b = xcd_remap(blockIdx.x, gridDim.x);
@@ -1467,7 +1640,8 @@ __global__ __launch_bounds__(kBlock) void k_mg_restrict(const Ent* __restrict__ 
 // hits).  The u rows just outside the tile (for the halo rows' v) and the u
 // planes before and after the tile come from memory.
 template <typename T, int VX, bool DOT, bool L0>
-__global__ __launch_bounds__(kPostBlock) void k_mg_post(const Ent* __restrict__ ents, const int* __restrict__ b2r, int l_arg,
+__global__ __launch_bounds__(kPostBlock) void k_mg_post(const Ent* __restrict__ ents,
+                                                        const int* __restrict__ b2r, int l_arg,
                                                         int wl, int so, int addzs) {
   const int l = L0 ? 0 : l_arg;
   using V = vec_t<T, VX>;
@@ -1624,7 +1798,7 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_post(const Ent* __restrict__ 
   }
   if constexpr (DOT) {
     double acc[1] = {dot};
-    block_partial<1, 0u, kPostBlock>(acc, s.partials, rc.nblk, lb);
+    block_partial<1, 0u, kPostBlock>(acc, s.ppc, rc.nblk, lb);
   }
 }
 
@@ -1651,7 +1825,8 @@ __device__ __forceinline__ vec_t<float, 4> bf4(unsigned a, unsigned b) {
 // ky and kx of the neighbouring cells instead of loading them again.  Same
 // arithmetic as k_mg_post.
 template <bool DOT, bool L0>
-__global__ __launch_bounds__(kPostBlock) void k_mg_post4(const Ent* __restrict__ ents, const int* __restrict__ b2r,
+__global__ __launch_bounds__(kPostBlock) void k_mg_post4(const Ent* __restrict__ ents,
+                                                         const int* __restrict__ b2r,
                                                          int l_arg, int wl, int so, int addzs) {
   using V = vec_t<float, 4>;
   using U4 = vec_t<unsigned, 4>;
@@ -1840,7 +2015,7 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_post4(const Ent* __restrict__
   }
   if constexpr (DOT) {
     double acc[1] = {dot};
-    block_partial<1, 0u, kPostBlock>(acc, s.partials, rc.nblk, lb);
+    block_partial<1, 0u, kPostBlock>(acc, s.ppc, rc.nblk, lb);
   }
 }
 
@@ -1857,7 +2032,8 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_post4(const Ent* __restrict__
 // rows hand their sums to the even row above).  One barrier per step; u and z
 // planes double-buffered in LDS.
 template <typename T, int VX, bool L0>
-__global__ __launch_bounds__(kPostBlock) void k_mg_pre(const Ent* __restrict__ ents, const int* __restrict__ b2r, int l_arg,
+__global__ __launch_bounds__(kPostBlock) void k_mg_pre(const Ent* __restrict__ ents,
+                                                       const int* __restrict__ b2r, int l_arg,
                                                        int wl, int so) {
   static_assert(VX >= 2, "x pairs of the restriction are summed in the thread");
   constexpr int NP = VX / 2;
@@ -1874,6 +2050,9 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_pre(const Ent* __restrict__ e
   if (s.sc->done) return;
   if (wl >= 0 && wl >= s.mg_w) return;
   if (so && !s.sc->first) return;
+  if constexpr (L0) {
+    if (s.lean && s.sc->ru && lean_verdict<kPostBlock>(s, s.sc, b - rc.blk0)) return;
+  }
   const MgLevel Lv = cload(&en->lv);
   const MgLevel Lc = cload(&en->lc);
   const int nx = Lv.nx, ny = Lv.ny, nz = Lv.nz;
@@ -2043,7 +2222,8 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_pre(const Ent* __restrict__ e
 // k + 1; plane k-1's packed coefficients, r, ky and kx wait in LDS slots for
 // the residual.  Same arithmetic as k_mg_pre.
 template <bool L0>
-__global__ __launch_bounds__(kPostBlock) void k_mg_pre4(const Ent* __restrict__ ents, const int* __restrict__ b2r, int l_arg,
+__global__ __launch_bounds__(kPostBlock) void k_mg_pre4(const Ent* __restrict__ ents,
+                                                        const int* __restrict__ b2r, int l_arg,
                                                         int wl, int so) {
   using V = vec_t<float, 4>;
   using U4 = vec_t<unsigned, 4>;
@@ -2068,6 +2248,9 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_pre4(const Ent* __restrict__ 
   if (s.sc->done) return;
   if (wl >= 0 && wl >= s.mg_w) return;
   if (so && !s.sc->first) return;
+  if constexpr (L0) {
+    if (s.lean && s.sc->ru && lean_verdict<kPostBlock>(s, s.sc, b - rc.blk0)) return;
+  }
   const MgLevel Lv = cload(&en->lv);
   const MgLevel Lc = cload(&en->lc);
   const int nx = Lv.nx, ny = Lv.ny, nz = Lv.nz;
@@ -2747,19 +2930,24 @@ __global__ __launch_bounds__(kBottomThreads) void k_mg_bottom(const SysDev* __re
 
 // (r, z) of the preconditioned CG: beta = (r,z) / (r,z)_old (0 after a start)
 __global__ __launch_bounds__(kBlock) void k_fin_precond(const SysDev* __restrict__ sds,
-                                                        int so) {
+                                                        int so, int close) {
   const SysDev& s = sds[blockIdx.x];
   Scalars* sc = s.sc;
   if (s.nlev <= 0 || sc->done) return;
   if (so && !sc->first) return;
+  if (s.lean && !close) return;
   double acc[1];
-  reduce_partials<1, 0u>(acc, s.partials, s.nblk_pc);
+  reduce_partials<1, 0u>(acc, s.ppc, s.nblk_pc);
   if (threadIdx.x == 0) {
     const double rz = acc[0];
-    sc->beta = sc->first ? 0.0 : rz / sc->rho;
-    sc->rho = rz;
     sc->rz = rz;
-    sc->first = 0;
+    if (s.lean) {
+      sc->rz_ok = 1;
+    } else {
+      sc->beta = sc->first ? 0.0 : rz / sc->rho;
+      sc->rho = rz;
+      sc->first = 0;
+    }
     if (!isfinite(rz)) {
       sc->status = 6;
       sc->done = 1;
@@ -3579,7 +3767,7 @@ static int launch_vcycle(const LaunchSet& L, hipStream_t st, hipEvent_t* ev = nu
   };
   launch_cycle<T>(L, st, 0, -1, false, mark);
   mark(4);
-  APH_LAUNCH(k_fin_precond, L.ns, st, L.sds, L.start_only);
+  if (L.any_plain || L.close) APH_LAUNCH(k_fin_precond, L.ns, st, L.sds, L.start_only, L.close);
   if (ev) (void)hipEventRecord(ev[k], st);
   return k;
 }
@@ -3632,20 +3820,29 @@ static void launch_pcg_kernel(const LaunchSet& L, hipStream_t st, int j) {
       else APH_LAUNCH((k_pcg_spmv<T, VX, true, true>), L.nst, st, L.ent_st, L.b2r_st);
       break;
     case 8: launch_vcycle<T>(L, st); break;
-    case 1: APH_LAUNCH(k_fin_pcg_spmv, L.ns, st, L.sds); break;
+    case 1:
+      if (L.any_plain) APH_LAUNCH(k_fin_pcg_spmv, L.ns, st, L.sds);
+      break;
     case 2:
       APH_LAUNCH((k_pcg_update<T, VX>), L.nsm, st, L.ent_sm, L.b2r_sm);
       break;
-    case 3: APH_LAUNCH(k_fin_pcg_update, L.ns, st, L.sds); break;
+    case 3:
+      if (L.any_plain) APH_LAUNCH(k_fin_pcg_update, L.ns, st, L.sds);
+      break;
     case 4:
-      APH_LAUNCH((k_ru_accum<T, VX>), L.nsm, st, L.ent_sm, L.b2r_sm);
+      if (L.any_plain || L.start_only)
+        APH_LAUNCH((k_ru_accum<T, VX>), L.nsm, st, L.ent_sm, L.b2r_sm, L.start_only);
       break;
-    case 5: APH_LAUNCH(k_fin_ru_accum, L.ns, st, L.sds); break;
+    case 5:
+      if (L.any_plain) APH_LAUNCH(k_fin_ru_accum, L.ns, st, L.sds, L.start_only);
+      break;
     case 6:
-      if (L.vx_ru == 2) APH_LAUNCH(k_ru_resid2<T>, L.nru, st, L.ent_ru, L.b2r_ru);
-      else APH_LAUNCH((k_ru_resid<T, 1>), L.nru, st, L.ent_ru, L.b2r_ru);
+      if (L.vx_ru == 2) APH_LAUNCH(k_ru_resid2<T>, L.nru, st, L.ent_ru, L.b2r_ru, L.start_only);
+      else APH_LAUNCH((k_ru_resid<T, 1>), L.nru, st, L.ent_ru, L.b2r_ru, L.start_only);
       break;
-    default: APH_LAUNCH(k_fin_ru_resid, L.ns, st, L.sds); break;
+    default:
+      if (L.any_plain) APH_LAUNCH(k_fin_ru_resid, L.ns, st, L.sds, L.start_only);
+      break;
   }
 }
 

@@ -83,7 +83,7 @@ __device__ __forceinline__ void block_partial(double (&v)[NV], double* partials,
 
 // Sums (or maxes) the partials of nblk workgroups in block order; result in
 // every thread of the calling workgroup.
-template <int NV, unsigned MaxMask>
+template <int NV, unsigned MaxMask, int NT = kBlock>
 __device__ __forceinline__ void reduce_partials(double (&v)[NV], const double* partials,
                                                 int nblk) {
 #pragma unroll
@@ -94,20 +94,20 @@ __device__ __forceinline__ void reduce_partials(double (&v)[NV], const double* p
     // fixed order
     double t[4] = {0.0, 0.0, 0.0, 0.0};
     int i = threadIdx.x;
-    for (; i + 3 * kBlock < nblk; i += 4 * kBlock) {
+    for (; i + 3 * NT < nblk; i += 4 * NT) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const double pv = pk[i + j * kBlock];
+        const double pv = pk[i + j * NT];
         t[j] = mx ? fmax(t[j], pv) : t[j] + pv;
       }
     }
-    for (int j = 0; i < nblk; i += kBlock, ++j) {
+    for (int j = 0; i < nblk; i += NT, ++j) {
       const double pv = pk[i];
       t[j] = mx ? fmax(t[j], pv) : t[j] + pv;
     }
     v[k] = mx ? fmax(fmax(t[0], t[1]), fmax(t[2], t[3])) : (t[0] + t[1]) + (t[2] + t[3]);
   }
-  block_reduce<NV, MaxMask>(v);
+  block_reduce<NV, MaxMask, NT>(v);
 }
 
 }  // namespace aph

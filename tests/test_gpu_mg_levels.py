@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from aphros_amd import _lib as L
+from aphros_amd.batch import Batch
 from aphros_amd.solver import Poisson
 from oracle import oracle as O
 
@@ -88,3 +89,36 @@ def test_largest_coarsest_level():
     x, info = s.solve(None)
     s.close()
     assert info["converged"] == 1 and O.true_relres(e, x) <= 1e-8 * (1 + 1e-6)
+
+
+@pytest.mark.parametrize("precision", [L.MIXED, L.FP64])
+def test_reductions_at_the_size_line(precision):
+    """2^23 cells (reductions finished by the kernels that need them), 5/4 as
+    many (by kernels of their own), both in one batch with a small system:
+    each as alone, bit for bit, also from a guess and cut short by maxiter."""
+    shapes = [(128, 256, 256), (160, 256, 256), (16, 24, 20)]
+    es = [_system(s, 5 + i, i == 2) for i, s in enumerate(shapes)]
+    b = Batch(precision=precision, tol=1e-8, maxiter=2000, precond=L.PRECOND_MG,
+              mg_w=L.MG_W_AUTO)
+    slots = [b.add(e) for e in es]
+    b.solve()
+    for e, shape, slot in zip(es, shapes, slots):
+        xb, ib = b.get(slot)
+        s = Poisson(shape, method=L.PCG, precision=precision, resmode=L.RES_REL_TRUE, tol=1e-8,
+                    maxiter=2000, precond=L.PRECOND_MG)
+        s.set_system(e)
+        x, info = s.solve(None)
+        assert ib["converged"] == info["converged"] == 1 and ib["iter"] == info["iter"]
+        assert np.array_equal(x, xb) and O.true_relres(e, x) <= 1e-8 * (1 + 1e-6)
+        x2, warm = s.solve(x + 3.0 if shape[0] != 16 else x)
+        assert warm["converged"] == 1 and warm["iter"] <= 2
+        assert O.true_relres(e, x2) <= 1e-8 * (1 + 1e-6)
+        s.close()
+        s = Poisson(shape, method=L.PCG, precision=precision, resmode=L.RES_REL_TRUE, tol=1e-8,
+                    maxiter=3, precond=L.PRECOND_MG)
+        s.set_system(e)
+        x3, cut = s.solve(None)
+        s.close()
+        assert cut["converged"] == 0 and cut["iter"] == 4
+        assert abs(O.true_relres(e, x3) / cut["true_relres"] - 1) <= 1e-6
+    b.close()
