@@ -70,6 +70,7 @@ struct MgLevel {
   const void* kc;
   void* r;         // right-hand side of the level (level 0: the CG residual)
   void* z[2];      // correction, ping-pong
+  int fuse;        // post == 1: workgroup size, an index of kFuseThreads
   void* zs;        // first of two coarse corrections (levels below a W level)
 };
 

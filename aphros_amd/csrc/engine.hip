@@ -46,25 +46,31 @@ Rec make_stencil_rec(int nx, int ny, int nz, int vx, int blocks_target, const Tu
 
 // Fused pre-smoothing + restriction (k_mg_pre) and post-smoothing (k_mg_post)
 // of a level: whole-row tiles of lx = nx / vx threads per row and
-// ty = min(kPostBlock / lx, ny + 2) rows of threads (even; ty - 2 output
-// rows), bz planes (even).  Only for the large levels (the march is long
-// enough to hide the halo rows and planes it recomputes; such a level
-// coarsens, so its edges are even) whose rows fit 1/8 of the workgroup (ty >=
-// 8 rows).
+// ty = min(threads / lx, ny + 2) rows of threads (even; ty - 2 output rows),
+// bz planes (even), by workgroups of kFuseThreads[kind] threads.  Only for
+// levels whose rows fit 1/8 of the workgroup (ty >= 8 rows; such a level
+// coarsens, so its edges are even) and with at least 8 rows and planes (those
+// ahead of a march wrap once).
 //
-// From 2^19 cells in FP64 and 3 x 2^20 in FP32 (ms per solve, four launches
-// -> fused): FP64 96^3 4.3 -> 3.8, 128^3 6.5 -> 5.8, 160^3 12.4 -> 10.4, 192^3
-// 19.9 -> 13.4, 224^3 29.3 -> 19.7; mixed 128 x 96 x 160 8.4 -> 8.5 and batched
-// 128^3 5 % slower, 160^3 7.0 -> 6.0, 192^3 9.6 -> 8.6, 224^3 13.9 -> 11.1, 256
-// x 192 x 128 9.2 -> 7.9: below, the level's bytes are in the caches and the
-// march has too few workgroups.  The planes and rows ahead of a march wrap
-// once: at least 8 of each.
-constexpr long long kFuseMinCells64 = 1LL << 19, kFuseMinCells32 = 3LL << 20;
-// Levels of FP32 engines with at most this many cells and nx % 4 == 0 smooth in
-// tile launches (k_mg_tile: one launch and one round of global loads per pre-
-// or post-smoothing instead of two z-marching launches).  Microseconds per
-// iteration of a whole solve, level 0 swept -> tiled: 32^3 65 -> 56, 48^3 81 ->
-// 73, 64^3 84 -> 80, 80^3 112 -> 108, but 96^3 113 -> 117 and 128^3 135 -> 160:
+// A step of the march (one plane) is latency: loads, LDS, one barrier; ~3.3 us
+// with 1024 threads, the one workgroup its CU holds, half of that with 256
+// threads, of which a CU holds four.  So small levels take the smallest
+// workgroup that has 8 rows: more of them, shorter marches, against the halo
+// rows they re-read from the caches.  Above kFuseSmallCells those reads reach
+// HBM.  ms per solve, 1024 threads (swept below 3 x 2^20 cells in FP32, 2^19 in
+// FP64) -> by this rule: mixed 80^3 4.76 -> 4.53, 96^3 5.53 -> 5.11, 112^3 6.96
+// -> 6.77, 128^3 7.75 -> 7.31, 160^3 10.73 -> 10.45, 192^3 15.37 -> 14.65, 256^3
+// 25.0 -> 24.5 (256^3 with 512 threads on level 0: 25.2); FP64 64^3 5.43 -> 4.81,
+// 96^3 6.98 -> 6.57, 128^3 11.64 -> 10.53, 192^3 25.6 -> 24.75.
+constexpr long long kFuseSmallCells = 1LL << 23;
+// FP32 levels below this smooth in tiles (64^3 fused with 256 threads: 2.17 ->
+// 2.38 ms); FP64 levels fuse down to the bottom kernel's.
+constexpr long long kFuseMinCells32 = 3LL << 17;
+// Levels of FP32 engines with at most this many cells, nx % 4 == 0 and not fused
+// smooth in tile launches (k_mg_tile: one launch and one round of global loads
+// per pre- or post-smoothing instead of two z-marching launches).
+// Microseconds per iteration of a whole solve, level 0 swept -> tiled: 32^3 65
+// -> 56, 48^3 81 -> 73, 64^3 84 -> 80, but 96^3 113 -> 117 and 128^3 135 -> 160:
 // the tiles' halos (4.5x the level's bytes) then miss L2.
 constexpr long long kTileMaxCells = 1LL << 19;
 // Multigrid systems of at most this many cells finish their reductions in the
@@ -80,31 +86,29 @@ constexpr long long kLeanCells = 1LL << 23;
 constexpr int kPersRunIters = 512;
 constexpr int kPersStepIters = 128;
 
-bool make_post_rec(int nx, int ny, int nz, int vx, int ncu, Rec* out) {
-  const long long n = (long long)nx * ny * nz;
+bool make_post_rec(int nx, int ny, int nz, int vx, int ncu, int kind, Rec* out) {
   if (vx <= 0 || nx % vx != 0 || ny < 8 || nz < 8) return false;
-  if (n < (vx == 4 ? kFuseMinCells32 : kFuseMinCells64)) return false;
-  const int lx = nx / vx;
-  if (lx > kPostBlock / 8) return false;
+  const int nt = kFuseThreads[kind], lx = nx / vx;
+  if (lx > nt / 8) return false;
   Rec r{};
   r.lx = lx;
   // even: the fused restriction pairs output rows from an even row
-  r.ty = std::min(kPostBlock / lx, ny + 2) & ~1;
+  r.ty = std::min(nt / lx, ny + 2) & ~1;
   r.tiles_x = 1;
   r.tiles_y = (int)cdiv(ny, r.ty - 2);
-  // One workgroup is resident per CU (1024 threads at 128 VGPRs per lane) and
-  // a workgroup's time grows with the planes it marches, bz plus two halo
-  // planes.  The z split minimises rounds * (bz + 2), rounds = workgroups / CUs
-  // rounded up; of equal costs the one with fewer workgroups (less halo) wins.
+  // 1024 threads at 128 VGPRs per lane are resident per CU and a workgroup's
+  // time grows with the planes it marches, bz plus two halo planes.  The z
+  // split minimises rounds * (bz + 2), rounds = workgroups / slots rounded up;
+  // of equal costs the one with fewer workgroups (less halo) wins.
   // bz is even: the restriction pairs planes (nz is even on these levels).
-  const long long cus = std::max(1, ncu);
+  const long long slots = std::max(1, ncu) * (kFuseThreads[0] / nt);
   long long best = -1;
   for (int tz = 1; tz <= nz; ++tz) {
     int bz = (int)cdiv(nz, tz);
     bz = std::min(bz + (bz & 1), nz);
     const int tiles_z = (int)cdiv(nz, bz);
     if (tiles_z != tz) continue;
-    const long long cost = cdiv((long long)r.tiles_y * tiles_z, cus) * (bz + 2);
+    const long long cost = cdiv((long long)r.tiles_y * tiles_z, slots) * (bz + 2);
     if (best < 0 || cost < best) {
       best = cost;
       r.bz = bz;
@@ -114,6 +118,16 @@ bool make_post_rec(int nx, int ny, int nz, int vx, int ncu, Rec* out) {
   r.nblk = r.tiles_y * r.tiles_z;
   *out = r;
   return true;
+}
+
+// Workgroup size of a fused level (an index of kFuseThreads), -1: not fused.
+int fuse_kind(int nx, int ny, int nz, int vx, int ncu) {
+  const long long n = (long long)nx * ny * nz;
+  if (vx == 4 && n < kFuseMinCells32) return -1;
+  Rec r;
+  for (int k = n < kFuseSmallCells ? kFuseKinds - 1 : 0; k >= 0; --k)
+    if (make_post_rec(nx, ny, nz, vx, ncu, k, &r)) return k;
+  return -1;
 }
 
 }  // namespace
@@ -469,11 +483,9 @@ int Engine::add_system(int nx, int ny, int nz, double h3, int* slot) {
       // levels above the bottom kernel that fuse their post-smoothing (a
       // property of the system alone, like all of its tiling)
       for (int l = 0; l < lb; ++l) {
-        Rec t;
         MgLevel& L = S.lev[l];
-        L.post = make_post_rec(L.nx, L.ny, L.nz, fp32_ ? 4 : 2, ncu_, &t)
-                     ? 1
-                     : (fp32_ && L.n <= kTileMaxCells && L.nx % 4 == 0 ? 2 : 0);
+        L.fuse = fuse_kind(L.nx, L.ny, L.nz, fp32_ ? 4 : 2, ncu_);
+        L.post = L.fuse >= 0 ? 1 : (fp32_ && L.n <= kTileMaxCells && L.nx % 4 == 0 ? 2 : 0);
       }
       for (int l = 1; l <= w && rc == APHPOIS_OK; ++l) {
         // a fused or tile level's second cycle leaves z[1] (the first
@@ -980,8 +992,12 @@ int Engine::build_tables() {
   // post-smoothing per level: fused for the systems whose level says so
   L_.any_lean = L_.any_plain = 0;
   int post_fused[kMaxLevels] = {}, post_plain[kMaxLevels] = {}, post_tile[kMaxLevels] = {};
-  std::vector<std::vector<Rec>> rlp(kMaxLevels), rlt(kMaxLevels);
-  std::vector<std::vector<int>> blp(kMaxLevels), blt(kMaxLevels);
+  std::vector<std::vector<Rec>> rlt(kMaxLevels), rlp[kFuseKinds];
+  std::vector<std::vector<int>> blt(kMaxLevels), blp[kFuseKinds];
+  for (int v = 0; v < kFuseKinds; ++v) {
+    rlp[v].resize(kMaxLevels);
+    blp[v].resize(kMaxLevels);
+  }
   for (int k = 0; k < ns; ++k) {
     System& s = *slots_[launch_slots_[k]];
     // per-system tile (autotuner) over the engine-wide override
@@ -1039,13 +1055,14 @@ int Engine::build_tables() {
         rlc[l].push_back(g);
         if (l == 0) nblk_pc = f.nblk;
         if (F.post == 1) {
-          post_fused[l] = 1;
+          const int v = F.fuse;
           Rec p{};
-          make_post_rec(F.nx, F.ny, F.nz, fp32_ ? 4 : 2, ncu_, &p);
+          make_post_rec(F.nx, F.ny, F.nz, fp32_ ? 4 : 2, ncu_, v, &p);
           p.sys = k;
-          p.blk0 = (int)blp[l].size();
-          for (int i = 0; i < p.nblk; ++i) blp[l].push_back((int)rlp[l].size());
-          rlp[l].push_back(p);
+          if (rlp[v][l].empty()) ++post_fused[l];
+          p.blk0 = (int)blp[v][l].size();
+          for (int i = 0; i < p.nblk; ++i) blp[v][l].push_back((int)rlp[v][l].size());
+          rlp[v][l].push_back(p);
           if (l == 0) nblk_pc = p.nblk;
         } else if (F.post == 2) {
           post_tile[l] = 1;
@@ -1145,8 +1162,12 @@ int Engine::build_tables() {
   long long nrec = (long long)rst.size() + rsm.size() + rru.size();
   long long nb2r = (long long)bst.size() + bsm.size() + bru.size();
   for (int l = 0; l < kMaxLevels; ++l) {
-    nrec += (long long)rlf[l].size() + rlc[l].size() + rlp[l].size() + rlt[l].size();
-    nb2r += (long long)blf[l].size() + blc[l].size() + blp[l].size() + blt[l].size();
+    nrec += (long long)rlf[l].size() + rlc[l].size() + rlt[l].size();
+    nb2r += (long long)blf[l].size() + blc[l].size() + blt[l].size();
+    for (int v = 0; v < kFuseKinds; ++v) {
+      nrec += (long long)rlp[v][l].size();
+      nb2r += (long long)blp[v][l].size();
+    }
   }
   if (nrec > rec_cap_) {
     if (d_rec_) APH_HIP(hipFree(d_rec_));
@@ -1177,15 +1198,19 @@ int Engine::build_tables() {
   for (int v : bru) b2r.push_back(v);
   rlev.assign(recs.size(), -1);
   size_t rec_lf_ofs[kMaxLevels], rec_lc_ofs[kMaxLevels], b2r_lf_ofs[kMaxLevels],
-      b2r_lc_ofs[kMaxLevels], rec_lp_ofs[kMaxLevels], b2r_lp_ofs[kMaxLevels],
+      b2r_lc_ofs[kMaxLevels], rec_lp_ofs[kFuseKinds][kMaxLevels], b2r_lp_ofs[kFuseKinds][kMaxLevels],
       rec_lt_ofs[kMaxLevels], b2r_lt_ofs[kMaxLevels];
   for (int l = 0; l < kMaxLevels; ++l) {
     rec_lf_ofs[l] = recs.size();
     recs.insert(recs.end(), rlf[l].begin(), rlf[l].end());
     rec_lc_ofs[l] = recs.size();
     recs.insert(recs.end(), rlc[l].begin(), rlc[l].end());
-    rec_lp_ofs[l] = recs.size();
-    recs.insert(recs.end(), rlp[l].begin(), rlp[l].end());
+    for (int v = 0; v < kFuseKinds; ++v) {
+      rec_lp_ofs[v][l] = recs.size();
+      recs.insert(recs.end(), rlp[v][l].begin(), rlp[v][l].end());
+      b2r_lp_ofs[v][l] = b2r.size();
+      b2r.insert(b2r.end(), blp[v][l].begin(), blp[v][l].end());
+    }
     rec_lt_ofs[l] = recs.size();
     recs.insert(recs.end(), rlt[l].begin(), rlt[l].end());
     rlev.resize(recs.size(), l);
@@ -1193,8 +1218,6 @@ int Engine::build_tables() {
     b2r.insert(b2r.end(), blf[l].begin(), blf[l].end());
     b2r_lc_ofs[l] = b2r.size();
     b2r.insert(b2r.end(), blc[l].begin(), blc[l].end());
-    b2r_lp_ofs[l] = b2r.size();
-    b2r.insert(b2r.end(), blp[l].begin(), blp[l].end());
     b2r_lt_ofs[l] = b2r.size();
     b2r.insert(b2r.end(), blt[l].begin(), blt[l].end());
   }
@@ -1256,10 +1279,11 @@ int Engine::build_tables() {
     L_.nlc[l] = (int)blc[l].size();
     L_.post_fused[l] = post_fused[l];
     L_.post_plain[l] = post_plain[l];
-    L_.vx_p[l] = fp32_ ? 4 : 2;
-    L_.ent_lp[l] = d_ent_ + rec_lp_ofs[l];
-    L_.b2r_lp[l] = map_of(b2r_lp_ofs[l], rlp[l].size());
-    L_.nlp[l] = (int)blp[l].size();
+    for (int v = 0; v < kFuseKinds; ++v) {
+      L_.ent_lp[v][l] = d_ent_ + rec_lp_ofs[v][l];
+      L_.b2r_lp[v][l] = map_of(b2r_lp_ofs[v][l], rlp[v][l].size());
+      L_.nlp[v][l] = (int)blp[v][l].size();
+    }
     L_.post_tile[l] = post_tile[l];
     L_.ent_lt[l] = d_ent_ + rec_lt_ofs[l];
     L_.b2r_lt[l] = map_of(b2r_lt_ofs[l], rlt[l].size());

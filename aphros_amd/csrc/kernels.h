@@ -12,6 +12,10 @@ namespace aph {
 // iterations, 20 the fastest or within 1 % at every size but 160^3 (12).
 constexpr int kCoarseSweeps = 20;
 
+// threads of a fused smoothing workgroup (MgLevel::fuse)
+constexpr int kFuseKinds = 3;
+constexpr int kFuseThreads[kFuseKinds] = {1024, 512, 256};
+
 // Device tables of one engine launch configuration.
 struct LaunchSet {
   const SysDev* sds = nullptr;
@@ -51,14 +55,14 @@ struct LaunchSet {
   const int* b2r_lc[kMaxLevels] = {};
   int nlc[kMaxLevels] = {};
   // post-smoothing of level l: some systems fused (k_mg_post over the
-  // whole-row tiles ent_lp, cells per thread vx_p), some with two sweeps
+  // whole-row tiles ent_lp[fuse]; post_fused counts the kinds present), some
+  // with two sweeps
   // (the sweep launches skip the systems whose level has post = 1)
   int post_fused[kMaxLevels] = {};
   int post_plain[kMaxLevels] = {};
-  int vx_p[kMaxLevels] = {};
-  const Ent* ent_lp[kMaxLevels] = {};
-  const int* b2r_lp[kMaxLevels] = {};
-  int nlp[kMaxLevels] = {};
+  const Ent* ent_lp[kFuseKinds][kMaxLevels] = {};
+  const int* b2r_lp[kFuseKinds][kMaxLevels] = {};
+  int nlp[kFuseKinds][kMaxLevels] = {};
   // small levels whose pre- and post-smoothing run as one tile launch each
   // (k_mg_tile, MgLevel::post == 2; 8^3 cells per workgroup, tiles_x/y/z)
   int post_tile[kMaxLevels] = {};
@@ -70,8 +74,6 @@ struct LaunchSet {
   hipGraphExec_t below0 = nullptr;
 };
 
-// threads of a k_mg_post workgroup
-constexpr int kPostBlock = 1024;
 // k_mg_tile: output cells per tile edge and threads per workgroup
 constexpr int kTile = 8;
 constexpr int kTileBlock = 512;

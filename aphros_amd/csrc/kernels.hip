@@ -1639,14 +1639,14 @@ __global__ __launch_bounds__(kBlock) void k_mg_restrict(const Ent* __restrict__ 
 // the neighbouring rows and columns, a plane after their first read (L2
 // hits).  The u rows just outside the tile (for the halo rows' v) and the u
 // planes before and after the tile come from memory.
-template <typename T, int VX, bool DOT, bool L0>
-__global__ __launch_bounds__(kPostBlock) void k_mg_post(const Ent* __restrict__ ents,
+template <typename T, int VX, int NT, bool DOT, bool L0>
+__global__ __launch_bounds__(NT, 4) void k_mg_post(const Ent* __restrict__ ents,
                                                         const int* __restrict__ b2r, int l_arg,
                                                         int wl, int so, int addzs) {
   const int l = L0 ? 0 : l_arg;
   using V = vec_t<T, VX>;
-  __shared__ T su[2][kPostBlock * VX];
-  __shared__ T sv[2][kPostBlock * VX];
+  __shared__ T su[2][NT * VX];
+  __shared__ T sv[2][NT * VX];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
   // launch tables (ents, b2r) are device arrays written by the host between launches only
   const gcp<Ent> en = gtab(ents + (b2r ? cload(gtab(b2r + b)) : 0));
@@ -1659,7 +1659,7 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_post(const Ent* __restrict__ 
   const MgLevel Lc = cload(&en->lc);
   const int nx = Lv.nx, ny = Lv.ny, nz = Lv.nz;
   const int lb = b - rc.blk0;
-  const int lx = rc.lx, ty = rc.ty;  // lx * VX == nx, ty <= kPostBlock / lx
+  const int lx = rc.lx, ty = rc.ty;  // lx * VX == nx, ty <= NT / lx
   const int tiy = lb % rc.tiles_y, tiz = lb / rc.tiles_y;
   const int ix = threadIdx.x % lx, iy = threadIdx.x / lx;
   const bool active = iy < ty;
@@ -1798,7 +1798,7 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_post(const Ent* __restrict__ 
   }
   if constexpr (DOT) {
     double acc[1] = {dot};
-    block_partial<1, 0u, kPostBlock>(acc, s.ppc, rc.nblk, lb);
+    block_partial<1, 0u, NT>(acc, s.ppc, rc.nblk, lb);
   }
 }
 
@@ -1824,8 +1824,8 @@ __device__ __forceinline__ vec_t<float, 4> bf4(unsigned a, unsigned b) {
 // (bfloat16 pairs) in registers; the second sweep reuses the first sweep's
 // ky and kx of the neighbouring cells instead of loading them again.  Same
 // arithmetic as k_mg_post.
-template <bool DOT, bool L0>
-__global__ __launch_bounds__(kPostBlock) void k_mg_post4(const Ent* __restrict__ ents,
+template <int NT, bool DOT, bool L0>
+__global__ __launch_bounds__(NT, 4) void k_mg_post4(const Ent* __restrict__ ents,
                                                          const int* __restrict__ b2r,
                                                          int l_arg, int wl, int so, int addzs) {
   using V = vec_t<float, 4>;
@@ -1834,8 +1834,8 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_post4(const Ent* __restrict__
   using V2 = vec_t<float, 2>;
   constexpr int VX = 4;
   const int l = L0 ? 0 : l_arg;
-  __shared__ float su[2][kPostBlock * VX];
-  __shared__ float sv[2][kPostBlock * VX];
+  __shared__ float su[2][NT * VX];
+  __shared__ float sv[2][NT * VX];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
   const gcp<Ent> en = gtab(ents + (b2r ? cload(gtab(b2r + b)) : 0));
   const Rec rc = cload(&en->rc);
@@ -2015,7 +2015,7 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_post4(const Ent* __restrict__
   }
   if constexpr (DOT) {
     double acc[1] = {dot};
-    block_partial<1, 0u, kPostBlock>(acc, s.ppc, rc.nblk, lb);
+    block_partial<1, 0u, NT>(acc, s.ppc, rc.nblk, lb);
   }
 }
 
@@ -2031,17 +2031,17 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_post4(const Ent* __restrict__
 // pairs across two steps, row pairs through LDS after the next barrier (odd
 // rows hand their sums to the even row above).  One barrier per step; u and z
 // planes double-buffered in LDS.
-template <typename T, int VX, bool L0>
-__global__ __launch_bounds__(kPostBlock) void k_mg_pre(const Ent* __restrict__ ents,
+template <typename T, int VX, int NT, bool L0>
+__global__ __launch_bounds__(NT, 4) void k_mg_pre(const Ent* __restrict__ ents,
                                                        const int* __restrict__ b2r, int l_arg,
                                                        int wl, int so) {
   static_assert(VX >= 2, "x pairs of the restriction are summed in the thread");
   constexpr int NP = VX / 2;
   const int l = L0 ? 0 : l_arg;
   using V = vec_t<T, VX>;
-  __shared__ T su[2][kPostBlock * VX];
-  __shared__ T sz[2][kPostBlock * VX];
-  __shared__ T sacc[kPostBlock * NP];
+  __shared__ T su[2][NT * VX];
+  __shared__ T sz[2][NT * VX];
+  __shared__ T sacc[NT * NP];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
   // launch tables (ents, b2r) are device arrays written by the host between launches only
   const gcp<Ent> en = gtab(ents + (b2r ? cload(gtab(b2r + b)) : 0));
@@ -2051,13 +2051,13 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_pre(const Ent* __restrict__ e
   if (wl >= 0 && wl >= s.mg_w) return;
   if (so && !s.sc->first) return;
   if constexpr (L0) {
-    if (s.lean && s.sc->ru && lean_verdict<kPostBlock>(s, s.sc, b - rc.blk0)) return;
+    if (s.lean && s.sc->ru && lean_verdict<NT>(s, s.sc, b - rc.blk0)) return;
   }
   const MgLevel Lv = cload(&en->lv);
   const MgLevel Lc = cload(&en->lc);
   const int nx = Lv.nx, ny = Lv.ny, nz = Lv.nz;
   const int lb = b - rc.blk0;
-  const int lx = rc.lx, ty = rc.ty;  // lx * VX == nx, ty even, <= kPostBlock / lx
+  const int lx = rc.lx, ty = rc.ty;  // lx * VX == nx, ty even, <= NT / lx
   const int tiy = lb % rc.tiles_y, tiz = lb / rc.tiles_y;
   const int ix = threadIdx.x % lx, iy = threadIdx.x / lx;
   const bool active = iy < ty;
@@ -2221,8 +2221,8 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_pre(const Ent* __restrict__ e
 // coefficients and the halo row's r and D^-1 on plane k + 1) are for step
 // k + 1; plane k-1's packed coefficients, r, ky and kx wait in LDS slots for
 // the residual.  Same arithmetic as k_mg_pre.
-template <bool L0>
-__global__ __launch_bounds__(kPostBlock) void k_mg_pre4(const Ent* __restrict__ ents,
+template <int NT, bool L0>
+__global__ __launch_bounds__(NT, 4) void k_mg_pre4(const Ent* __restrict__ ents,
                                                         const int* __restrict__ b2r, int l_arg,
                                                         int wl, int so) {
   using V = vec_t<float, 4>;
@@ -2231,16 +2231,16 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_pre4(const Ent* __restrict__ 
   constexpr int VX = 4;
   constexpr int NP = VX / 2;
   const int l = L0 ? 0 : l_arg;
-  __shared__ float su[2][kPostBlock * VX];
-  __shared__ float sz[2][kPostBlock * VX];
-  __shared__ float sacc[kPostBlock * NP];
+  __shared__ float su[2][NT * VX];
+  __shared__ float sz[2][NT * VX];
+  __shared__ float sacc[NT * NP];
   // each thread's plane k-1 data for the residual (own slots only): packed
   // coefficients, r, and {ky of row ym, kz of plane k-2}
-  __shared__ U4 sq[2][kPostBlock];
-  __shared__ V sr[kPostBlock];
-  __shared__ U4 sm[kPostBlock];
-  __shared__ unsigned skx[kPostBlock];               // kx of cell xm, plane k-1
-  __shared__ vec_t<float, NP> spend[kPostBlock];     // even rows' pending sums
+  __shared__ U4 sq[2][NT];
+  __shared__ V sr[NT];
+  __shared__ U4 sm[NT];
+  __shared__ unsigned skx[NT];               // kx of cell xm, plane k-1
+  __shared__ vec_t<float, NP> spend[NT];     // even rows' pending sums
   const int b = xcd_remap(blockIdx.x, gridDim.x);
   const gcp<Ent> en = gtab(ents + (b2r ? cload(gtab(b2r + b)) : 0));
   const Rec rc = cload(&en->rc);
@@ -2249,7 +2249,7 @@ __global__ __launch_bounds__(kPostBlock) void k_mg_pre4(const Ent* __restrict__ 
   if (wl >= 0 && wl >= s.mg_w) return;
   if (so && !s.sc->first) return;
   if constexpr (L0) {
-    if (s.lean && s.sc->ru && lean_verdict<kPostBlock>(s, s.sc, b - rc.blk0)) return;
+    if (s.lean && s.sc->ru && lean_verdict<NT>(s, s.sc, b - rc.blk0)) return;
   }
   const MgLevel Lv = cload(&en->lv);
   const MgLevel Lc = cload(&en->lc);
@@ -3619,43 +3619,46 @@ static void launch_sweep_l(const LaunchSet& L, hipStream_t st, int l, int zin, i
   }
 }
 
-// pre-smoothing + restriction of level l, fused, for the systems in ent_lp[l]
-template <typename T, bool L0>
-static void launch_pre_l(const LaunchSet& L, hipStream_t st, int l, int wl) {
-  const dim3 g(L.nlp[l]), t(kPostBlock);
-  if (L.vx_p[l] == 4) {
-    if constexpr (sizeof(T) == 4) {
-      hipLaunchKernelGGL((k_mg_pre4<L0>), g, t, 0, st, L.ent_lp[l], L.b2r_lp[l], l, wl,
-                         L.start_only);
-    }
+// pre-smoothing + restriction of level l, fused, for the systems in ent_lp[v][l]
+template <typename T, int NT, bool L0>
+static void launch_pre_n(const LaunchSet& L, hipStream_t st, int l, int wl, int v) {
+  if (L.nlp[v][l] == 0) return;
+  // FP32 engines use 4 cells per thread, FP64 engines 2 (the LDS planes of a
+  // 1024-thread workgroup: 5 x 1024 x VX x sizeof(T) bytes)
+  if constexpr (sizeof(T) == 4) {
+    hipLaunchKernelGGL((k_mg_pre4<NT, L0>), dim3(L.nlp[v][l]), dim3(NT), 0, st, L.ent_lp[v][l],
+                       L.b2r_lp[v][l], l, wl, L.start_only);
   } else {
-    hipLaunchKernelGGL((k_mg_pre<T, 2, L0>), g, t, 0, st, L.ent_lp[l], L.b2r_lp[l], l, wl,
-                       L.start_only);
+    hipLaunchKernelGGL((k_mg_pre<T, 2, NT, L0>), dim3(L.nlp[v][l]), dim3(NT), 0, st,
+                       L.ent_lp[v][l], L.b2r_lp[v][l], l, wl, L.start_only);
   }
 }
 
-// both post-smoothing sweeps of level l, fused, for the systems in ent_lp[l]
+template <typename T, bool L0>
+static void launch_pre_l(const LaunchSet& L, hipStream_t st, int l, int wl) {
+  launch_pre_n<T, kFuseThreads[0], L0>(L, st, l, wl, 0);
+  launch_pre_n<T, kFuseThreads[1], L0>(L, st, l, wl, 1);
+  launch_pre_n<T, kFuseThreads[2], L0>(L, st, l, wl, 2);
+}
+
+// both post-smoothing sweeps of level l, fused, for the same systems
+template <typename T, int NT, bool DOT, bool L0>
+static void launch_post_n(const LaunchSet& L, hipStream_t st, int l, int wl, int addzs, int v) {
+  if (L.nlp[v][l] == 0) return;
+  if constexpr (sizeof(T) == 4) {
+    hipLaunchKernelGGL((k_mg_post4<NT, DOT, L0>), dim3(L.nlp[v][l]), dim3(NT), 0, st,
+                       L.ent_lp[v][l], L.b2r_lp[v][l], l, wl, L.start_only, addzs);
+  } else {
+    hipLaunchKernelGGL((k_mg_post<T, 2, NT, DOT, L0>), dim3(L.nlp[v][l]), dim3(NT), 0, st,
+                       L.ent_lp[v][l], L.b2r_lp[v][l], l, wl, L.start_only, addzs);
+  }
+}
+
 template <typename T, bool DOT, bool L0>
 static void launch_post_l(const LaunchSet& L, hipStream_t st, int l, int wl, int addzs) {
-  const dim3 g(L.nlp[l]), t(kPostBlock);
-  // FP32 engines use 4 cells per thread, FP64 engines 2 (the LDS planes of a
-  // 1024-thread workgroup: 5 x 1024 x VX x sizeof(T) bytes)
-  switch (L.vx_p[l]) {
-    case 4:
-      if constexpr (sizeof(T) == 4) {
-        hipLaunchKernelGGL((k_mg_post4<DOT, L0>), g, t, 0, st, L.ent_lp[l], L.b2r_lp[l], l,
-                           wl, L.start_only, addzs);
-      }
-      break;
-    case 2:
-      hipLaunchKernelGGL((k_mg_post<T, 2, DOT, L0>), g, t, 0, st, L.ent_lp[l], L.b2r_lp[l],
-                         l, wl, L.start_only, addzs);
-      break;
-    default:
-      hipLaunchKernelGGL((k_mg_post<T, 1, DOT, L0>), g, t, 0, st, L.ent_lp[l], L.b2r_lp[l],
-                         l, wl, L.start_only, addzs);
-      break;
-  }
+  launch_post_n<T, kFuseThreads[0], DOT, L0>(L, st, l, wl, addzs, 0);
+  launch_post_n<T, kFuseThreads[1], DOT, L0>(L, st, l, wl, addzs, 1);
+  launch_post_n<T, kFuseThreads[2], DOT, L0>(L, st, l, wl, addzs, 2);
 }
 
 template <typename T, int MODE, bool DOT>
@@ -3804,7 +3807,7 @@ hipError_t capture_below0(int fp32, const LaunchSet& L, hipStream_t st) {
 static int cycle_launches(const LaunchSet& L, int l) {
   int n = L.bottom_at[l] ? 1 : 0;
   if (l >= L.deep) return n;
-  n += (L.post_fused[l] ? 2 : 0) + (L.post_plain[l] ? 4 : 0) + (L.post_tile[l] ? 2 : 0) +
+  n += 2 * L.post_fused[l] + (L.post_plain[l] ? 4 : 0) + (L.post_tile[l] ? 2 : 0) +
        cycle_launches(L, l + 1);
   if (l < L.mg_w) n += 1 + cycle_launches(L, l + 1);
   return n;

@@ -1,6 +1,5 @@
 """One multigrid cycle against the oracle's at the sizes where a level changes
-its kernels: the smallest fused levels (2^19 cells in FP64, 3 * 2^20 in
-mixed precision), short and long rows, partial row tiles, with and without a mass
+its kernels: small fused levels and their workgroup sizes, short and long rows, partial row tiles, with and without a mass
 term and W levels."""
 import numpy as np
 import pytest
@@ -55,6 +54,26 @@ def _cycle_error(shape, precision, w, mass, seed=1):
     (L.MIXED, (16, 768, 256), 1),     # rows of 64 threads, 16 planes
 ])
 def test_smallest_fused_levels(precision, shape, w, mass):
+    assert _cycle_error(shape, precision, w, mass) <= TOL[precision]
+
+
+@pytest.mark.parametrize("mass", [False, True])
+@pytest.mark.parametrize("precision,shape,w", [
+    (L.MIXED, (64, 64, 96), 0),       # 3 * 2^17 cells, 256 threads
+    (L.MIXED, (40, 136, 80), 0),      # 12 rows of 20 threads, a partial row tile
+    (L.MIXED, (96, 80, 64), 1),       # 16 rows of 16 threads, partial in y and z
+    (L.MIXED, (24, 128, 128), 0),     # 8 rows of 32 threads, 256 threads
+    (L.MIXED, (24, 128, 144), 0),     # 36 threads a row: 512 threads
+    (L.MIXED, (8, 200, 256), 0),      # 64 threads a row, 8 planes, partial
+    (L.MIXED, (24, 64, 272), 0),      # 68 threads a row: 1024 threads
+    (L.MIXED, (128, 256, 256), 1),    # 2^23 cells, levels of 1024 and 256 threads
+    (L.FP64, (16, 16, 16), 0),        # the smallest fused level
+    (L.FP64, (8, 8, 66), 0),          # 33 threads a row: 512 threads, 10 rows
+    (L.FP64, (8, 34, 64), 0),         # 8 rows of 32 threads, partial, 8 planes
+    (L.FP64, (8, 32, 136), 0),        # 68 threads a row: 1024 threads
+    (L.FP64, (40, 48, 20), 1),        # 24 rows of 10 threads
+])
+def test_fused_workgroup_sizes(precision, shape, w, mass):
     assert _cycle_error(shape, precision, w, mass) <= TOL[precision]
 
 
