@@ -19,23 +19,62 @@ long long cdiv(long long a, long long b) { return (a + b - 1) / b; }
 
 // Stencil tiling of one system: lx lanes of VX cells per row (at most
 // lx_max by default), kBlock/lx rows, bz planes per workgroup.
+//
+// slots > 0 (the PCG kernels): the workgroups the device holds at once.  Rows
+// whose power-of-two lanes would leave a tenth of the lanes idle take the lane
+// count that fills most of a workgroup's threads instead (72 columns: 3 rows of
+// 72 lanes, not a full and an eighth-full tile of 64), and launches of `slots`
+// workgroups or more split z so that the rounds times the planes of one (bz and
+// two around them) are least: a target of 1024 workgroups met by rounding up was
+// 1040 to 1280 at most sizes, a second round for a few of them.  even: an even
+// number of rows.  ms per multigrid solve: mixed 144^3 12.5 -> 10.8, 160^3 10.4 ->
+// 10.0, 192^3 14.6 -> 12.6, 224^3 22.4 -> 20.3, 288^3 45.2 -> 36.0, 320^3 43.1 ->
+// 35.0, 384^3 60.3 -> 51.7, 448^3 93.8 -> 83.8; FP64 160^3 18.6 -> 15.7, 192^3 24.7
+// -> 22.1; powers of two the same tiling as before.
 Rec make_stencil_rec(int nx, int ny, int nz, int vx, int blocks_target, const Tuning& tu,
-                     int lx_max = 64) {
+                     int lx_max = 64, int slots = 0, bool even = false) {
   Rec r{};
   const int cols = std::max(1, nx / vx);
   int lx = tu.lx > 0 ? tu.lx : std::min(lx_max, pow2floor(cols));
   lx = std::max(1, std::min(lx, kBlock));
+  // cells over lanes of a row of tiles, threads used over threads
+  auto fill = [&](int v) {
+    return (double)cols / (double)(cdiv(cols, v) * v) * (double)(kBlock / v * v) / kBlock;
+  };
+  if (slots > 0 && tu.lx <= 0 && fill(lx) < 0.9) {
+    // of the lane counts, the one with the most cells per access: a row of a
+    // tile also reads the cells beside it, a tile the rows beside it
+    auto worth = [&](int v) {
+      const double rows = kBlock / v;
+      return fill(v) * v / (v + 4.0) * rows / (rows + 1.0);
+    };
+    for (int v = std::min(cols, kBlock / 2); v >= 8; --v) {
+      if (even && (kBlock / v) % 2 != 0) continue;
+      if (worth(v) > worth(lx)) lx = v;
+    }
+  }
   const int rows = kBlock / lx;
   r.lx = lx;
   r.tiles_x = (int)cdiv(cols, lx);
   r.tiles_y = (int)cdiv(ny, rows);
+  const long long cols_tiles = (long long)r.tiles_x * r.tiles_y;
   int bz;
   if (tu.bz > 0) {
     bz = tu.bz;
   } else {
-    const long long cols_tiles = (long long)r.tiles_x * r.tiles_y;
     const long long tz = std::max(1LL, cdiv(blocks_target, cols_tiles));
     bz = (int)cdiv(nz, tz);
+    if (slots > 0 && blocks_target >= slots) {
+      long long best = -1;
+      for (int k = 1; k <= nz; ++k) {
+        const int b = (int)cdiv(nz, k);
+        const long long cost = cdiv(cols_tiles * cdiv(nz, b), slots) * (b + 2);
+        if (best < 0 || cost < best) {
+          best = cost;
+          bz = b;
+        }
+      }
+    }
   }
   bz = std::max(1, std::min(bz, nz));
   r.bz = bz;
@@ -145,10 +184,12 @@ void system_tiling(int method, int nx, int ny, int nz, int vx, const Tuning& tu,
   // 64: whole rows at 512^3 took 0.718 against 0.722 ms but fetched 3.51
   // instead of 3.15 GB per launch (two output rows per block re-read two halo
   // rows of z and p)
+  // (the PCG kernels hold four workgroups per CU, 256 CUs)
+  const int slots = method == kPcg ? 1024 : 0;
   *st = make_stencil_rec(nx, ny, nz, method == kPcg ? vx : 1, tgt, tu,
-                         method == kPcg && fp64 ? 128 : 64);
+                         method == kPcg && fp64 ? 128 : 64, slots);
   Tuning none;
-  *ru = make_stencil_rec(nx, ny, nz, vx_ru, tgt, none);
+  *ru = make_stencil_rec(nx, ny, nz, vx_ru, tgt, none, 64, slots);
   Rec b{};
   const int cells = tu.sm > 0 ? tu.sm : (method == kPcg ? 4 * vx : 4);
   b.nblk = (int)std::min(16384LL, std::max(1LL, cdiv(n, (long long)kBlock * cells)));
@@ -1035,7 +1076,7 @@ int Engine::build_tables() {
         const long long ftgt = F.n >= (1LL << 21) ? std::min(1024LL, cdiv(F.n, 2048))
                                                   : std::max(1LL, cdiv(F.n, 512));
         // level 0 follows the system's stencil tuning (autotuner / set_tile)
-        Rec f = make_stencil_rec(F.nx, F.ny, F.nz, vxl[l], ftgt, l == 0 ? tu : none);
+        Rec f = make_stencil_rec(F.nx, F.ny, F.nz, vxl[l], ftgt, l == 0 ? tu : none, 64, 1024, true);
         // the fused restriction sums plane pairs inside one workgroup: even
         // plane counts per tile (F.nz is even on every coarsened level)
         if (f.bz & 1) {

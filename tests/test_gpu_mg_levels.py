@@ -141,3 +141,23 @@ def test_reductions_at_the_size_line(precision):
         assert cut["converged"] == 0 and cut["iter"] == 4
         assert abs(O.true_relres(e, x3) / cut["true_relres"] - 1) <= 1e-6
     b.close()
+
+
+@pytest.mark.parametrize("precond", [L.PRECOND_MG, L.PRECOND_JACOBI])
+@pytest.mark.parametrize("precision", [L.MIXED, L.FP64])
+@pytest.mark.parametrize("shape", [
+    (16, 40, 288),    # 72 / 144 columns
+    (48, 40, 160),    # 40 / 80 columns
+    (16, 24, 104),    # 26 / 52 columns
+    (64, 128, 288),   # beyond the resident solves
+    (80, 96, 336),    # 84 / 168 columns
+])
+def test_row_tiles_that_are_no_power_of_two(shape, precision, precond):
+    e = _system(shape, 9, False)
+    s = Poisson(shape, method=L.PCG, precision=precision, resmode=L.RES_REL_TRUE, tol=1e-8,
+                maxiter=5000, precond=precond)
+    s.set_system(e)
+    x, info = s.solve(None)
+    s.close()
+    assert info["converged"] == 1
+    assert abs(O.true_relres(e, x) / info["true_relres"] - 1) <= 1e-6
