@@ -247,7 +247,8 @@ __device__ __forceinline__ Tile tile_of(const Rec& rc, const SysDev& s, int lb) 
 // reliable update follows, before it touches r.  Six of an iteration's launches
 // fall away (four finalize kernels, an accumulation pass, (r, z)), which cost
 // ~4 us each while the kernels of a small system take 5 to 10 us: 64^3 63 -> 54
-// us per iteration of a solve, 32^3 46 -> 38.
+// us per iteration of a solve, 32^3 46 -> 38.  The operator's and the update's
+// first loads are issued before the sums: 32^3 2.53 -> 2.42 ms, 64^3 2.18 -> 2.11.
 // ===========================================================================
 
 // Before the operator: beta from (r, z).  False: the solve ends.
@@ -428,9 +429,6 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
   const int nx = s.nx, ny = s.ny, nz = s.nz;
   const int cur = sc->cur;
   double beta = sc->beta;
-  if constexpr (!SC) {
-    if (lean && !lean_beta(s, sc, lb, beta)) return;
-  }
   const gcp<T> __restrict__ r = (gcp<T>)s.z;  // r (Jacobi-scaled) or z = M^-1 r
   const gcp<T> __restrict__ pin = (gcp<T>)s.p[cur];
   const gmp<T> __restrict__ pout = (gmp<T>)s.p[cur ^ 1];
@@ -467,8 +465,8 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
   const double xa = sc->alpha;
   const gmp<T> __restrict__ xh = (gmp<T>)s.xh;
   // pnew_st, and the x^ update on cells the tile owns
-  auto pnew_own = [&](long long i) -> V {
-    const vec_t<double, VX> po = ldd<T, VX>(pin, i);
+  auto pnew_own_of = [&](long long i, V zv, V pv) -> V {
+    const vec_t<double, VX> po = cvt<VX>(pv);
     if constexpr (XH) {
       using D1 = vec_t<double, VX>;
       if (xs == 0) {
@@ -477,7 +475,10 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
         std_<T, VX>(xh, i, (D1)(0.0) + xa * po);  // the sum with x^ = 0, to the bit
       }
     }
-    return __builtin_convertvector(ldd<T, VX>(r, i) + beta * po, V);
+    return __builtin_convertvector(cvt<VX>(zv) + beta * po, V);
+  };
+  auto pnew_own = [&](long long i) -> V {
+    return pnew_own_of(i, ldv<T, VX>(r, i), ldv<T, VX>(pin, i));
   };
   auto sld = [&](long long i) -> V {
     if constexpr (SC) return ldv<T, VX>(S, i);
@@ -495,14 +496,31 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
   // registers: u of planes z-1, z, z+1 in A; p, S and kz kept as stored (T)
   D um = (A)0, uc = (A)0;
   V pc = (T)0, Sc = (T)0, kzm = (T)0;
+  const long long i0 = (long long)(t.za == 0 ? nz - 1 : t.za - 1) * pl + row + t.x0;
+  const long long i1 = (long long)t.za * pl + row + t.x0;
+  V zv0 = (T)0, pv0 = (T)0, zv1 = (T)0, pv1 = (T)0;
+  if constexpr (!SC) {
+    // the first planes' loads under way while a lean system's beta is summed up
+    if (t.active) {
+      zv0 = ldv<T, VX>(r, i0);
+      pv0 = ldv<T, VX>(pin, i0);
+      kzm = ldv<T, VX>(kz, i0);
+      zv1 = ldv<T, VX>(r, i1);
+      pv1 = ldv<T, VX>(pin, i1);
+    }
+    if (lean && !lean_beta(s, sc, lb, beta)) return;
+  }
   if (t.active) {
-    const int zm0 = t.za == 0 ? nz - 1 : t.za - 1;
-    long long i = (long long)zm0 * pl + row + t.x0;
-    um = unew(i);
-    kzm = ldv<T, VX>(kz, i);
-    i = (long long)t.za * pl + row + t.x0;
-    pc = pnew_own(i);
-    Sc = sld(i);
+    if constexpr (SC) {
+      um = unew(i0);
+      kzm = ldv<T, VX>(kz, i0);
+      pc = pnew_own(i1);
+    } else {
+      um = __builtin_convertvector(
+          __builtin_convertvector(cvt<VX>(zv0) + beta * cvt<VX>(pv0), V), D);
+      pc = pnew_own_of(i1, zv1, pv1);
+    }
+    Sc = sld(i1);
     uc = cva<A, VX>(Sc) * cva<A, VX>(pc);
 #pragma unroll
     for (int v = 0; v < VX; ++v) su[0][lofs + v] = uc[v];
@@ -653,6 +671,19 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update(const Ent* __restrict__ e
   long long beg, end;
   stream_range<VX>(s.n, rc.nblk, lb, beg, end);
   if (lean) {
+    // the first cells' loads under way while alpha is summed up
+    constexpr int NP = 2;
+    using V = vec_t<T, VX>;
+    V rv[NP], qv[NP];
+    const long long own = beg + (long long)threadIdx.x * VX;
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      const long long i = own + (long long)k * kBlock * VX;
+      if (i < end) {
+        rv[k] = ldv<T, VX>((gcp<T>)r, i);
+        qv[k] = ldv<T, VX>((gcp<T>)q, i);
+      }
+    }
     const int what = lean_step(s, sc, lb, alpha);
     if (what < 0) return;
     if (what > 0) {
@@ -663,9 +694,13 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update(const Ent* __restrict__ e
       block_partial<1, 0u>(acc, s.pacc, rc.nblk, lb);
       return;
     }
-    for (long long i = beg + (long long)threadIdx.x * VX; i < end;
-         i += (long long)kBlock * VX)
-      std_<T, VX>(r, i, rnd<T, VX>(ldd<T, VX>(r, i) - alpha * ldd<T, VX>(q, i)));
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      const long long i = own + (long long)k * kBlock * VX;
+      if (i < end) std_<T, VX>(r, i, cvt<VX>(rv[k]) - alpha * cvt<VX>(qv[k]));
+    }
+    for (long long i = own + (long long)NP * kBlock * VX; i < end; i += (long long)kBlock * VX)
+      std_<T, VX>(r, i, ldd<T, VX>(r, i) - alpha * ldd<T, VX>(q, i));
     return;
   }
   for (long long i = beg + (long long)threadIdx.x * VX; i < end; i += (long long)kBlock * VX) {

@@ -86,26 +86,31 @@ __device__ __forceinline__ void block_partial(double (&v)[NV], double* partials,
 template <int NV, unsigned MaxMask, int NT = kBlock>
 __device__ __forceinline__ void reduce_partials(double (&v)[NV], const double* partials,
                                                 int nblk) {
+  // J independent accumulators per value (all of their loads in flight; two of
+  // four values, for the registers), combined in a fixed order
+  constexpr int J = NV > 3 ? 2 : 4;
+  double t[NV][4] = {};
+  auto add = [&](int j, int i) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const double pv = partials[(long long)k * nblk + i];
+      t[k][j] = ((MaxMask >> k) & 1u) ? fmax(t[k][j], pv) : t[k][j] + pv;
+    }
+  };
+  int i = threadIdx.x;
+#pragma unroll 1
+  for (; i + (J - 1) * NT < nblk; i += J * NT) {
+#pragma unroll
+    for (int j = 0; j < J; ++j) add(j, i + j * NT);
+  }
+  if (i < nblk) add(0, i);
+  if (J > 2 && i + NT < nblk) add(1, i + NT);
+  if (J > 2 && i + 2 * NT < nblk) add(2, i + 2 * NT);
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const bool mx = (MaxMask >> k) & 1u;
-    const double* pk = partials + (long long)k * nblk;
-    // four independent accumulators (four loads in flight), combined in a
-    // fixed order
-    double t[4] = {0.0, 0.0, 0.0, 0.0};
-    int i = threadIdx.x;
-    for (; i + 3 * NT < nblk; i += 4 * NT) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const double pv = pk[i + j * NT];
-        t[j] = mx ? fmax(t[j], pv) : t[j] + pv;
-      }
-    }
-    for (int j = 0; i < nblk; i += NT, ++j) {
-      const double pv = pk[i];
-      t[j] = mx ? fmax(t[j], pv) : t[j] + pv;
-    }
-    v[k] = mx ? fmax(fmax(t[0], t[1]), fmax(t[2], t[3])) : (t[0] + t[1]) + (t[2] + t[3]);
+    const double* s = t[k];
+    v[k] = ((MaxMask >> k) & 1u) ? fmax(fmax(s[0], s[1]), fmax(s[2], s[3]))
+                                 : (s[0] + s[1]) + (s[2] + s[3]);
   }
   block_reduce<NV, MaxMask, NT>(v);
 }
