@@ -175,10 +175,14 @@ void system_tiling(int method, int nx, int ny, int nz, int vx, const Tuning& tu,
                    Rec* sm, Rec* ru, int vx_ru, int fp64) {
   // The tiling of a system depends on that system only, so its reduction
   // trees (and results) are the same alone and inside a batch.
-  // ~one workgroup per 2048 cells, at most 1024 (about one resident wave
-  // set of the 256 CUs: long z marches, few re-read halo planes)
+  // ~one workgroup per 2048 cells (PCG: 512), at most 1024 (about one resident
+  // wave set of the 256 CUs: long z marches, few re-read halo planes).  A small
+  // operator is a chain of planes, so fewer planes beat the halo re-read from
+  // the caches: multigrid solves with 2048 -> 512, mixed 32^3 2.44 -> 2.31 ms,
+  // 64^3 2.14 -> 2.05, 96^3 4.92 -> 4.75, FP64 64^3 4.71 -> 4.57; 128^3 the same.
   const long long n = (long long)nx * ny * nz;
-  const long long tgt = std::min(1024LL, std::max(1LL, cdiv(n, 2048)));
+  const long long tgt =
+      std::min(1024LL, std::max(1LL, cdiv(n, method == kPcg ? 512 : 2048)));
   // the FP64 PCG operator: rows of up to 128 lanes (whole rows at 256^3:
   // 0.249 -> 0.240 ms per launch against 64 lanes).  The FP32 operator keeps
   // 64: whole rows at 512^3 took 0.718 against 0.722 ms but fetched 3.51
@@ -191,7 +195,7 @@ void system_tiling(int method, int nx, int ny, int nz, int vx, const Tuning& tu,
   Tuning none;
   *ru = make_stencil_rec(nx, ny, nz, vx_ru, tgt, none, 64, slots);
   Rec b{};
-  const int cells = tu.sm > 0 ? tu.sm : (method == kPcg ? 4 * vx : 4);
+  const int cells = tu.sm > 0 ? tu.sm : (method == kPcg ? (n <= (1LL << 18) ? 2 : 4) * vx : 4);
   b.nblk = (int)std::min(16384LL, std::max(1LL, cdiv(n, (long long)kBlock * cells)));
   b.tiles_x = b.nblk;
   b.tiles_y = b.tiles_z = 1;
