@@ -107,8 +107,9 @@ struct SysDev {
   double* pacc;
   double* pres;
   double* ppc;
-  // 1: a multigrid system whose reductions are finished by every workgroup of
-  // the kernel that needs the result (kernels.hip), not by finalize kernels
+  // a multigrid system whose reductions are finished by every workgroup of the
+  // kernel that needs the result (kernels.hip), not by finalize kernels: 1 all,
+  // 2 all but the update's
   int lean;
   unsigned* counter;
   Scalars* sc;

@@ -118,6 +118,8 @@ constexpr long long kTileMaxCells = 1LL << 19;
 // -> 5.57, 128^3 8.17 -> 7.79, 192^3 15.6 -> 15.4; FP64 64^3 5.96 -> 5.35, 128^3
 // 12.2 -> 11.7, 192^3 the same; above, the operator's reads of r cost more than
 // the launches: 224 x 192 x 256 23.5 -> 24.2, 320^3 42.9 -> 44.3 (256^3 the same).
+// There the update keeps its own finalize kernel (lean 2): 192 x 192 x 256 16.64
+// -> 16.33, 256^3 24.4 -> 23.9, 320^3 34.8 -> 34.6, 512^3 175.4 -> 174.9.
 constexpr long long kLeanCells = 1LL << 23;
 // Iterations of one resident launch: a launch costs about 30 us more than its
 // iterations (of 7 to 25 us); the server's steps are shorter, so that a new
@@ -1035,7 +1037,7 @@ int Engine::build_tables() {
     }
   }
   // post-smoothing per level: fused for the systems whose level says so
-  L_.any_lean = L_.any_plain = 0;
+  L_.any_mid = L_.any_plain = 0;
   int post_fused[kMaxLevels] = {}, post_plain[kMaxLevels] = {}, post_tile[kMaxLevels] = {};
   std::vector<std::vector<Rec>> rlt(kMaxLevels), rlp[kFuseKinds];
   std::vector<std::vector<int>> blt(kMaxLevels), blp[kFuseKinds];
@@ -1132,7 +1134,7 @@ int Engine::build_tables() {
     // partials: 3 values per block of the largest reducing launch of this
     // system; lean: 4 (operator) + 1 (x64) + 3 (residual) + 1 ((r, z)), apart
     const long long nmax = std::max(std::max(a.nblk, nblk_pc), std::max(b.nblk, c.nblk));
-    s.dev.lean = pc_ && s.dev.mg_lb > 0 && s.n <= kLeanCells ? 1 : 0;
+    s.dev.lean = !pc_ || s.dev.mg_lb == 0 ? 0 : (s.n <= kLeanCells ? 1 : 2);
     const long long need = (s.dev.lean ? 9 : 3) * nmax * 8;
     if (need > s.partials_cap) {
       if (s.partials) APH_HIP(hipFree(s.partials));
@@ -1145,7 +1147,7 @@ int Engine::build_tables() {
     s.dev.pacc = s.dev.partials + (s.dev.lean ? 4 * nmax : 0);
     s.dev.pres = s.dev.partials + (s.dev.lean ? 5 * nmax : 0);
     s.dev.ppc = s.dev.partials + (s.dev.lean ? 8 * nmax : 0);
-    (s.dev.lean ? L_.any_lean : L_.any_plain) = 1;
+    if (s.dev.lean != 1) (s.dev.lean ? L_.any_mid : L_.any_plain) = 1;
     s.dev.nblk_st = a.nblk;
     s.dev.nblk_sm = b.nblk;
     s.dev.nblk_ru = c.nblk;
@@ -1346,7 +1348,8 @@ int Engine::capture() {
   const int nk = iter_kernels(method_, pc_ ? 1 : 0);
   const int ng = graph_kernels(method_, pc_ ? 1 : 0);  // of them in the graph
   // launches per iteration (the multigrid cycle counts as one kernel in nk)
-  const int nl = (L_.any_plain ? ng + (pc_ ? 1 : 0) : 4) + (pc_ ? vcycle_launches(L_) - 2 : 0);
+  const int nl = (L_.any_plain ? ng + (pc_ ? 1 : 0) : (L_.any_mid ? 6 : 4)) +
+                 (pc_ ? vcycle_launches(L_) - 2 : 0);
   int k = check_every_;
   if (k <= 0) {
     // about 4 ms of work per replay (iterations past convergence cost a

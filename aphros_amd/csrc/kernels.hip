@@ -239,7 +239,7 @@ __device__ __forceinline__ Tile tile_of(const Rec& rc, const SysDev& s, int lb) 
 }
 
 // ===========================================================================
-// Lean systems (SysDev::lean: multigrid, at most kLeanCells cells).  The kernel
+// Lean systems (SysDev::lean: multigrid of two or more levels).  The kernel
 // after a reducing one sums its partials itself, every workgroup the same way,
 // and workgroup 0 stores what the iteration keeps; no field is stored by a
 // kernel whose other workgroups still read it.  The operator also forms (r, r),
@@ -249,6 +249,8 @@ __device__ __forceinline__ Tile tile_of(const Rec& rc, const SysDev& s, int lb) 
 // ~4 us each while the kernels of a small system take 5 to 10 us: 64^3 63 -> 54
 // us per iteration of a solve, 32^3 46 -> 38.  The operator's and the update's
 // first loads are issued before the sums: 32^3 2.53 -> 2.42 ms, 64^3 2.18 -> 2.11.
+// lean == 2 (more than kLeanCells cells): the operator does not read r, so the update keeps its
+// finalize kernel and the accumulation pass follows it; four launches fall away.
 // ===========================================================================
 
 // Before the operator: beta from (r, z).  False: the solve ends.
@@ -301,6 +303,32 @@ __device__ __forceinline__ int lean_step(const SysDev& s, Scalars* sc, int lb, d
     }
   }
   return bad ? -1 : (trig ? 1 : 0);
+}
+
+// The same with lean == 2: alpha; the update's own finalize kernel decides on
+// the reliable update.  False: the solve ends.
+__device__ __forceinline__ bool mid_step(const SysDev& s, Scalars* sc, int lb, double& alpha) {
+  double pq[1];
+  reduce_partials<1, 0u>(pq, s.partials, s.nblk_st);
+  const bool bad = !(pq[0] != 0.0) || !isfinite(pq[0]);
+  const double rz = sc->rz;
+  alpha = rz / pq[0];
+  if (lb == 0 && threadIdx.x == 0) {
+    if (bad) {
+      sc->status = 6;
+      sc->done = 1;
+    } else {
+      sc->alpha = alpha;
+      sc->cur = sc->cur_next;
+      sc->iter = sc->iter_next;
+      sc->xh_fold = sc->xf_next;
+      sc->rho = rz;
+      sc->first = 0;
+      sc->rz_ok = 0;
+      sc->ru = 0;
+    }
+  }
+  return !bad;
 }
 
 // Before the FP64 residual: the mean of x64.
@@ -421,7 +449,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
   const Rec rc = en.rc;
   const SysDev& s = en.s;
   Scalars* sc = s.sc;
-  const bool lean = !SC && s.lean;
+  const bool lean = !SC && s.lean, dots = !SC && s.lean == 1;
   // ru: a reliable update is pending (lean: the last one, done by now)
   if (sc->done || (!lean && sc->ru) || s.pers) return;
   const int lb = b - rc.blk0;
@@ -536,7 +564,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
       const long long in = (long long)wrapp(z, nz) * pl + row + t.x0;
       V rv = (T)0;
       if constexpr (!SC) {
-        if (lean) rv = ldv<T, VX>(rr, ic);
+        if (dots) rv = ldv<T, VX>(rr, ic);
       }
       const V pn = z + 1 < t.zb ? pnew_own(in) : pnew_st(in);
       const V Sn = sld(in);
@@ -587,7 +615,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
 #pragma unroll
       for (int v = 0; v < VX; ++v) dot += pcd[v] * qd[v];
       if constexpr (!SC) {
-        if (lean) {
+        if (dots) {
           const vec_t<double, VX> rd = cvt<VX>(rv);
 #pragma unroll
           for (int v = 0; v < VX; ++v) {
@@ -605,7 +633,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
     __syncthreads();
   }
   if constexpr (!SC) {
-    if (lean) {
+    if (dots) {
       double acc[4] = {dot, dr[0], dr[1], dr[2]};
       block_partial<4, 0u>(acc, s.partials, rc.nblk, lb);
       return;
@@ -660,7 +688,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update(const Ent* __restrict__ e
   const Rec rc = en.rc;
   const SysDev& s = en.s;
   Scalars* sc = s.sc;
-  const bool lean = s.lean;
+  const int lean = s.lean;
   // ru: a reliable update is pending (lean: the last one, done by now)
   if (sc->done || (!lean && sc->ru) || s.pers) return;
   const int lb = b - rc.blk0;
@@ -670,7 +698,11 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update(const Ent* __restrict__ e
   double acc[1] = {0.0};
   long long beg, end;
   stream_range<VX>(s.n, rc.nblk, lb, beg, end);
-  if (lean) {
+  double* part = s.partials;
+  if (lean == 2) {
+    if (!mid_step(s, sc, lb, alpha)) return;
+    part = s.pres;
+  } else if (lean) {
     // the first cells' loads under way while alpha is summed up
     constexpr int NP = 2;
     using V = vec_t<T, VX>;
@@ -709,18 +741,18 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update(const Ent* __restrict__ e
 #pragma unroll
     for (int v = 0; v < VX; ++v) acc[0] += rv[v] * rv[v];
   }
-  block_partial<1, 0u>(acc, s.partials, rc.nblk, lb);
+  block_partial<1, 0u>(acc, part, rc.nblk, lb);
 }
 
 __global__ __launch_bounds__(kBlock) void k_fin_pcg_update(const SysDev* __restrict__ sds) {
   const SysDev& s = sds[blockIdx.x];
   Scalars* sc = s.sc;
-  if (s.lean || sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
+  if (s.lean == 1 || sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
   double acc[1];
-  reduce_partials<1, 0u>(acc, s.partials, s.nblk_sm);
+  reduce_partials<1, 0u>(acc, s.lean ? s.pres : s.partials, s.nblk_sm);
   if (threadIdx.x == 0) {
     const double rn = acc[0];
-    sc->iter += 1;
+    if (!s.lean) sc->iter += 1;  // else counted by the update
     const double est = sc->gamma * sqrt(rn);
     const bool trig = !isfinite(rn) || sqrt(rn) < sc->delta * sqrt(sc->rmax2) ||
                       est <= 0.9 * sc->tol || sc->iter > sc->maxiter;
@@ -754,7 +786,7 @@ __global__ __launch_bounds__(kBlock) void k_ru_accum(const Ent* __restrict__ ent
   Scalars* sc = s.sc;
   // a zero start: x64 and x^ are zero already, and so is their mean
   if (sc->done || !sc->ru || sc->zero_start) return;
-  if (s.lean && !so) return;
+  if (s.lean == 1 && !so) return;
   if (so && sc->pc && !sc->first) return;
   const int lb = b - rc.blk0;
   long long beg, end;
@@ -3865,10 +3897,10 @@ static void launch_pcg_kernel(const LaunchSet& L, hipStream_t st, int j) {
       APH_LAUNCH((k_pcg_update<T, VX>), L.nsm, st, L.ent_sm, L.b2r_sm);
       break;
     case 3:
-      if (L.any_plain) APH_LAUNCH(k_fin_pcg_update, L.ns, st, L.sds);
+      if (L.any_plain || L.any_mid) APH_LAUNCH(k_fin_pcg_update, L.ns, st, L.sds);
       break;
     case 4:
-      if (L.any_plain || L.start_only)
+      if (L.any_plain || L.any_mid || L.start_only)
         APH_LAUNCH((k_ru_accum<T, VX>), L.nsm, st, L.ent_sm, L.b2r_sm, L.start_only);
       break;
     case 5:
