@@ -249,8 +249,9 @@ __device__ __forceinline__ Tile tile_of(const Rec& rc, const SysDev& s, int lb) 
 // ~4 us each while the kernels of a small system take 5 to 10 us: 64^3 63 -> 54
 // us per iteration of a solve, 32^3 46 -> 38.  The operator's and the update's
 // first loads are issued before the sums: 32^3 2.53 -> 2.42 ms, 64^3 2.18 -> 2.11.
-// lean == 2 (more than kLeanCells cells): the operator does not read r, so the update keeps its
-// finalize kernel and the accumulation pass follows it; four launches fall away.
+// lean == 2 (more than kLeanCells cells): the operator does not read r, so the
+// update keeps its finalize kernel and the accumulation pass follows it; four
+// launches fall away.
 // ===========================================================================
 
 // Before the operator: beta from (r, z).  False: the solve ends.

@@ -90,9 +90,9 @@ def launched_name(name, elem, vx):
     kernels k_mg_pre4 / k_mg_post4."""
     if elem == 4 and vx == 4:
         if name == "k_mg_post<T, VX, true, true>":
-            return "k_mg_post4<true, true>"
+            return "k_mg_post4<1024, true, true>"
         if name == "k_mg_pre<T, VX, true>":
-            return "k_mg_pre4<true>"
+            return "k_mg_pre4<1024, true>"
     return name.replace("T, VX", f"{'float' if elem == 4 else 'double'}, {vx}")
 
 

@@ -161,3 +161,26 @@ def test_row_tiles_that_are_no_power_of_two(shape, precision, precond):
     s.close()
     assert info["converged"] == 1
     assert abs(O.true_relres(e, x) / info["true_relres"] - 1) <= 1e-6
+
+
+@pytest.mark.parametrize("precision", [L.MIXED, L.FP64])
+def test_new_systems_in_one_slot(precision):
+    """A time loop's systems, some with a mass term, one after the other in a
+    solver: each as in a solver of its own, bit for bit."""
+    shape = (24, 40, 48)
+
+    def solver():
+        return Poisson(shape, method=L.PCG, precision=precision, resmode=L.RES_REL_TRUE, tol=1e-8,
+                       maxiter=2000, precond=L.PRECOND_MG)
+    loop = solver()
+    for seed, mass in ((1, False), (2, False), (3, True), (4, False), (5, True)):
+        e = _system(shape, seed, mass)
+        loop.set_system(e)
+        x, info = loop.solve(None)
+        own = solver()
+        own.set_system(e)
+        xo, io = own.solve(None)
+        own.close()
+        assert info["converged"] == 1 and info["iter"] == io["iter"]
+        assert np.array_equal(x, xo) and O.true_relres(e, x) <= 1e-8 * (1 + 1e-6)
+    loop.close()
