@@ -93,7 +93,8 @@ def launched_name(name, elem, vx):
             return "k_mg_post4<1024, true, true>"
         if name == "k_mg_pre<T, VX, true>":
             return "k_mg_pre4<1024, true>"
-    return name.replace("T, VX", f"{'float' if elem == 4 else 'double'}, {vx}")
+    threads = ", 1024" if name.startswith(("k_mg_post<", "k_mg_pre<")) else ""
+    return name.replace("T, VX", f"{'float' if elem == 4 else 'double'}, {vx}{threads}")
 
 
 def xh_vectors(solves):
