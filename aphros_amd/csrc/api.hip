@@ -168,8 +168,15 @@ int aphpois_launch_info(aphpois* h, int* stencil_blocks, int* stream_blocks, int
 }
 
 int aphpois_set_resident_wait(aphpois* h, long long ticks) {
+  return aphpois_set_resident_waits(h, ticks, ticks);
+}
+
+int aphpois_set_resident_waits(aphpois* h, long long ticks, long long early_ticks) {
   APH_CHECK_H(h);
-  h->eng.set_pers_wait(ticks);
+  aph::PersWait w;
+  w.gather = ticks;
+  w.early = early_ticks;
+  h->eng.set_pers_wait(w);
   return APHPOIS_OK;
 }
 

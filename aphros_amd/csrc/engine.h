@@ -152,8 +152,8 @@ class Engine {
   // z = M r with the multigrid preconditioner of the resident system (dense
   // host arrays, x fastest); leaves any solve state of the slot as it was.
   int precond_apply(int slot, const double* r, double* z);
-  // Ticks (100 MHz) that a resident launch's workgroups wait for each other
-  void set_pers_wait(long long ticks) { pers_wait_ = ticks; }
+  // How long a resident launch's workgroups wait for each other
+  void set_pers_wait(PersWait w) { pers_wait_ = w; }
   long long bytes() const;
   int nslots() const { return (int)slots_.size(); }
   System* sys(int slot) {
@@ -263,7 +263,7 @@ class Engine {
   bool need_graph_ = false;  // some system of the tables is not resident
   int pers_cu_ = 0;          // compute units resident launches may count on
   bool pers_off_ = false;    // a resident launch failed: iteration kernels only
-  long long pers_wait_ = kPersWait;
+  PersWait pers_wait_;
   hipGraphExec_t gexec_ = nullptr;
   hipGraph_t graph_ = nullptr;
   int graph_k_ = 0;

@@ -231,7 +231,7 @@ int solve_noalloc(const aphpois_desc* d, const double* expr, const double* x0, d
       const unsigned tag = take_tags(d->device, 2u * iters + 2u, &restart);
       if (restart) NA_HIP(launch_fill(slots, kPersSlotBytes / 8, 8, st));
       NA_HIP(launch_pers(method, 0, 0, plan.shape, plan.lds, L.sds, &dh->prec, b2r, plan.nblk, iters,
-                         tag, kPersWait, st));
+                         tag, PersWait(), st));
     }
     for (int i = 0; i < k && !pers; ++i) {
       for (int j = 0; j < iter_kernels(method); ++j) NA_HIP(launch_kernel(method, 0, 1, L, st, j));

@@ -30,6 +30,14 @@ struct PersRec {
   unsigned long long* slots;  // kPersSlotBytes, zeroed once
 };
 
+// Ticks of the 100 MHz counter (negative: none at all) after which a workgroup
+// stops waiting for the others' sums (gather) and a wavefront for its
+// neighbours' before it loads their rows early (early; it then loads them
+// behind the gather).
+struct PersWait {
+  long long gather = 200000000, early = 200000000;
+};
+
 // Plan of a system of method (Method), element type and size on a device of
 // ncu compute units; false: the system is not for a resident launch.
 bool pers_plan(int method, int fp32, int nx, int ny, int nz, int ncu, PersPlan* out);
@@ -38,14 +46,12 @@ bool pers_plan(int method, int fp32, int nx, int ny, int nz, int ncu, PersPlan* 
 // instance: shape and, for PCG, has_m) in one cooperative launch of nblk
 // workgroups with `lds` bytes of dynamic LDS.  recs and b2r (workgroup ->
 // record) are device arrays; tag: the launch's first tag, larger than every
-// tag the slots have seen (a launch uses fewer than 2 * iters + 2); wait:
-// ticks of the 100 MHz counter after which a workgroup stops waiting for the
-// others (kPersWait; negative: at once).  A system whose workgroups did not
-// meet keeps the state it had before the launch and gets pers_fail = 1.
-constexpr long long kPersWait = 200000000;
+// tag the slots have seen (a launch uses fewer than 2 * iters + 2).  A system
+// whose workgroups did not meet keeps the state it had before the launch and
+// gets pers_fail = 1.
 hipError_t launch_pers(int method, int fp32, int has_m, int shape, int lds, const SysDev* sds,
                        const PersRec* recs, const int* b2r, int nblk, int iters, unsigned tag,
-                       long long wait, hipStream_t st);
+                       PersWait wait, hipStream_t st);
 
 // Compute units of a device for pers_plan: 0 if it cannot launch
 // cooperatively.

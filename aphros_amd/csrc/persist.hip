@@ -262,11 +262,14 @@ constexpr int early_halo(int bytes) { return bytes >= 128 ? 0 : (bytes >= 64 ? 2
 
 // The first HR halo values of a thread, loaded while the gather that follows
 // their stores is under way: a neighbour's values in that gather say that its
-// rows are in memory.
+// rows are in memory.  A wavefront that has waited too long for a neighbour
+// loads nothing early; its values are then loaded when they are used, behind
+// the gather, whose result says the same of every neighbour.
 template <typename T, int HR>
 struct EarlyHalo {
   T v[HR > 0 ? HR : 1];
-  int nb;  // slot of the neighbour in y-, y+, z-, z+ (lane % 4)
+  bool late = true;  // v holds nothing (the same in every lane)
+  int nb;            // slot of the neighbour in y-, y+, z-, z+ (lane % 4)
   __device__ EarlyHalo(const PersRec& rc, int lb) {
     const int pz = rc.nblk / rc.py, jy = lb % rc.py, jz = lb / rc.py;
     const int q = threadIdx.x & 3;
@@ -276,15 +279,19 @@ struct EarlyHalo {
                          : (q == 3 ? (jz == pz - 1 ? 0 : jz + 1) : jz);
     nb = (z * rc.py + y) * kPersWords;
   }
-  // waits for the neighbours' values of gather `tag` in `slots` (as long as the
-  // gather itself would), then starts the loads of rows of src
+  // waits for the neighbours' values of gather `tag` in `slots`, then starts the
+  // loads of rows of src
   __device__ __forceinline__ void load(const Box& b, const int2* tab, const T* src,
                                        const u64* slots, unsigned tag, long long wait) {
     if (HR == 0) return;
+    late = false;
     const long long t0 = wall_clock64();
     for (int n = 1;; ++n) {
+      if (wait < 0 || ((n & 255) == 0 && wall_clock64() - t0 > wait)) {
+        late = true;
+        return;
+      }
       if (!__any((unsigned)ld_agent(slots + nb) != tag)) break;
-      if (((n & 255) == 0 && wall_clock64() - t0 > wait) || wait < 0) break;
     }
 #pragma unroll
     for (int k = 0; k < HR; ++k) {
@@ -295,16 +302,17 @@ struct EarlyHalo {
       }
     }
   }
-  // f(h, global index, value, lds offset) of the cells loaded
+  // f(h, global index, value, lds offset) of those cells, behind the gather
+  // that load() ran ahead of
   template <class F>
-  __device__ __forceinline__ void use(const Box& b, const int2* tab, F f) const {
+  __device__ __forceinline__ void use(const Box& b, const int2* tab, const T* src, F f) const {
 #pragma unroll
     for (int k = 0; k < HR; ++k) {
       const int h = (int)threadIdx.x + k * kT;
       if (h < b.nhalo) {
         const int row = b.row_of(h), x = h - row * b.nx;
         const int2 t = tab[row];
-        f(h, t.x + x, v[k], t.y + x);
+        f(h, t.x + x, late ? ld_agent(src + t.x + x) : v[k], t.y + x);
       }
     }
   }
@@ -325,7 +333,7 @@ template <int CC, int ZC, int NR>
 __global__ __launch_bounds__(kT) void k_pers_cg(const SysDev* __restrict__ sds,
                                                 const PersRec* __restrict__ recs,
                                                 const int* __restrict__ b2r, int iters,
-                                                unsigned tag, long long wait) {
+                                                unsigned tag, PersWait wait) {
   extern __shared__ __align__(16) double sp[];
   __shared__ Shared sh;
   const PersRec rc = recs[b2r[blockIdx.x]];
@@ -380,7 +388,7 @@ __global__ __launch_bounds__(kT) void k_pers_cg(const SysDev* __restrict__ sds,
     if (!first) {
       const double* hs = it == 0 ? rg : hg;
       if (it > 0)
-        eh.use(b, tab, [&](int, int, double v, int o) { sp[o] = v + beta * sp[o]; });
+        eh.use(b, tab, hs, [&](int, int, double v, int o) { sp[o] = v + beta * sp[o]; });
       for_halo(b, tab, [&](int gi) { return ld_agent(hs + gi); },
                [&](int, double v, int o) { sp[o] = v + beta * sp[o]; }, it > 0 ? HR : 0);
 #pragma unroll
@@ -424,7 +432,7 @@ __global__ __launch_bounds__(kT) void k_pers_cg(const SysDev* __restrict__ sds,
         }
       }
     }
-    ok = gather<1, 0u>(acc, sl0, rc.nblk, lb, tag + 2 * it, wait, sh, [] {});
+    ok = gather<1, 0u>(acc, sl0, rc.nblk, lb, tag + 2 * it, wait.gather, sh, [] {});
     if (!ok) break;
     const double alpha = rho / (acc[0] + 1e-100);
     double ac2[2] = {0.0, 0.0};
@@ -443,8 +451,8 @@ __global__ __launch_bounds__(kT) void k_pers_cg(const SysDev* __restrict__ sds,
         }
       }
     }
-    ok = gather<2, 2u>(ac2, sl1, rc.nblk, lb, tag + 2 * it + 1, wait, sh,
-                       [&] { eh.load(b, tab, hg, sl1, tag + 2 * it + 1, wait); });
+    ok = gather<2, 2u>(ac2, sl1, rc.nblk, lb, tag + 2 * it + 1, wait.gather, sh,
+                       [&] { eh.load(b, tab, hg, sl1, tag + 2 * it + 1, wait.early); });
     if (!ok) break;
     const double dot_r = ac2[0];
     res = rmode == 1 ? ac2[1] / h3 : sqrt(dot_r / h3);
@@ -494,7 +502,7 @@ template <int CC, int ZC, int NR>
 __global__ __launch_bounds__(kT) void k_pers_jacobi(const SysDev* __restrict__ sds,
                                                     const PersRec* __restrict__ recs,
                                                     const int* __restrict__ b2r, int iters,
-                                                    unsigned tag, long long wait) {
+                                                    unsigned tag, PersWait wait) {
   extern __shared__ __align__(16) double sp[];
   __shared__ Shared sh;
   const PersRec rc = recs[b2r[blockIdx.x]];
@@ -576,8 +584,8 @@ __global__ __launch_bounds__(kT) void k_pers_jacobi(const SysDev* __restrict__ s
     }
     // (the gather's barriers separate these reads of LDS from the writes below)
     u64* const sl = (it & 1) ? sl1 : sl0;
-    ok = gather<1, 1u>(acc, sl, rc.nblk, lb, tag + it, wait, sh,
-                       [&] { eh.load(b, tab, ub, sl, tag + it, wait); });
+    ok = gather<1, 1u>(acc, sl, rc.nblk, lb, tag + it, wait.gather, sh,
+                       [&] { eh.load(b, tab, ub, sl, tag + it, wait.early); });
     if (!ok) break;
     res = acc[0];
     iter += 1;
@@ -585,7 +593,7 @@ __global__ __launch_bounds__(kT) void k_pers_jacobi(const SysDev* __restrict__ s
       conv = res < tol ? 1 : 0;
       done = 1;
     }
-    eh.use(b, tab, [&](int, int, double w, int o) { sp[o] = w; });
+    eh.use(b, tab, ub, [&](int, int, double w, int o) { sp[o] = w; });
     for_halo(b, tab, [&](int gi) { return ld_agent(ub + gi); },
              [&](int, double w, int o) { sp[o] = w; }, HR);
 #pragma unroll
@@ -632,7 +640,7 @@ template <typename T, int CC, int ZC, bool HM, bool KXY>
 __global__ __launch_bounds__(kT) void k_pers_pcg(const SysDev* __restrict__ sds,
                                                  const PersRec* __restrict__ recs,
                                                  const int* __restrict__ b2r, int iters,
-                                                 unsigned tag, long long wait) {
+                                                 unsigned tag, PersWait wait) {
   extern __shared__ __align__(16) double sp[];
   __shared__ Shared sh;
   const PersRec rc = recs[b2r[blockIdx.x]];
@@ -733,7 +741,7 @@ __global__ __launch_bounds__(kT) void k_pers_pcg(const SysDev* __restrict__ sds,
       sp[o] = (double)Sh * (double)pn;
     };
     if (it > 0)
-      eh.use(b, tab, [&](int h, int gi, T rh, int o) { halo_p(h, rh, Sg[gi], o); });
+      eh.use(b, tab, hs, [&](int h, int gi, T rh, int o) { halo_p(h, rh, Sg[gi], o); });
     for_halo(
         b, tab, [&](int gi) { return RS{ld_agent(hs + gi), Sg[gi]}; },
         [&](int h, RS v, int o) { halo_p(h, v.r, v.S, o); }, it > 0 ? HR : 0);
@@ -785,7 +793,7 @@ __global__ __launch_bounds__(kT) void k_pers_pcg(const SysDev* __restrict__ sds,
         }
       }
     }
-    ok = gather<1, 0u>(acc, sl0, rc.nblk, lb, tag + 2 * it, wait, sh, [] {});
+    ok = gather<1, 0u>(acc, sl0, rc.nblk, lb, tag + 2 * it, wait.gather, sh, [] {});
     if (!ok) break;
     const double pq = acc[0];
     fold = fold == 1 ? 2 : 0;
@@ -809,8 +817,8 @@ __global__ __launch_bounds__(kT) void k_pers_pcg(const SysDev* __restrict__ sds,
         }
       }
     }
-    ok = gather<1, 0u>(ac2, sl1, rc.nblk, lb, tag + 2 * it + 1, wait, sh,
-                       [&] { eh.load(b, tab, hg, sl1, tag + 2 * it + 1, wait); });
+    ok = gather<1, 0u>(ac2, sl1, rc.nblk, lb, tag + 2 * it + 1, wait.gather, sh,
+                       [&] { eh.load(b, tab, hg, sl1, tag + 2 * it + 1, wait.early); });
     if (!ok) break;
     const double rn = ac2[0];
     iter += 1;
@@ -930,7 +938,7 @@ namespace {
 
 template <typename K>
 hipError_t coop(K kernel, int nblk, int lds, hipStream_t st, const SysDev* sds,
-                const PersRec* recs, const int* b2r, int iters, unsigned tag, long long wait) {
+                const PersRec* recs, const int* b2r, int iters, unsigned tag, PersWait wait) {
   void* args[] = {(void*)&sds,   (void*)&recs, (void*)&b2r,
                   (void*)&iters, (void*)&tag,  (void*)&wait};
   return hipLaunchCooperativeKernel((const void*)kernel, dim3(nblk), dim3(kT), args,
@@ -941,7 +949,7 @@ hipError_t coop(K kernel, int nblk, int lds, hipStream_t st, const SysDev* sds,
 
 hipError_t launch_pers(int method, int fp32, int has_m, int shape, int lds, const SysDev* sds,
                        const PersRec* recs, const int* b2r, int nblk, int iters, unsigned tag,
-                       long long wait, hipStream_t st) {
+                       PersWait wait, hipStream_t st) {
 #define APH_COOP(...) return coop(__VA_ARGS__, nblk, lds, st, sds, recs, b2r, iters, tag, wait)
   if (method == kConjugate) {
     switch (shape) {

@@ -90,8 +90,9 @@ class Poisson:
         L.check(L.lib().aphpois_launch_info(self.h, C.byref(a), C.byref(b), C.byref(v)))
         return {"stencil_blocks": a.value, "stream_blocks": b.value, "vx": v.value}
 
-    def set_resident_wait(self, ticks):
-        L.check(L.lib().aphpois_set_resident_wait(self.h, ticks))
+    def set_resident_wait(self, ticks, early_ticks=None):
+        early = ticks if early_ticks is None else early_ticks
+        L.check(L.lib().aphpois_set_resident_waits(self.h, ticks, early))
 
     def set_tile(self, lx=0, bz=0, vx=0, sm=0):
         L.check(L.lib().aphpois_set_tile(self.h, lx, bz, vx, sm))

@@ -293,6 +293,9 @@ int aphpois_set_tile(aphpois* h, int lx, int bz, int vx, int sm);
  * set_profiling or set_tile address the iteration kernels.  Negative: they
  * give up at once. */
 int aphpois_set_resident_wait(aphpois* h, long long ticks);
+/* The same with a wait of its own for the loads of neighbouring rows that start
+ * ahead of the sums (early_ticks; once it has passed they follow the sums). */
+int aphpois_set_resident_waits(aphpois* h, long long ticks, long long early_ticks);
 /* Practical HBM bandwidth of a plain streaming copy kernel on `device`:
  * copies `bytes` (two buffers of that size are allocated and freed) `reps`
  * times after one warm-up copy; *gbps = 2 * bytes * reps / time. */

@@ -168,3 +168,33 @@ def test_served_large_and_small_lanes():
     srv.close()
     assert all(r["status"] == 0 and r["last_relres"] <= 1e-8 for r in res)
     assert np.array_equal(res[2]["x"], alone["x"])
+
+
+@pytest.mark.parametrize("shape", [(33, 35, 37), (52, 45, 60), (93, 75, 101), (121, 117, 127)])
+@pytest.mark.parametrize("method", [L.CONJUGATE, L.JACOBI, L.PCG])
+def test_early_row_loads_that_lapse(method, shape):
+    """The wait for the neighbours' rows gives up at once while the workgroups do
+    meet: the rows are then loaded behind the sums, so the solve is the same, bit
+    for bit (JACOBI: the oracle's)."""
+    E = _system(shape, 8)
+    got = []
+    for early in (None, -1):
+        if method == L.JACOBI:
+            kw = dict(resmode=L.RES_L2, tol=0.0, maxiter=11)
+        elif method == L.CONJUGATE:
+            kw = dict(resmode=L.RES_L2, tol=1e-6, maxiter=2000)
+        else:
+            kw = dict(resmode=L.RES_REL_TRUE, tol=1e-9, maxiter=2000)
+        s = Poisson(shape, method=method, miniter=0, h3=1.0, **kw)
+        s.set_system(E)
+        if early is not None:
+            s.set_resident_wait(200000000, early)
+        got.append(s.solve(None))
+        s.close()
+    (x, i), (y, j) = got
+    assert i["iter"] == j["iter"] and np.array_equal(x, y)
+    if method == L.JACOBI:
+        xo, ito, _, _ = O.jacobi(E, tol=0.0, miniter=0, maxiter=11)
+        assert ito == j["iter"] and np.array_equal(y, xo)
+    else:
+        assert j["converged"] == 1
