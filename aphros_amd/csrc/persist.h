@@ -11,8 +11,9 @@ constexpr int kPersThreads = 512;
 constexpr int kPersMaxBlocks = 256;  // workgroups of one launch (slots per phase)
 constexpr int kPersPhases = 2;
 constexpr int kPersWords = 4;        // 64-bit words of one slot (two tagged doubles)
-// slots of one system: phases x workgroups x words
-constexpr long long kPersSlotBytes = 8LL * kPersPhases * kPersMaxBlocks * kPersWords;
+// slots of one system: phases x workgroups x words, and the word in which a
+// launch is kept or given up
+constexpr long long kPersSlotBytes = 8LL * kPersPhases * kPersMaxBlocks * kPersWords + 256;
 
 // How one system runs in a resident launch (a property of the system and the
 // device alone): boxes of by x bz whole rows, py x pz of them, one workgroup

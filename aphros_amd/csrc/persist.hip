@@ -35,10 +35,13 @@
 //
 // The launch is cooperative (all workgroups resident).  Every wait ends all the
 // same: a workgroup that has waited too long (another process's resident
-// launch may hold half of the device and wait for the other half) leaves the
-// kernel.  A launch writes a system's state only at its end, so the state is
-// then still the one before the launch, and the host goes on with the
-// iteration kernels.
+// launch may hold half of the device and wait for the other half) asks for the
+// launch to be given up.  Whether a system's launch counts is decided once, in
+// one word that the first workgroup to ask sets (decide()): one that has all
+// sums of the last gather asks to keep the launch, one whose wait has passed to
+// give it up, and all follow that word.  No workgroup writes any state before a
+// launch is kept; a given-up launch leaves the state as it was, and the host
+// goes on with the iteration kernels.
 #include "persist.h"
 
 #include "kernels.h"
@@ -70,48 +73,57 @@ __device__ __forceinline__ void opaque(T& v) {
   asm volatile("" : "+v"(v));
 }
 
+constexpr long long kPersAgain = 200000000;  // ticks; values known to be there
 constexpr int kGroups = kPersMaxBlocks / 64;  // slot groups, one wave reads each
 
 struct Shared {
   double red[2][kWaves];
   double out[2][kGroups];
   int bad[kGroups];
+  int flag;  // what one thread read for all
 };
 
-// All-gather reduction of NV values (sums, or maxima where flagged in MaxMask)
-// over the nblk workgroups of a system; the result is valid in every thread of
-// every workgroup, summed in workgroup order.  Every global store this thread
-// issued before the call is complete before the workgroup's values appear.
-// meanwhile(): run by every wavefront once the workgroup's values are on their
-// way, before it waits for the others'.
-// Returns false if some workgroup's values did not appear in time.
-template <int NV, unsigned MaxMask, class F>
-__device__ __forceinline__ bool gather(double (&v)[NV], u64* slots, int nblk, int me,
-                                       unsigned tag, long long wait, Shared& sh,
-                                       F meanwhile) {
-  wave_reduce<NV, MaxMask>(v);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) {
-#pragma unroll
-    for (int k = 0; k < NV; ++k) sh.red[k][wave] = v[k];
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  const int ngrp = (nblk + 63) >> 6;
-  if (wave == 0 && lane < 2 * NV) {
-    // lane 2 k publishes the low half of value k, lane 2 k + 1 the high half
-    const int k = NV > 1 ? lane >> 1 : 0;
-    double t = sh.red[k][0];
-#pragma unroll
-    for (int w = 1; w < kWaves; ++w) {
-      const double x = sh.red[k][w];
-      t = ((MaxMask >> k) & 1u) ? fmax(t, x) : t + x;
+// Keeps (keep) a system's launch, whose first tag is `launch`, or gives it up:
+// true if it is kept.  The first workgroup's answer holds for all.
+__device__ __forceinline__ bool decide(u64* word, unsigned launch, bool keep, Shared& sh) {
+  if (threadIdx.x == 0) {
+    u64 w = ld_agent(word);
+    // (other launches' words have other tags; this one's is never replaced, so
+    // a failed exchange has found it)
+    if ((unsigned)(w >> 32) != launch) {
+      const u64 mine = ((u64)launch << 32) | (keep ? 1u : 0u);
+      if (__hip_atomic_compare_exchange_strong(word, &w, mine, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT))
+        w = mine;
     }
-    const u64 b = (u64)__double_as_longlong(t);
-    st_agent(slots + (long long)me * kPersWords + lane,
-             ((lane & 1) ? (b & 0xffffffff00000000ull) : (b << 32)) | tag);
+    sh.flag = (int)(w & 1u);
   }
-  meanwhile();
+  __syncthreads();
+  const bool kept = sh.flag != 0;
+  __syncthreads();
+  return kept;
+}
+
+__device__ __forceinline__ u64* pers_word(const PersRec& rc) {
+  return rc.slots + kPersPhases * kPersMaxBlocks * kPersWords;
+}
+
+// Whether a system takes no part in this launch, read once for the workgroup
+// (one that gives up stores pers_fail while others may just start).
+__device__ __forceinline__ bool passed_by(bool skip, Shared& sh) {
+  if (threadIdx.x == 0) sh.flag = skip ? 1 : 0;
+  __syncthreads();
+  const bool out = sh.flag != 0;
+  __syncthreads();
+  return out;
+}
+
+// The second half of gather(): waits for the values of all workgroups.
+template <int NV, unsigned MaxMask>
+__device__ __forceinline__ bool collect(double (&v)[NV], const u64* slots, int nblk, unsigned tag,
+                                        long long wait, Shared& sh) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int ngrp = (nblk + 63) >> 6;
   if (wave < ngrp) {
     // wave w reads the slots 64 w .. 64 w + 63, one per lane
     const int i = lane + 64 * wave;
@@ -158,6 +170,42 @@ __device__ __forceinline__ bool gather(double (&v)[NV], u64* slots, int nblk, in
       v[k] = ((MaxMask >> k) & 1u) ? fmax(v[k], sh.out[k][w]) : v[k] + sh.out[k][w];
   }
   return ok;
+}
+
+// All-gather reduction of NV values (sums, or maxima where flagged in MaxMask)
+// over the nblk workgroups of a system; the result is valid in every thread of
+// every workgroup, summed in workgroup order.  Every global store this thread
+// issued before the call is complete before the workgroup's values appear.
+// meanwhile(): run by every wavefront once the workgroup's values are on their
+// way, before it waits for the others'.
+// Returns false if some workgroup's values did not appear in time.
+template <int NV, unsigned MaxMask, class F>
+__device__ __forceinline__ bool gather(double (&v)[NV], u64* slots, int nblk, int me,
+                                       unsigned tag, long long wait, Shared& sh,
+                                       F meanwhile) {
+  wave_reduce<NV, MaxMask>(v);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (lane == 0) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) sh.red[k][wave] = v[k];
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (wave == 0 && lane < 2 * NV) {
+    // lane 2 k publishes the low half of value k, lane 2 k + 1 the high half
+    const int k = NV > 1 ? lane >> 1 : 0;
+    double t = sh.red[k][0];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) {
+      const double x = sh.red[k][w];
+      t = ((MaxMask >> k) & 1u) ? fmax(t, x) : t + x;
+    }
+    const u64 b = (u64)__double_as_longlong(t);
+    st_agent(slots + (long long)me * kPersWords + lane,
+             ((lane & 1) ? (b & 0xffffffff00000000ull) : (b << 32)) | tag);
+  }
+  meanwhile();
+  return collect<NV, MaxMask>(v, slots, nblk, tag, wait, sh);
 }
 
 // The box of a workgroup and its place in LDS: rows of nx values, (bz + 2) x
@@ -263,13 +311,13 @@ constexpr int early_halo(int bytes) { return bytes >= 128 ? 0 : (bytes >= 64 ? 2
 // The first HR halo values of a thread, loaded while the gather that follows
 // their stores is under way: a neighbour's values in that gather say that its
 // rows are in memory.  A wavefront that has waited too long for a neighbour
-// loads nothing early; its values are then loaded when they are used, behind
-// the gather, whose result says the same of every neighbour.
+// (late) loads them again when they are used, behind the gather, whose result
+// says the same of every neighbour.
 template <typename T, int HR>
 struct EarlyHalo {
   T v[HR > 0 ? HR : 1];
-  bool late = true;  // v holds nothing (the same in every lane)
-  int nb;            // slot of the neighbour in y-, y+, z-, z+ (lane % 4)
+  bool late = false;  // (the same in every lane)
+  int nb;             // slot of the neighbour in y-, y+, z-, z+ (lane % 4)
   __device__ EarlyHalo(const PersRec& rc, int lb) {
     const int pz = rc.nblk / rc.py, jy = lb % rc.py, jz = lb / rc.py;
     const int q = threadIdx.x & 3;
@@ -279,20 +327,7 @@ struct EarlyHalo {
                          : (q == 3 ? (jz == pz - 1 ? 0 : jz + 1) : jz);
     nb = (z * rc.py + y) * kPersWords;
   }
-  // waits for the neighbours' values of gather `tag` in `slots`, then starts the
-  // loads of rows of src
-  __device__ __forceinline__ void load(const Box& b, const int2* tab, const T* src,
-                                       const u64* slots, unsigned tag, long long wait) {
-    if (HR == 0) return;
-    late = false;
-    const long long t0 = wall_clock64();
-    for (int n = 1;; ++n) {
-      if (wait < 0 || ((n & 255) == 0 && wall_clock64() - t0 > wait)) {
-        late = true;
-        return;
-      }
-      if (!__any((unsigned)ld_agent(slots + nb) != tag)) break;
-    }
+  __device__ __forceinline__ void rows(const Box& b, const int2* tab, const T* src) {
 #pragma unroll
     for (int k = 0; k < HR; ++k) {
       const int h = (int)threadIdx.x + k * kT;
@@ -302,17 +337,35 @@ struct EarlyHalo {
       }
     }
   }
-  // f(h, global index, value, lds offset) of those cells, behind the gather
+  // waits for the neighbours' values of gather `tag` in `slots`, then starts the
+  // loads of rows of src
+  __device__ __forceinline__ void load(const Box& b, const int2* tab, const T* src,
+                                       const u64* slots, unsigned tag, long long wait) {
+    if (HR == 0) return;
+    late = wait < 0;
+    const long long t0 = wall_clock64();
+    for (int n = 1;; ++n) {
+      if (!__any((unsigned)ld_agent(slots + nb) != tag)) break;
+      if (((n & 255) == 0 && wall_clock64() - t0 > wait) || wait < 0) {
+        late = true;
+        break;
+      }
+    }
+    rows(b, tab, src);
+  }
+  // f(h, global index, value, lds offset) of the cells loaded, behind the gather
   // that load() ran ahead of
   template <class F>
-  __device__ __forceinline__ void use(const Box& b, const int2* tab, const T* src, F f) const {
+  __device__ __forceinline__ void use(const Box& b, const int2* tab, const T* src, F f) {
+    if (HR == 0) return;
+    if (late) rows(b, tab, src);
 #pragma unroll
     for (int k = 0; k < HR; ++k) {
       const int h = (int)threadIdx.x + k * kT;
       if (h < b.nhalo) {
         const int row = b.row_of(h), x = h - row * b.nx;
         const int2 t = tab[row];
-        f(h, t.x + x, late ? ld_agent(src + t.x + x) : v[k], t.y + x);
+        f(h, t.x + x, v[k], t.y + x);
       }
     }
   }
@@ -339,7 +392,7 @@ __global__ __launch_bounds__(kT) void k_pers_cg(const SysDev* __restrict__ sds,
   const PersRec rc = recs[b2r[blockIdx.x]];
   const SysDev& s = sds[rc.sys];
   Scalars* sc = s.sc;
-  if (sc->done || sc->pers_fail) return;
+  if (passed_by(sc->done || sc->pers_fail, sh)) return;
   const int lb = (int)blockIdx.x - rc.blk0;
   const Box b(s, rc, lb);
   const int nx = b.nx, zs = b.ly * nx, pl = nx * b.ny, bz = b.bz;
@@ -379,7 +432,21 @@ __global__ __launch_bounds__(kT) void k_pers_cg(const SysDev* __restrict__ sds,
   constexpr int HR = early_halo(8 * CC * ZC);
   EarlyHalo<double, HR> eh(rc, lb);
   bool ok = true;
-  for (int it = 0; it < iters && !done; ++it) {
+  // the iteration's end, from the sum of r^2 and the largest |r|
+  auto step = [&](const double (&v)[2]) {
+    const double dot_r = v[0];
+    res = rmode == 1 ? v[1] / h3 : sqrt(dot_r / h3);
+    iter += 1;
+    beta = dot_r / (rho + 1e-100);
+    rho = dot_r;
+    first = 0;
+    if (iter >= miniter && (iter > maxiter || res < tol)) {
+      conv = res < tol ? 1 : 0;
+      done = 1;
+    }
+  };
+  int it = 0;
+  for (; it < iters && !done; ++it) {
 #pragma unroll
     for (int c = 0; c < CC; ++c) {
       opaque(d[c]);
@@ -454,20 +521,17 @@ __global__ __launch_bounds__(kT) void k_pers_cg(const SysDev* __restrict__ sds,
     ok = gather<2, 2u>(ac2, sl1, rc.nblk, lb, tag + 2 * it + 1, wait.gather, sh,
                        [&] { eh.load(b, tab, hg, sl1, tag + 2 * it + 1, wait.early); });
     if (!ok) break;
-    const double dot_r = ac2[0];
-    res = rmode == 1 ? ac2[1] / h3 : sqrt(dot_r / h3);
-    iter += 1;
-    beta = dot_r / (rho + 1e-100);
-    rho = dot_r;
-    first = 0;
-    if (iter >= miniter && (iter > maxiter || res < tol)) {
-      conv = res < tol ? 1 : 0;
-      done = 1;
-    }
+    step(ac2);
   }
-  if (!ok) {
+  if (!decide(pers_word(rc), tag, ok, sh)) {
     if (threadIdx.x == 0) st_agent(&sc->pers_fail, 1);
     return;
+  }
+  if (!ok) {
+    // kept by a workgroup that found this gather, the last, complete
+    double v[2];
+    collect<2, 2u>(v, sl1, rc.nblk, tag + 2 * it + 1, kPersAgain, sh);
+    step(v);
   }
 #pragma unroll
   for (int c = 0; c < CC; ++c) {
@@ -508,7 +572,7 @@ __global__ __launch_bounds__(kT) void k_pers_jacobi(const SysDev* __restrict__ s
   const PersRec rc = recs[b2r[blockIdx.x]];
   const SysDev& s = sds[rc.sys];
   Scalars* sc = s.sc;
-  if (sc->done || sc->pers_fail) return;
+  if (passed_by(sc->done || sc->pers_fail, sh)) return;
   const int lb = (int)blockIdx.x - rc.blk0;
   const Box b(s, rc, lb);
   const int nx = b.nx, zs = b.ly * nx, pl = nx * b.ny, bz = b.bz;
@@ -543,8 +607,18 @@ __global__ __launch_bounds__(kT) void k_pers_jacobi(const SysDev* __restrict__ s
   constexpr int HR = early_halo(8 * CC * ZC);
   EarlyHalo<double, HR> eh(rc, lb);
   bool ok = true;
+  // the sweep's end, from its largest change
+  auto step = [&](const double (&v)[1]) {
+    res = v[0];
+    iter += 1;
+    if (iter >= miniter && (iter > maxiter || res < tol)) {
+      conv = res < tol ? 1 : 0;
+      done = 1;
+    }
+  };
   __syncthreads();
-  for (int it = 0; it < iters && !done; ++it) {
+  int it = 0;
+  for (; it < iters && !done; ++it) {
     double* const ub = (double*)s.halo[it & 1];
 #pragma unroll
     for (int c = 0; c < CC; ++c) {
@@ -587,12 +661,7 @@ __global__ __launch_bounds__(kT) void k_pers_jacobi(const SysDev* __restrict__ s
     ok = gather<1, 1u>(acc, sl, rc.nblk, lb, tag + it, wait.gather, sh,
                        [&] { eh.load(b, tab, ub, sl, tag + it, wait.early); });
     if (!ok) break;
-    res = acc[0];
-    iter += 1;
-    if (iter >= miniter && (iter > maxiter || res < tol)) {
-      conv = res < tol ? 1 : 0;
-      done = 1;
-    }
+    step(acc);
     eh.use(b, tab, ub, [&](int, int, double w, int o) { sp[o] = w; });
     for_halo(b, tab, [&](int gi) { return ld_agent(ub + gi); },
              [&](int, double w, int o) { sp[o] = w; }, HR);
@@ -605,9 +674,15 @@ __global__ __launch_bounds__(kT) void k_pers_jacobi(const SysDev* __restrict__ s
     }
     __syncthreads();
   }
-  if (!ok) {
+  if (!decide(pers_word(rc), tag, ok, sh)) {
     if (threadIdx.x == 0) st_agent(&sc->pers_fail, 1);
     return;
+  }
+  if (!ok) {
+    // kept by a workgroup that found this gather, the last, complete
+    double v[1];
+    collect<1, 1u>(v, (it & 1) ? sl1 : sl0, rc.nblk, tag + it, kPersAgain, sh);
+    step(v);
   }
 #pragma unroll
   for (int c = 0; c < CC; ++c) {
@@ -646,7 +721,7 @@ __global__ __launch_bounds__(kT) void k_pers_pcg(const SysDev* __restrict__ sds,
   const PersRec rc = recs[b2r[blockIdx.x]];
   const SysDev& s = sds[rc.sys];
   Scalars* sc = s.sc;
-  if (sc->done || sc->ru || sc->pers_fail) return;
+  if (passed_by(sc->done || sc->ru || sc->pers_fail, sh)) return;
   const int lb = (int)blockIdx.x - rc.blk0;
   const Box b(s, rc, lb);
   const int nx = b.nx, ny = b.ny, zs = b.ly * nx, pl = nx * b.ny, bz = b.bz;
@@ -713,7 +788,14 @@ __global__ __launch_bounds__(kT) void k_pers_pcg(const SysDev* __restrict__ sds,
   struct RS {
     T r, S;
   };
-  for (int it = 0; it < iters && !done && !ru; ++it) {
+  // (r, r) says that a reliable update is due
+  auto due = [&](double rn) {
+    const double est = gamma * sqrt(rn);
+    return !isfinite(rn) || sqrt(rn) < delta * sqrt(rmax2) || est <= 0.9 * tol || iter > maxiter;
+  };
+  int it = 0, half = 0;  // half: the iteration's gathers passed
+  for (; it < iters && !done && !ru; ++it) {
+    half = 0;
 #pragma unroll
     for (int c = 0; c < CC; ++c) {
       opaque(d[c]);
@@ -803,6 +885,7 @@ __global__ __launch_bounds__(kT) void k_pers_pcg(const SysDev* __restrict__ sds,
       break;
     }
     alpha = rho / pq;
+    half = 1;
     double ac2[1] = {0.0};
 #pragma unroll
     for (int c = 0; c < CC; ++c) {
@@ -822,10 +905,7 @@ __global__ __launch_bounds__(kT) void k_pers_pcg(const SysDev* __restrict__ sds,
     if (!ok) break;
     const double rn = ac2[0];
     iter += 1;
-    const double est = gamma * sqrt(rn);
-    const bool trig = !isfinite(rn) || sqrt(rn) < delta * sqrt(rmax2) || est <= 0.9 * tol ||
-                      iter > maxiter;
-    if (trig) {
+    if (due(rn)) {
       ru = 1;
       rho_pend = rn;
     } else {
@@ -833,9 +913,30 @@ __global__ __launch_bounds__(kT) void k_pers_pcg(const SysDev* __restrict__ sds,
       rho = rn;
     }
   }
-  if (!ok) {
+  if (!decide(pers_word(rc), tag, ok, sh)) {
     if (threadIdx.x == 0) st_agent(&sc->pers_fail, 1);
     return;
+  }
+  if (!ok) {
+    // kept by a workgroup that found this gather, the last, complete: the second
+    // of an iteration, or the first of one whose operator ends the solve
+    double v[1];
+    collect<1, 0u>(v, half ? sl1 : sl0, rc.nblk, tag + 2 * it + half, kPersAgain, sh);
+    const double rn = v[0];
+    if (!half) {
+      fold = fold == 1 ? 2 : 0;
+      status = 6;
+      done = 1;
+    } else {
+      iter += 1;
+      if (due(rn)) {
+        ru = 1;
+        rho_pend = rn;
+      } else {
+        beta = rn / rho;
+        rho = rn;
+      }
+    }
   }
 #pragma unroll
   for (int c = 0; c < CC; ++c) {

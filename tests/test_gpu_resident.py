@@ -198,3 +198,31 @@ def test_early_row_loads_that_lapse(method, shape):
         assert ito == j["iter"] and np.array_equal(y, xo)
     else:
         assert j["converged"] == 1
+
+
+@pytest.mark.parametrize("shape", [(33, 35, 37), (93, 75, 101)])
+@pytest.mark.parametrize("method", [L.CONJUGATE, L.JACOBI, L.PCG])
+def test_wait_that_lapses_in_the_last_gather(method, shape):
+    """One iteration, whose last gather some workgroups may find complete while
+    others give up at once: the launch counts for all of them or for none, so
+    every solve is that of the resident or that of the iteration kernels, bit for
+    bit (JACOBI: the oracle's)."""
+    E = _system(shape, 9)
+    kw = dict(resmode=L.RES_REL_TRUE, tol=1e-14) if method == L.PCG else \
+        dict(resmode=L.RES_L2, tol=0.0)
+
+    def solve(setup):
+        s = Poisson(shape, method=method, miniter=0, maxiter=0, h3=1.0, **kw)
+        s.set_system(E)
+        setup(s)
+        x, info = s.solve(None)
+        s.close()
+        assert info["iter"] == 1 and info["converged"] == 0
+        return x
+    whole = [solve(lambda s: None), solve(lambda s: s.set_profiling(True))]
+    for _ in range(12):
+        x = solve(lambda s: s.set_resident_wait(-1))
+        assert any(np.array_equal(x, w) for w in whole)
+    if method == L.JACOBI:
+        xo, ito, _, _ = O.jacobi(E, tol=0.0, miniter=0, maxiter=0)
+        assert ito == 1 and np.array_equal(x, xo)
