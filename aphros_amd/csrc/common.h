@@ -47,6 +47,9 @@ struct Scalars {
   // what the CG operator of a lean system (SysDev::lean) leaves for its update,
   // and rz is (r, z) itself rather than a sum over its partials
   int cur_next, iter_next, xf_next, rz_ok;
+  int end;         // lean systems: the solve ends, as one workgroup of a kernel
+                   // has found whose others may still read `done`; the cycle's
+                   // bottom kernel sets that
   int zero_start;  // PCG: the start's x64 is zero-filled (the start's
                    // residual is b, with no accumulation pass); cleared by it
 };

@@ -242,7 +242,9 @@ __device__ __forceinline__ Tile tile_of(const Rec& rc, const SysDev& s, int lb) 
 // Lean systems (SysDev::lean: multigrid of two or more levels).  The kernel
 // after a reducing one sums its partials itself, every workgroup the same way,
 // and workgroup 0 stores what the iteration keeps; no field is stored by a
-// kernel whose other workgroups still read it.  The operator also forms (r, r),
+// kernel whose other workgroups still need the value before (hence `end` beside
+// `done`: a workgroup of which only some wavefronts see `done` would sum up
+// what the others never wrote).  The operator also forms (r, r),
 // (r, q) and (q, q), so the update knows |r - alpha q|^2, and with it whether a
 // reliable update follows, before it touches r.  Six of an iteration's launches
 // fall away (four finalize kernels, an accumulation pass, (r, z)), which cost
@@ -254,24 +256,19 @@ __device__ __forceinline__ Tile tile_of(const Rec& rc, const SysDev& s, int lb) 
 // launches fall away.
 // ===========================================================================
 
-// Before the operator: beta from (r, z).  False: the solve ends.
-__device__ __forceinline__ bool lean_beta(const SysDev& s, Scalars* sc, int lb, double& beta) {
+// Before the operator: beta from (r, z) (not finite: the update ends the solve).
+__device__ __forceinline__ double lean_beta(const SysDev& s, Scalars* sc, int lb) {
   const bool ok = sc->rz_ok;
   double acc[1] = {sc->rz};
   if (!ok) reduce_partials<1, 0u>(acc, s.ppc, s.nblk_pc);
   const double rz = acc[0];
-  beta = sc->first ? 0.0 : rz / sc->rho;
   if (lb == 0 && threadIdx.x == 0) {
-    if (!isfinite(rz)) {
-      sc->status = 6;
-      sc->done = 1;
-    }
     if (!ok) sc->rz = rz;
     sc->cur_next = sc->cur ^ 1;
     sc->iter_next = sc->iter + 1;
     sc->xf_next = sc->xh_fold == 1 ? 2 : 0;
   }
-  return isfinite(rz);
+  return sc->first ? 0.0 : rz / sc->rho;
 }
 
 // Before the update: alpha, and whether a reliable update follows (1), not (0),
@@ -279,8 +276,8 @@ __device__ __forceinline__ bool lean_beta(const SysDev& s, Scalars* sc, int lb, 
 __device__ __forceinline__ int lean_step(const SysDev& s, Scalars* sc, int lb, double& alpha) {
   double d[4];  // (p, q), (r, r), (r, q), (q, q)
   reduce_partials<4, 0u>(d, s.partials, s.nblk_st);
-  const bool bad = !(d[0] != 0.0) || !isfinite(d[0]);
   const double rz = sc->rz;
+  const bool bad = !(d[0] != 0.0) || !isfinite(d[0]) || !isfinite(rz);
   const int iter = sc->iter_next;
   alpha = rz / d[0];
   const double rn = d[1] - alpha * (2.0 * d[2] - alpha * d[3]);
@@ -290,7 +287,8 @@ __device__ __forceinline__ int lean_step(const SysDev& s, Scalars* sc, int lb, d
   if (lb == 0 && threadIdx.x == 0) {
     if (bad) {
       sc->status = 6;
-      sc->done = 1;
+      sc->end = 1;
+      sc->ru = 0;
     } else {
       sc->alpha = alpha;
       sc->cur = sc->cur_next;
@@ -311,13 +309,14 @@ __device__ __forceinline__ int lean_step(const SysDev& s, Scalars* sc, int lb, d
 __device__ __forceinline__ bool mid_step(const SysDev& s, Scalars* sc, int lb, double& alpha) {
   double pq[1];
   reduce_partials<1, 0u>(pq, s.partials, s.nblk_st);
-  const bool bad = !(pq[0] != 0.0) || !isfinite(pq[0]);
   const double rz = sc->rz;
+  const bool bad = !(pq[0] != 0.0) || !isfinite(pq[0]) || !isfinite(rz);
   alpha = rz / pq[0];
   if (lb == 0 && threadIdx.x == 0) {
     if (bad) {
       sc->status = 6;
-      sc->done = 1;
+      sc->end = 1;
+      sc->ru = 0;
     } else {
       sc->alpha = alpha;
       sc->cur = sc->cur_next;
@@ -345,8 +344,10 @@ __device__ __forceinline__ double lean_mean(const SysDev& s, Scalars* sc, int lb
 }
 
 // What a reliable update's true residual (acc: |r^|^2, |r|^2, max |r|) says:
-// true if the solve ends.  `store`: by one thread of one workgroup.
-__device__ __forceinline__ bool ru_verdict(Scalars* sc, const double (&acc)[3], bool store) {
+// true if the solve ends (then *end is set).  `store`: by one thread of one
+// workgroup.
+__device__ __forceinline__ bool ru_verdict(Scalars* sc, const double (&acc)[3], bool store,
+                                           int* end) {
   const double rh2 = acc[0], rr = acc[1], mx = acc[2];
   const double relres = sc->bnorm2 > 0 ? sqrt(rr / sc->bnorm2) : sqrt(rr);
   const double l2 = sqrt(rr / sc->h3), lmax = mx / sc->h3;
@@ -364,10 +365,10 @@ __device__ __forceinline__ bool ru_verdict(Scalars* sc, const double (&acc)[3], 
     sc->nru += 1;
     if (bad) {
       sc->status = 6;
-      sc->done = 1;
+      *end = 1;
     } else if (stop) {
       sc->converged = conv ? 1 : 0;
-      sc->done = 1;
+      *end = 1;
     } else {
       if (!sc->pc) {
         sc->beta = sc->first ? 0.0 : rh2 / sc->rho;
@@ -387,7 +388,7 @@ template <int NT>
 __device__ __forceinline__ bool lean_verdict(const SysDev& s, Scalars* sc, int lb) {
   double acc[3];
   reduce_partials<3, 4u, NT>(acc, s.pres, s.nblk_ru);
-  return ru_verdict(sc, acc, lb == 0 && threadIdx.x == 0);
+  return ru_verdict(sc, acc, lb == 0 && threadIdx.x == 0, &sc->end);
 }
 
 // x64 = (x64 - mp) + S * (x^ + fa p) on cells [beg, end) (stale: x^ counts as
@@ -537,7 +538,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
       zv1 = ldv<T, VX>(r, i1);
       pv1 = ldv<T, VX>(pin, i1);
     }
-    if (lean && !lean_beta(s, sc, lb, beta)) return;
+    if (lean) beta = lean_beta(s, sc, lb);
   }
   if (t.active) {
     if constexpr (SC) {
@@ -748,7 +749,8 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update(const Ent* __restrict__ e
 __global__ __launch_bounds__(kBlock) void k_fin_pcg_update(const SysDev* __restrict__ sds) {
   const SysDev& s = sds[blockIdx.x];
   Scalars* sc = s.sc;
-  if (s.lean == 1 || sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
+  // ru: a reliable update is pending
+  if (s.lean == 1 || sc->done || sc->end || sc->ru || s.pers) return;
   double acc[1];
   reduce_partials<1, 0u>(acc, s.lean ? s.pres : s.partials, s.nblk_sm);
   if (threadIdx.x == 0) {
@@ -1058,7 +1060,7 @@ __global__ __launch_bounds__(kBlock) void k_fin_ru_resid(const SysDev* __restric
   double acc[3];
   reduce_partials<3, 4u>(acc, s.pres, s.nblk_ru);
   if (threadIdx.x == 0) {
-    ru_verdict(sc, acc, true);
+    ru_verdict(sc, acc, true, &sc->done);
     sc->ru = 0;
   }
 }
@@ -2957,6 +2959,10 @@ __global__ __launch_bounds__(kBottomThreads) void k_mg_bottom(const SysDev* __re
   if (s.nlev <= 0 || s.sc->done || s.mg_lb != l0) return;
   if (wl >= 0 && wl >= s.mg_w) return;
   if (so && !s.sc->first) return;
+  if (s.sc->end) {
+    if (threadIdx.x == 0) s.sc->done = 1;
+    return;
+  }
   constexpr int NV = sizeof(T) == 4 ? 8 : 4;
   const int top = s.nlev - 1;
   const int tid = threadIdx.x;

@@ -184,3 +184,32 @@ def test_new_systems_in_one_slot(precision):
         assert info["converged"] == 1 and info["iter"] == io["iter"]
         assert np.array_equal(x, xo) and O.true_relres(e, x) <= 1e-8 * (1 + 1e-6)
     loop.close()
+
+
+@pytest.mark.parametrize("precision", [L.MIXED, L.FP64])
+@pytest.mark.parametrize("shape", [(16, 24, 20), (64, 96, 80), (160, 256, 256)])
+def test_breakdown_ends_the_solve(shape, precision):
+    """b = 0 and more iterations asked for: (p, q) = 0 in the first, which ends the
+    solve and leaves x as it was, at sizes of either form of the reductions; the
+    solver then solves as a new one, bit for bit."""
+    e = _system(shape, 7, False)
+
+    def solver():
+        s = Poisson(shape, method=L.PCG, precision=precision, resmode=L.RES_REL_TRUE, tol=1e-8,
+                    miniter=3, maxiter=2000, precond=L.PRECOND_MG)
+        s.set_system(e)
+        return s
+    s = solver()
+    for _ in range(3):
+        s.set_rhs(np.zeros(shape))
+        x, info = s.solve(None)
+        assert info["status"] == L.ENUMERIC and info["iter"] == 0 and info["converged"] == 0
+        assert not x.any()
+        s.set_rhs(e[..., 7])
+        x, info = s.solve(None)
+        assert info["status"] == 0 and info["converged"] == 1
+    s.close()
+    own = solver()
+    xo, io = own.solve(None)
+    own.close()
+    assert info["iter"] == io["iter"] and np.array_equal(x, xo)
