@@ -263,6 +263,7 @@ class Engine {
   bool need_graph_ = false;  // some system of the tables is not resident
   int pers_cu_ = 0;          // compute units resident launches may count on
   bool pers_off_ = false;    // a resident launch failed: iteration kernels only
+  bool pers_refused_ = false;  // the runtime refused one since the last look
   PersWait pers_wait_;
   hipGraphExec_t gexec_ = nullptr;
   hipGraph_t graph_ = nullptr;

@@ -955,9 +955,12 @@ bool Engine::use_pers(const System& s) const {
          tuning_.sm == 0 && s.tune_lx == 0 && s.tune_bz == 0;
 }
 
-// Up to `iters` more iterations of every resident system of the tables.
+// Up to `iters` more iterations of every resident system of the tables.  A
+// launch that the runtime refuses (compute units held back from the process or
+// the stream) is left to pers_fallback().
 int Engine::advance_pers(int iters) {
   for (const PersGroup& g : pers_groups_) {
+    if (pers_refused_) break;
     if (pers_tag_ > 0xffffffffu - 2u * (unsigned)iters - 4u) {
       // the tags start over: no slot may hold one of them
       for (auto& s : slots_) {
@@ -965,18 +968,22 @@ int Engine::advance_pers(int iters) {
       }
       pers_tag_ = 1;
     }
-    APH_HIP(launch_pers(method_, fp32_, g.has_m, g.shape, g.lds, L_.sds, g.recs, g.b2r, g.nblk,
-                        iters, pers_tag_, pers_wait_, st_));
+    if (launch_pers(method_, fp32_, g.has_m, g.shape, g.lds, L_.sds, g.recs, g.b2r, g.nblk, iters,
+                    pers_tag_, pers_wait_, st_) != hipSuccess) {
+      (void)hipGetLastError();
+      pers_refused_ = true;
+    }
     pers_tag_ += 2u * (unsigned)iters + 2u;
   }
   return APHPOIS_OK;
 }
 
-// After the scalars were read: if some resident launch gave up (its systems
-// then hold the state before it), the engine goes on with the iteration
-// kernels, from here on for good.
+// After the scalars were read: if some resident launch was refused or gave up
+// (its systems then hold the state before it), the engine goes on with the
+// iteration kernels, from here on for good.
 int Engine::pers_fallback(bool* failed) {
-  *failed = false;
+  *failed = pers_refused_;
+  pers_refused_ = false;
   for (int i : launch_slots_) *failed = *failed || h_sc_[i].pers_fail;
   if (!*failed) return APHPOIS_OK;
   for (int i : launch_slots_) {

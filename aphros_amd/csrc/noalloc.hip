@@ -230,8 +230,12 @@ int solve_noalloc(const aphpois_desc* d, const double* expr, const double* x0, d
       bool restart = false;
       const unsigned tag = take_tags(d->device, 2u * iters + 2u, &restart);
       if (restart) NA_HIP(launch_fill(slots, kPersSlotBytes / 8, 8, st));
-      NA_HIP(launch_pers(method, 0, 0, plan.shape, plan.lds, L.sds, &dh->prec, b2r, plan.nblk, iters,
-                         tag, PersWait(), st));
+      if (launch_pers(method, 0, 0, plan.shape, plan.lds, L.sds, &dh->prec, b2r, plan.nblk, iters,
+                      tag, PersWait(), st) != hipSuccess) {
+        // refused by the runtime: the iteration kernels
+        (void)hipGetLastError();
+        pers = false;
+      }
     }
     for (int i = 0; i < k && !pers; ++i) {
       for (int j = 0; j < iter_kernels(method); ++j) NA_HIP(launch_kernel(method, 0, 1, L, st, j));

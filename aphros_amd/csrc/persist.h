@@ -38,6 +38,9 @@ struct PersRec {
 struct PersWait {
   long long gather = 200000000, early = 200000000;
 };
+// a wait (gather) with which launch_pers() answers as the runtime does when it
+// cannot place a cooperative launch
+constexpr long long kPersRefuse = -0x7fffffffffffffffLL - 1;
 
 // Plan of a system of method (Method), element type and size on a device of
 // ncu compute units; false: the system is not for a resident launch.
@@ -49,7 +52,7 @@ bool pers_plan(int method, int fp32, int nx, int ny, int nz, int ncu, PersPlan* 
 // record) are device arrays; tag: the launch's first tag, larger than every
 // tag the slots have seen (a launch uses fewer than 2 * iters + 2).  A system
 // whose workgroups did not meet keeps the state it had before the launch and
-// gets pers_fail = 1.
+// gets pers_fail = 1.  An error of the launch itself leaves everything as it was.
 hipError_t launch_pers(int method, int fp32, int has_m, int shape, int lds, const SysDev* sds,
                        const PersRec* recs, const int* b2r, int nblk, int iters, unsigned tag,
                        PersWait wait, hipStream_t st);

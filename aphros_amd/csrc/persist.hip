@@ -1051,6 +1051,7 @@ hipError_t coop(K kernel, int nblk, int lds, hipStream_t st, const SysDev* sds,
 hipError_t launch_pers(int method, int fp32, int has_m, int shape, int lds, const SysDev* sds,
                        const PersRec* recs, const int* b2r, int nblk, int iters, unsigned tag,
                        PersWait wait, hipStream_t st) {
+  if (wait.gather == kPersRefuse) return hipErrorCooperativeLaunchTooLarge;
 #define APH_COOP(...) return coop(__VA_ARGS__, nblk, lds, st, sds, recs, b2r, iters, tag, wait)
   if (method == kConjugate) {
     switch (shape) {

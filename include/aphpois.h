@@ -291,7 +291,7 @@ int aphpois_set_tile(aphpois* h, int lx, int bz, int vx, int sm);
  * launch per iteration kernel.  Systems of at most 2^21 cells without the
  * multigrid preconditioner run their iterations in such launches, unless
  * set_profiling or set_tile address the iteration kernels.  Negative: they
- * give up at once. */
+ * give up at once; INT64_MIN: the launch counts as refused by the runtime. */
 int aphpois_set_resident_wait(aphpois* h, long long ticks);
 /* The same with a wait of its own for the loads of neighbouring rows that start
  * ahead of the sums (early_ticks; once it has passed they follow the sums). */

@@ -226,3 +226,23 @@ def test_wait_that_lapses_in_the_last_gather(method, shape):
     if method == L.JACOBI:
         xo, ito, _, _ = O.jacobi(E, tol=0.0, miniter=0, maxiter=0)
         assert ito == 1 and np.array_equal(x, xo)
+
+
+@pytest.mark.parametrize("method", [L.CONJUGATE, L.JACOBI, L.PCG])
+def test_refused_launch(method):
+    """A resident launch that the runtime refuses is answered by the iteration
+    kernels, in this solve and the next."""
+    shape = (40, 36, 44)
+    E = _system(shape, 10)
+    kw = dict(resmode=L.RES_REL_TRUE, tol=1e-9) if method == L.PCG else \
+        dict(resmode=L.RES_L2, tol=1e-6)
+    got = []
+    for setup in (lambda s: s.set_profiling(True), lambda s: s.set_resident_wait(-2 ** 63)):
+        s = Poisson(shape, method=method, miniter=0, maxiter=2000, h3=1.0, **kw)
+        s.set_system(E)
+        setup(s)
+        got.append([s.solve(None), s.solve(None)])
+        s.close()
+    for (xk, ik), (x, i) in zip(*got):
+        assert i["converged"] == ik["converged"] == 1 and i["iter"] == ik["iter"]
+        assert np.array_equal(x, xk)
