@@ -52,8 +52,8 @@ struct System {
   int tune_lx = 0, tune_bz = 0;  // stencil tile of this system (0 = engine default)
   bool pers_ok = false;          // may run in resident launches, as pers says
   PersPlan pers{};
-  // their gather slots and, for JACOBI, a second buffer of boundary rows
-  // (outside the budget, as the reduction scratch is)
+  // their gather slots (kPersSlotBytes, outside the budget, as the reduction
+  // scratch is)
   unsigned long long* slots = nullptr;
   // multigrid levels (host copy; device copy in d_lev)
   std::vector<MgLevel> lev;

@@ -587,8 +587,7 @@ int Engine::add_system(int nx, int ny, int nz, double h3, int* slot) {
   (void)p;
   S.pers_ok = !pc_ && pers_plan(method_, fp32_, nx, ny, nz, pers_cu_, &S.pers);
   if (S.pers_ok) {
-    hipError_t e = hipMalloc((void**)&S.slots,
-                             (size_t)(kPersSlotBytes + (method_ == kJacobi ? 8 * n : 0)));
+    hipError_t e = hipMalloc((void**)&S.slots, (size_t)kPersSlotBytes);
     if (e == hipSuccess) {
       e = launch_fill(S.slots, kPersSlotBytes / 8, 8, st_);
       if (e == hipSuccess) e = hipStreamSynchronize(st_);
@@ -605,8 +604,7 @@ int Engine::add_system(int nx, int ny, int nz, double h3, int* slot) {
     } else if (method_ == kConjugate) {
       S.dev.halo[0] = S.dev.qq;
     } else {
-      S.dev.halo[0] = S.dev.u[1];
-      S.dev.halo[1] = (char*)S.slots + kPersSlotBytes;
+      S.dev.halo[0] = S.dev.u[1];  // (halo[1]: build_tables)
     }
   }
   slots_[id] = std::move(s);
@@ -670,6 +668,7 @@ int Engine::ensure_staging(long long need) {
     return hip(e, "hipMalloc (staging)");
   }
   staging_bytes_ = need;
+  if (method_ == kJacobi) dirty_ = true;  // (SysDev::halo[1])
   return APHPOIS_OK;
 }
 
@@ -951,6 +950,10 @@ int Engine::prepare(int slot, const double* x0, bool on_device, long long start,
 // system and of the measurement hooks (event timing and tile overrides address
 // the iteration kernels), so its results do not depend on its neighbours.
 bool Engine::use_pers(const System& s) const {
+  // JACOBI exchanges the rows of odd sweeps through the staging buffer, idle
+  // during a solve and large enough since set_system (an array of its own would
+  // not fit budgets that the iteration kernels meet)
+  if (method_ == kJacobi && (staging_bytes_ < 8 * s.n || launch_slots_.size() != 1)) return false;
   return s.pers_ok && !pers_off_ && !profile_ && tuning_.lx == 0 && tuning_.bz == 0 && tuning_.vx == 0 &&
          tuning_.sm == 0 && s.tune_lx == 0 && s.tune_bz == 0;
 }
@@ -1159,6 +1162,7 @@ int Engine::build_tables() {
     s.dev.nblk_sm = b.nblk;
     s.dev.nblk_ru = c.nblk;
     s.dev.pers = use_pers(s) ? 1 : 0;
+    if (method_ == kJacobi) s.dev.halo[1] = staging_;
     sds.push_back(s.dev);
   }
   // resident launches: systems of one kernel instance share a launch as long

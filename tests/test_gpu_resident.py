@@ -8,10 +8,13 @@ timing on).
 Systems: random symmetric face coefficients in [0.5, 1.5] plus a mass term of
 1, so the spectrum of A lies in [1, 19] and an error in x is at most 19 times
 the relative residual (2-norms)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from aphros_amd import _lib as L
+from aphros_amd.devmem import hip
 from aphros_amd.solver import Poisson
 from oracle import oracle as O
 
@@ -246,3 +249,33 @@ def test_refused_launch(method):
     for (xk, ik), (x, i) in zip(*got):
         assert i["converged"] == ik["converged"] == 1 and i["iter"] == ik["iter"]
         assert np.array_equal(x, xk)
+
+
+@pytest.mark.parametrize("method", [L.CONJUGATE, L.JACOBI, L.PCG])
+def test_device_memory_is_what_the_budget_counts(method):
+    """A 128^3 solver holds the bytes it reports (and a budget of these lets it
+    solve), up to scratch that does not grow with the system."""
+    shape = (128, 128, 128)
+    E = _system(shape, 11)
+    kw = dict(resmode=L.RES_REL_TRUE, tol=1e-6) if method == L.PCG else \
+        dict(resmode=L.RES_L2, tol=0.0)
+
+    def unused():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert hip().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    def solve(budget):
+        free = unused()
+        s = Poisson(shape, method=method, miniter=0, maxiter=3, h3=1.0, mem_budget=budget, **kw)
+        s.set_system(E)
+        x, info = s.solve(None)
+        used, told = free - unused(), s.device_bytes()
+        s.close()
+        return x, used, told
+    solve(0)  # (code objects and the like)
+    x, used, told = solve(0)
+    print(method, used, told, flush=True)
+    assert used <= told + (14 << 20)
+    y, _, again = solve(told)
+    assert again == told and np.array_equal(x, y)
