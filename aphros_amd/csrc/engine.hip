@@ -591,13 +591,16 @@ int Engine::add_system(int nx, int ny, int nz, double h3, int* slot) {
     if (e == hipSuccess) {
       e = launch_fill(S.slots, kPersSlotBytes / 8, 8, st_);
       if (e == hipSuccess) e = hipStreamSynchronize(st_);
+      if (e != hipSuccess) {
+        free_system(S);
+        slots_[id].reset();
+        return hip(e, "gather slots");
+      }
     } else {
+      // no memory left for them: the iteration kernels need none
+      (void)hipGetLastError();
       S.slots = nullptr;
-    }
-    if (e != hipSuccess) {
-      free_system(S);
-      slots_[id].reset();
-      return hip(e, "gather slots");
+      S.pers_ok = false;
     }
     if (method_ == kPcg) {
       S.dev.halo[0] = S.dev.q;
@@ -1207,7 +1210,13 @@ int Engine::build_tables() {
       all.insert(all.end(), prec[gi].begin(), prec[gi].end());
     }
     const size_t rbytes = all.size() * sizeof(PersRec);
-    APH_HIP(hipMalloc(&d_pers_, rbytes + map.size() * sizeof(int)));
+    if (hipMalloc(&d_pers_, rbytes + map.size() * sizeof(int)) != hipSuccess) {
+      // no memory left for the tables: the iteration kernels need none
+      (void)hipGetLastError();
+      d_pers_ = nullptr;
+      pers_off_ = true;
+      return build_tables();
+    }
     int* dmap = (int*)((char*)d_pers_ + rbytes);
     APH_HIP(hipMemcpy(d_pers_, all.data(), rbytes, hipMemcpyHostToDevice));
     APH_HIP(hipMemcpy(dmap, map.data(), map.size() * sizeof(int), hipMemcpyHostToDevice));
