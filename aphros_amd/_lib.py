@@ -126,6 +126,7 @@ SIGNATURES = {
                                       C.POINTER(C.c_int)]),
     "aphpois_set_resident_wait": (C.c_int, [_vp, _ll]),
     "aphpois_set_resident_waits": (C.c_int, [_vp, _ll, _ll]),
+    "aphpois_noalloc_set_resident_wait": (C.c_int, [C.c_int, _ll]),
     "aphpois_set_tile": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, C.c_int]),
     "aphpois_precond_apply": (C.c_int, [_vp, _dp, _dp]),
     "aphpois_copy_bandwidth": (C.c_int, [C.c_int, _ll, C.c_int, _dp]),

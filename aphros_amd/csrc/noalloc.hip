@@ -76,6 +76,10 @@ constexpr int kMaxDevices = 64;
 std::mutex g_mu;
 unsigned char* g_ptr[kMaxDevices] = {};
 unsigned g_tag[kMaxDevices] = {};  // last tag the device's gather slots have seen
+PersWait g_wait[kMaxDevices];
+// a resident launch on the device gave up or was refused: later calls start with
+// the iteration kernels rather than with another wait
+bool g_off[kMaxDevices] = {};
 
 // The first of `count` tags for the gather slots of a device; *restart: the
 // tags start over and the slots have to be cleared first.
@@ -85,6 +89,18 @@ unsigned take_tags(int device, unsigned count, bool* restart) {
   const unsigned first = *restart ? 1 : g_tag[device] + 1;
   g_tag[device] = first + count;
   return first;
+}
+
+// Whether resident launches may be tried on a device, and their wait.
+bool pers_allowed(int device, PersWait* wait) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  *wait = g_wait[device];
+  return !g_off[device];
+}
+
+void pers_failed(int device) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  g_off[device] = true;
 }
 
 // Address of `scratch` on the current device (taken once per device).
@@ -183,7 +199,9 @@ int solve_noalloc(const aphpois_desc* d, const double* expr, const double* x0, d
   h.rec[1] = rsm;
   h.rec[2] = rru;
   PersPlan plan;
-  bool pers = pers_plan(method, 0, d->nx, d->ny, d->nz, pers_units(d->device), &plan);
+  PersWait wait;
+  bool pers = pers_allowed(d->device, &wait) &&
+              pers_plan(method, 0, d->nx, d->ny, d->nz, pers_units(d->device), &plan);
   unsigned long long* slots = (unsigned long long*)(base + kOfsSlots);
   if (pers) h.prec = {0, 0, plan.nblk, plan.by, plan.bz, plan.py, slots};
 
@@ -231,9 +249,10 @@ int solve_noalloc(const aphpois_desc* d, const double* expr, const double* x0, d
       const unsigned tag = take_tags(d->device, 2u * iters + 2u, &restart);
       if (restart) NA_HIP(launch_fill(slots, kPersSlotBytes / 8, 8, st));
       if (launch_pers(method, 0, 0, plan.shape, plan.lds, L.sds, &dh->prec, b2r, plan.nblk, iters,
-                      tag, PersWait(), st) != hipSuccess) {
+                      tag, wait, st) != hipSuccess) {
         // refused by the runtime: the iteration kernels
         (void)hipGetLastError();
+        pers_failed(d->device);
         pers = false;
       }
     }
@@ -246,6 +265,7 @@ int solve_noalloc(const aphpois_desc* d, const double* expr, const double* x0, d
       // the resident launch gave up and left the state as it was
       hs.pers_fail = 0;
       NA_HIP(hipMemcpyAsync(&dh->sc, &hs, sizeof(hs), hipMemcpyHostToDevice, st));
+      pers_failed(d->device);
       pers = false;
       continue;
     }
@@ -290,5 +310,19 @@ int aphpois_solve_device_noalloc(const aphpois_desc* desc, const double* expr_de
 }
 
 long long aphpois_noalloc_max_cells(void) { return aph::kNaMaxCells; }
+
+int aphpois_noalloc_set_resident_wait(int device, long long ticks) {
+  using namespace aph;
+  if (device < 0 || device >= kMaxDevices)
+    return set_api_error(APHPOIS_EINVAL, "no such device");
+  std::lock_guard<std::mutex> lk(g_mu);
+  g_wait[device] = PersWait();
+  if (ticks != 0) {
+    g_wait[device].gather = g_wait[device].early = ticks;
+  } else {
+    g_off[device] = false;
+  }
+  return APHPOIS_OK;
+}
 
 }  // extern "C"

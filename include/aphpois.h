@@ -187,6 +187,11 @@ int aphpois_solve_device_noalloc(const aphpois_desc* desc, const double* expr_de
                                  const double* x0_dev, double* x_dev, void* stream,
                                  aphpois_info* info);
 long long aphpois_noalloc_max_cells(void);
+/* aphpois_set_resident_wait for the no-allocation solves of a device.  Once a
+ * resident launch has given up there, later calls start with one launch per
+ * iteration kernel; ticks 0 restores the default wait and lets resident launches
+ * be tried again. */
+int aphpois_noalloc_set_resident_wait(int device, long long ticks);
 
 /* Sets the reference solution that every later solve of the handle is
  * compared with (aphpois_info.max_diff): an FP64 solution of the resident
