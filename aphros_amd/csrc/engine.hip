@@ -4,6 +4,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <map>
+#include <tuple>
 
 namespace aph {
 
@@ -974,8 +976,8 @@ int Engine::advance_pers(int iters) {
       }
       pers_tag_ = 1;
     }
-    if (launch_pers(method_, fp32_, g.has_m, g.shape, g.lds, L_.sds, g.recs, g.b2r, g.nblk, iters,
-                    pers_tag_, pers_wait_, st_) != hipSuccess) {
+    if (launch_pers(method_, fp32_, g.has_m, g.shape, g.lds, L_.sds, g.recs, g.b2r, g.nblk,
+                    g.nblk > pers_cu_, iters, pers_tag_, pers_wait_, st_) != hipSuccess) {
       (void)hipGetLastError();
       pers_refused_ = true;
     }
@@ -1168,11 +1170,19 @@ int Engine::build_tables() {
     if (method_ == kJacobi) s.dev.halo[1] = staging_;
     sds.push_back(s.dev);
   }
-  // resident launches: systems of one kernel instance share a launch as long
-  // as every workgroup can have a compute unit
+  // resident launches: systems of one kernel instance share a launch as long as
+  // the device holds all of its workgroups.  One per compute unit, whatever the
+  // unit holds, lost against the iteration kernels in large batches: mixed 32^3
+  // x 96 HAVE against STREAM ms, now NOW.
   pers_groups_.clear();
   need_graph_ = false;
   std::vector<std::vector<PersRec>> prec;
+  std::map<std::tuple<int, int, int>, int> per_unit;
+  auto room = [&](int shape, int has_m, int lds) {
+    int& n = per_unit[{shape, has_m, lds}];
+    if (n == 0) n = pers_per_unit(method_, fp32_, has_m, shape, lds);
+    return n * pers_cu_;
+  };
   for (int k = 0; k < ns; ++k) {
     System& s = *slots_[launch_slots_[k]];
     if (!s.dev.pers) {
@@ -1184,7 +1194,7 @@ int Engine::build_tables() {
     for (; gi < pers_groups_.size(); ++gi) {
       const PersGroup& g = pers_groups_[gi];
       if (g.shape == s.pers.shape && g.has_m == has_m &&
-          g.nblk + s.pers.nblk <= std::min(pers_cu_, kPersMaxBlocks))
+          g.nblk + s.pers.nblk <= room(g.shape, has_m, std::max(g.lds, s.pers.lds)))
         break;
     }
     if (gi == pers_groups_.size()) {

@@ -248,8 +248,8 @@ int solve_noalloc(const aphpois_desc* d, const double* expr, const double* x0, d
       bool restart = false;
       const unsigned tag = take_tags(d->device, 2u * iters + 2u, &restart);
       if (restart) NA_HIP(launch_fill(slots, kPersSlotBytes / 8, 8, st));
-      if (launch_pers(method, 0, 0, plan.shape, plan.lds, L.sds, &dh->prec, b2r, plan.nblk, iters,
-                      tag, wait, st) != hipSuccess) {
+      if (launch_pers(method, 0, 0, plan.shape, plan.lds, L.sds, &dh->prec, b2r, plan.nblk, false,
+                      iters, tag, wait, st) != hipSuccess) {
         // refused by the runtime: the iteration kernels
         (void)hipGetLastError();
         pers_failed(d->device);

@@ -711,8 +711,9 @@ __global__ __launch_bounds__(kT) void k_pers_jacobi(const SysDev* __restrict__ s
 // conductances are read from memory in every iteration (FP64 boxes of more
 // than 8 cells per thread).  Ends early when a reliable update is due
 // (sc->ru), with the state that k_ru_accum expects.
-template <typename T, int CC, int ZC, bool HM, bool KXY>
-__global__ __launch_bounds__(kT) void k_pers_pcg(const SysDev* __restrict__ sds,
+// WG: workgroups that a compute unit is to hold, as far as registers go.
+template <typename T, int CC, int ZC, bool HM, bool KXY, int WG = 1>
+__global__ __launch_bounds__(kT, WG * kT / 256) void k_pers_pcg(const SysDev* __restrict__ sds,
                                                  const PersRec* __restrict__ recs,
                                                  const int* __restrict__ b2r, int iters,
                                                  unsigned tag, PersWait wait) {
@@ -1037,47 +1038,44 @@ bool pers_plan(int method, int fp32, int nx, int ny, int nz, int ncu, PersPlan* 
 
 namespace {
 
-template <typename K>
-hipError_t coop(K kernel, int nblk, int lds, hipStream_t st, const SysDev* sds,
-                const PersRec* recs, const int* b2r, int iters, unsigned tag, PersWait wait) {
-  void* args[] = {(void*)&sds,   (void*)&recs, (void*)&b2r,
-                  (void*)&iters, (void*)&tag,  (void*)&wait};
-  return hipLaunchCooperativeKernel((const void*)kernel, dim3(nblk), dim3(kT), args,
-                                    (unsigned)lds, st);
-}
+template <typename T>
+constexpr int kCrowd = sizeof(T) == 4 ? 2 : 1;
 
-}  // namespace
-
-hipError_t launch_pers(int method, int fp32, int has_m, int shape, int lds, const SysDev* sds,
-                       const PersRec* recs, const int* b2r, int nblk, int iters, unsigned tag,
-                       PersWait wait, hipStream_t st) {
-  if (wait.gather == kPersRefuse) return hipErrorCooperativeLaunchTooLarge;
-#define APH_COOP(...) return coop(__VA_ARGS__, nblk, lds, st, sds, recs, b2r, iters, tag, wait)
+// The kernel instance of a system; crowded: of a launch with more workgroups
+// than compute units.  Only FP32 PCG at four cells per thread has one of its
+// own, for two workgroups per unit: the others fit two with the registers they
+// take (up to 2 cells), or would spill for it.  Its 6 to 9 spilled registers cost a
+// lone 64^3 solve 4 % (4.60 -> 4.76 ms), and two per unit save a batch of eight
+// a third (19.0 -> 12.4 ms).
+const void* pers_kernel(int method, int fp32, int has_m, int shape, bool crowded) {
+#define APH_K(...) return (const void*)(__VA_ARGS__)
   if (method == kConjugate) {
     switch (shape) {
-      case 0: APH_COOP((k_pers_cg<1, 1, 7>));
-      case 1: APH_COOP((k_pers_cg<1, 2, 7>));
-      case 2: APH_COOP((k_pers_cg<1, 4, 7>));
-      case 3: APH_COOP((k_pers_cg<1, 8, 7>));
-      default: APH_COOP((k_pers_cg<2, 8, 2>));
+      case 0: APH_K(k_pers_cg<1, 1, 7>);
+      case 1: APH_K(k_pers_cg<1, 2, 7>);
+      case 2: APH_K(k_pers_cg<1, 4, 7>);
+      case 3: APH_K(k_pers_cg<1, 8, 7>);
+      default: APH_K(k_pers_cg<2, 8, 2>);
     }
   }
   if (method == kJacobi) {
     switch (shape) {
-      case 0: APH_COOP((k_pers_jacobi<1, 1, 8>));
-      case 1: APH_COOP((k_pers_jacobi<1, 2, 8>));
-      case 2: APH_COOP((k_pers_jacobi<1, 4, 8>));
-      case 3: APH_COOP((k_pers_jacobi<1, 8, 8>));
-      default: APH_COOP((k_pers_jacobi<2, 8, 4>));
+      case 0: APH_K(k_pers_jacobi<1, 1, 8>);
+      case 1: APH_K(k_pers_jacobi<1, 2, 8>);
+      case 2: APH_K(k_pers_jacobi<1, 4, 8>);
+      case 3: APH_K(k_pers_jacobi<1, 8, 8>);
+      default: APH_K(k_pers_jacobi<2, 8, 4>);
     }
   }
-#define APH_PCG(T, HM)                                                          \
-  switch (shape) {                                                              \
-    case 0: APH_COOP((k_pers_pcg<T, 1, 1, HM, true>));                          \
-    case 1: APH_COOP((k_pers_pcg<T, 1, 2, HM, true>));                          \
-    case 2: APH_COOP((k_pers_pcg<T, 1, 4, HM, true>));                          \
-    case 3: APH_COOP((k_pers_pcg<T, 1, 8, HM, true>));                          \
-    default: APH_COOP((k_pers_pcg<T, 2, 8, HM, (sizeof(T) == 4)>));             \
+#define APH_PCG(T, HM)                                                 \
+  switch (shape) {                                                     \
+    case 0: APH_K(k_pers_pcg<T, 1, 1, HM, true>);                      \
+    case 1: APH_K(k_pers_pcg<T, 1, 2, HM, true>);                      \
+    case 2:                                                            \
+      if (crowded) APH_K(k_pers_pcg<T, 1, 4, HM, true, kCrowd<T>>);    \
+      APH_K(k_pers_pcg<T, 1, 4, HM, true>);                            \
+    case 3: APH_K(k_pers_pcg<T, 1, 8, HM, true>);                      \
+    default: APH_K(k_pers_pcg<T, 2, 8, HM, (sizeof(T) == 4)>);         \
   }
   if (fp32) {
     if (has_m) {
@@ -1093,7 +1091,29 @@ hipError_t launch_pers(int method, int fp32, int has_m, int shape, int lds, cons
     }
   }
 #undef APH_PCG
-#undef APH_COOP
+#undef APH_K
+}
+
+}  // namespace
+
+int pers_per_unit(int method, int fp32, int has_m, int shape, int lds) {
+  int n = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+          &n, pers_kernel(method, fp32, has_m, shape, true), kT, (size_t)lds) != hipSuccess) {
+    (void)hipGetLastError();
+    return 1;
+  }
+  return n < 1 ? 1 : n;
+}
+
+hipError_t launch_pers(int method, int fp32, int has_m, int shape, int lds, const SysDev* sds,
+                       const PersRec* recs, const int* b2r, int nblk, bool crowded, int iters,
+                       unsigned tag, PersWait wait, hipStream_t st) {
+  if (wait.gather == kPersRefuse) return hipErrorCooperativeLaunchTooLarge;
+  void* args[] = {(void*)&sds,   (void*)&recs, (void*)&b2r,
+                  (void*)&iters, (void*)&tag,  (void*)&wait};
+  return hipLaunchCooperativeKernel(pers_kernel(method, fp32, has_m, shape, crowded), dim3(nblk),
+                                    dim3(kT), args, (unsigned)lds, st);
 }
 
 }  // namespace aph

@@ -279,3 +279,38 @@ def test_device_memory_is_what_the_budget_counts(method):
     assert used <= told + (14 << 20)
     y, _, again = solve(told)
     assert again == told and np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("mass", [False, True])
+@pytest.mark.parametrize("precision", [L.MIXED, L.FP64])
+def test_launches_with_several_workgroups_per_unit(precision, mass):
+    """A batch of more systems than compute units have workgroups for, of one to
+    four cells per thread: each as alone, bit for bit."""
+    from aphros_amd.batch import Batch
+    shapes = [(16, 16, 16), (32, 32, 32), (33, 40, 48), (64, 64, 64)]
+    es = []
+    for k, shape in enumerate(shapes):
+        e = _system(shape, 20 + k)
+        if not mass:
+            e[..., 0] = -e[..., 1:7].sum(-1)
+            e[..., 7] -= e[..., 7].mean()
+        es.append(e)
+    b = Batch(precision=precision, tol=1e-8, maxiter=5000, precond=L.PRECOND_JACOBI)
+    slots = [(b.add(es[k]), k, c) for c in range(9) for k in range(len(es))]
+    for sl, k, c in slots:  # nine right-hand sides per system
+        b.set_rhs(sl, np.roll(es[k][..., 7], c, axis=0), np.zeros(shapes[k]))
+    b.solve()
+    for k, shape in enumerate(shapes):
+        s = Poisson(shape, method=L.PCG, precision=precision, resmode=L.RES_REL_TRUE, tol=1e-8,
+                    maxiter=5000, precond=L.PRECOND_JACOBI)
+        s.set_system(es[k])
+        for sl, kk, c in slots:
+            if kk != k:
+                continue
+            s.set_rhs(np.roll(es[k][..., 7], c, axis=0))
+            x, info = s.solve(None)
+            xb, ib = b.get(sl)
+            assert info["converged"] == ib["converged"] == 1 and info["iter"] == ib["iter"]
+            assert np.array_equal(x, xb)
+        s.close()
+    b.close()
