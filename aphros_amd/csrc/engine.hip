@@ -1171,9 +1171,12 @@ int Engine::build_tables() {
     sds.push_back(s.dev);
   }
   // resident launches: systems of one kernel instance share a launch as long as
-  // the device holds all of its workgroups.  One per compute unit, whatever the
-  // unit holds, lost against the iteration kernels in large batches: mixed 32^3
-  // x 96 HAVE against STREAM ms, now NOW.
+  // the device holds all of its workgroups.  With one per compute unit, whatever
+  // the unit holds, large batches lost against the iteration kernels: ms per solve
+  // in iteration kernels / one per unit / now, mixed 32^3 x 96 15.0 / 22.0 / 14.3,
+  // 64^3 x 96 210 / 225 / 147, 16^3 x 600 12.9 / 18.9 / 10.3, FP64 16^3 x 400 9.1 /
+  // 13.2 / 8.2.  (A few stay behind: mixed 80^3 x 48 306 / 333 / 333, whose 140
+  // workgroups of 8 cells per thread leave 116 units idle, 24^3 x 300 23.8 / 24.9.)
   pers_groups_.clear();
   need_graph_ = false;
   std::vector<std::vector<PersRec>> prec;

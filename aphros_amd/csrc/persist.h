@@ -49,11 +49,12 @@ bool pers_plan(int method, int fp32, int nx, int ny, int nz, int ncu, PersPlan* 
 // Runs up to `iters` iterations of every system of recs (all of one kernel
 // instance: shape and, for PCG, has_m) in one cooperative launch of nblk
 // workgroups with `lds` bytes of dynamic LDS; crowded: nblk is more than the
-// device's compute units (at most pers_per_unit() times as many).  recs and b2r (workgroup ->
-// record) are device arrays; tag: the launch's first tag, larger than every
-// tag the slots have seen (a launch uses fewer than 2 * iters + 2).  A system
-// whose workgroups did not meet keeps the state it had before the launch and
-// gets pers_fail = 1.  An error of the launch itself leaves everything as it was.
+// device's compute units (at most pers_per_unit() times as many).  recs and b2r
+// (workgroup -> record) are device arrays; tag: the launch's first tag, larger
+// than every tag the slots have seen (a launch uses fewer than 2 * iters + 2).
+// A system whose workgroups did not meet keeps the state it had before the
+// launch and gets pers_fail = 1.  An error of the launch itself leaves
+// everything as it was.
 hipError_t launch_pers(int method, int fp32, int has_m, int shape, int lds, const SysDev* sds,
                        const PersRec* recs, const int* b2r, int nblk, bool crowded, int iters,
                        unsigned tag, PersWait wait, hipStream_t st);

@@ -1002,51 +1002,73 @@ bool pers_plan(int method, int fp32, int nx, int ny, int nz, int ncu, PersPlan* 
   // 32^3 with 16 / 32 / 64 / 128 5.9 / 5.7 / 5.5 / 6.0; PCG mixed 101 x 75 x
   // 93 with 96 / 128 / 180 / 240 14.4 / 13.1 / 11.6 / 11.6.  2^21 cells are
   // what 256 workgroups of 16 cells per thread hold.
-  double best = -1;
-  PersPlan p{};
-  for (int pz = 1; pz <= nz && pz <= nbmax; ++pz) {
-    const int bz = (nz + pz - 1) / pz;
-    if ((nz + bz - 1) / bz != pz) continue;
-    for (int py = 1; py <= ny && py * pz <= nbmax; ++py) {
-      const int by = (ny + py - 1) / py;
-      if ((ny + by - 1) / by != py) continue;
-      int shape = 0;
-      while (shape < kNumShapes &&
-             ((long long)nx * by > (long long)kShapes[shape][0] * kPersThreads ||
-              bz > kShapes[shape][1]))
-        ++shape;
-      if (shape == kNumShapes) continue;
-      const long long lds = lds_bytes(method, fp32, nx, by, bz);
-      if (lds > 156 * 1024) continue;
-      const int nb = py * pz;
-      const int cpt = kShapes[shape][0] * kShapes[shape][1];
-      // gathers, own cells (twice the price with two columns per thread:
-      // fewer wavefronts' worth of latency hidden per cell), halo cells
-      const double cost = 4.2 + (nb <= 64 ? 0.04 * nb : 2.56 + 0.02 * (nb - 64)) +
-                          0.4 * kShapes[shape][0] * bz * (cpt == 16 ? 2.0 : 1.0) +
-                          0.0007 * (2.0 * nx * (by + bz));
-      if (best < 0 || cost < best) {
-        best = cost;
-        p = {by, bz, py, pz, nb, shape, (int)lds};
+  auto each = [&](auto f) {
+    for (int pz = 1; pz <= nz && pz <= nbmax; ++pz) {
+      const int bz = (nz + pz - 1) / pz;
+      if ((nz + bz - 1) / bz != pz) continue;
+      for (int py = 1; py <= ny && py * pz <= nbmax; ++py) {
+        const int by = (ny + py - 1) / py;
+        if ((ny + by - 1) / by != py) continue;
+        int shape = 0;
+        while (shape < kNumShapes &&
+               ((long long)nx * by > (long long)kShapes[shape][0] * kPersThreads ||
+                bz > kShapes[shape][1]))
+          ++shape;
+        if (shape == kNumShapes) continue;
+        const long long lds = lds_bytes(method, fp32, nx, by, bz);
+        if (lds > 156 * 1024) continue;
+        const int nb = py * pz;
+        const int cpt = kShapes[shape][0] * kShapes[shape][1];
+        // gathers, own cells (twice the price with two columns per thread:
+        // fewer wavefronts' worth of latency hidden per cell), halo cells
+        const double cost = 4.2 + (nb <= 64 ? 0.04 * nb : 2.56 + 0.02 * (nb - 64)) +
+                            0.4 * kShapes[shape][0] * bz * (cpt == 16 ? 2.0 : 1.0) +
+                            0.0007 * (2.0 * nx * (by + bz));
+        f(cost, PersPlan{by, bz, py, pz, nb, shape, (int)lds});
       }
     }
-  }
+  };
+  double best = -1;
+  each([&](double cost, const PersPlan& p) {
+    if (best < 0 || cost < best) {
+      best = cost;
+      *out = p;
+    }
+  });
   if (best < 0) return false;
-  *out = p;
+  // PCG systems come in batches, whose launches hold more of them the fewer
+  // workgroups each takes.  Up to 2^13 cells the fewest within 2 % of the best
+  // (16^3 with 16 / 8 alone 0.97 / 0.98 ms, 400 in a batch mixed 12.9 / 7.2, FP64
+  // 13.2 / 8.2); above, half the device's within 2.5 % (mixed 72^3 with 132 / 121
+  // alone 5.73 / 5.86 ms, 24 in a batch 133 / 71).
+  if (method != kPcg) return true;
+  if (n <= (1LL << 13)) {
+    double bc = best;
+    each([&](double cost, const PersPlan& p) {
+      if (cost > 1.02 * best || p.nblk > out->nblk || (p.nblk == out->nblk && cost >= bc)) return;
+      bc = cost;
+      *out = p;
+    });
+  } else if (out->nblk > nbmax / 2) {
+    double bc = 1.025 * best;
+    each([&](double cost, const PersPlan& p) {
+      if (p.nblk > nbmax / 2 || cost > bc) return;
+      bc = cost;
+      *out = p;
+    });
+  }
   return true;
 }
 
 namespace {
 
-template <typename T>
-constexpr int kCrowd = sizeof(T) == 4 ? 2 : 1;
-
 // The kernel instance of a system; crowded: of a launch with more workgroups
-// than compute units.  Only FP32 PCG at four cells per thread has one of its
-// own, for two workgroups per unit: the others fit two with the registers they
-// take (up to 2 cells), or would spill for it.  Its 6 to 9 spilled registers cost a
-// lone 64^3 solve 4 % (4.60 -> 4.76 ms), and two per unit save a batch of eight
-// a third (19.0 -> 12.4 ms).
+// than compute units.  PCG at 4 cells per thread in FP32 and 2 in FP64 then has
+// an instance of its own with the registers that let a unit hold two
+// workgroups (fewer cells fit two anyway; mixed at 8 cells would spill 300 and
+// more, 80^3 x 24 166 -> 178 ms).  The registers it spills cost a lone solve
+// (mixed 64^3 4.60 -> 4.76 ms), two workgroups per unit shorten a batch: mixed
+// 64^3 x 96 225 -> 147 ms, FP64 24^3 x 200 27.1 -> 19.3, 32^3 x 96 22.9 -> 17.0.
 const void* pers_kernel(int method, int fp32, int has_m, int shape, bool crowded) {
 #define APH_K(...) return (const void*)(__VA_ARGS__)
   if (method == kConjugate) {
@@ -1070,9 +1092,11 @@ const void* pers_kernel(int method, int fp32, int has_m, int shape, bool crowded
 #define APH_PCG(T, HM)                                                 \
   switch (shape) {                                                     \
     case 0: APH_K(k_pers_pcg<T, 1, 1, HM, true>);                      \
-    case 1: APH_K(k_pers_pcg<T, 1, 2, HM, true>);                      \
+    case 1:                                                            \
+      if (crowded) APH_K(k_pers_pcg<T, 1, 2, HM, true, 2>);            \
+      APH_K(k_pers_pcg<T, 1, 2, HM, true>);                            \
     case 2:                                                            \
-      if (crowded) APH_K(k_pers_pcg<T, 1, 4, HM, true, kCrowd<T>>);    \
+      if (crowded) APH_K(k_pers_pcg<T, 1, 4, HM, true, (sizeof(T) == 4 ? 2 : 1)>);  \
       APH_K(k_pers_pcg<T, 1, 4, HM, true>);                            \
     case 3: APH_K(k_pers_pcg<T, 1, 8, HM, true>);                      \
     default: APH_K(k_pers_pcg<T, 2, 8, HM, (sizeof(T) == 4)>);         \
