@@ -213,3 +213,32 @@ def test_breakdown_ends_the_solve(shape, precision):
     xo, io = own.solve(None)
     own.close()
     assert info["iter"] == io["iter"] and np.array_equal(x, xo)
+
+
+@pytest.mark.parametrize("precision", [L.MIXED, L.FP64])
+@pytest.mark.parametrize("shape", [
+    (16, 40, 288),    # 72 / 144 columns
+    (48, 40, 160),    # 40 / 80 columns
+    (16, 24, 104),    # 26 / 52 columns
+    (20, 18, 77),     # 77 columns of one cell
+])
+def test_row_tiles_of_the_jacobi_scaled_operator(shape, precision):
+    """The same tiles in the Jacobi-scaled operator and update, which systems of
+    these sizes launch only with event timing on: the resident solve's iterations
+    and solution."""
+    e = _system(shape, 9, True)
+    got = []
+    for timed in (False, True):
+        s = Poisson(shape, method=L.PCG, precision=precision, resmode=L.RES_REL_TRUE, tol=1e-10,
+                    maxiter=5000, precond=L.PRECOND_JACOBI)
+        s.set_system(e)
+        s.set_profiling(timed)
+        x, info = s.solve(None)
+        s.close()
+        assert info["converged"] == 1
+        assert O.true_relres(e, x) <= 1e-10 * (1 + 1e-6)
+        got.append((x, info["iter"]))
+    (x, i), (xk, ik) = got
+    err = np.linalg.norm((x - xk).ravel()) / np.linalg.norm(x.ravel())
+    print(shape, precision, i, ik, err, flush=True)
+    assert abs(i - ik) <= max(1, i // 50)
