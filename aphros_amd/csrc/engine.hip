@@ -1052,7 +1052,7 @@ int Engine::build_tables() {
     }
   }
   // post-smoothing per level: fused for the systems whose level says so
-  L_.any_mid = L_.any_plain = 0;
+  L_.any_mid = 0;
   int post_fused[kMaxLevels] = {}, post_plain[kMaxLevels] = {}, post_tile[kMaxLevels] = {};
   std::vector<std::vector<Rec>> rlt(kMaxLevels), rlp[kFuseKinds];
   std::vector<std::vector<int>> blt(kMaxLevels), blp[kFuseKinds];
@@ -1149,7 +1149,7 @@ int Engine::build_tables() {
     // partials: 3 values per block of the largest reducing launch of this
     // system; lean: 4 (operator) + 1 (x64) + 3 (residual) + 1 ((r, z)), apart
     const long long nmax = std::max(std::max(a.nblk, nblk_pc), std::max(b.nblk, c.nblk));
-    s.dev.lean = !pc_ || s.dev.mg_lb == 0 ? 0 : (s.n <= kLeanCells ? 1 : 2);
+    s.dev.lean = !pc_ ? 0 : (s.n <= kLeanCells ? 1 : 2);
     const long long need = (s.dev.lean ? 9 : 3) * nmax * 8;
     if (need > s.partials_cap) {
       if (s.partials) APH_HIP(hipFree(s.partials));
@@ -1162,7 +1162,7 @@ int Engine::build_tables() {
     s.dev.pacc = s.dev.partials + (s.dev.lean ? 4 * nmax : 0);
     s.dev.pres = s.dev.partials + (s.dev.lean ? 5 * nmax : 0);
     s.dev.ppc = s.dev.partials + (s.dev.lean ? 8 * nmax : 0);
-    if (s.dev.lean != 1) (s.dev.lean ? L_.any_mid : L_.any_plain) = 1;
+    if (s.dev.lean == 2) L_.any_mid = 1;
     s.dev.nblk_st = a.nblk;
     s.dev.nblk_sm = b.nblk;
     s.dev.nblk_ru = c.nblk;
@@ -1381,8 +1381,7 @@ int Engine::capture() {
   const int nk = iter_kernels(method_, pc_ ? 1 : 0);
   const int ng = graph_kernels(method_, pc_ ? 1 : 0);  // of them in the graph
   // launches per iteration (the multigrid cycle counts as one kernel in nk)
-  const int nl = (L_.any_plain ? ng + (pc_ ? 1 : 0) : (L_.any_mid ? 6 : 4)) +
-                 (pc_ ? vcycle_launches(L_) - 2 : 0);
+  const int nl = pc_ ? (L_.any_mid ? 6 : 4) + vcycle_launches(L_) - 2 : ng;
   int k = check_every_;
   if (k <= 0) {
     // about 4 ms of work per replay (iterations past convergence cost a

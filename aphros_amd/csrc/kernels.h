@@ -41,9 +41,9 @@ struct LaunchSet {
   int deep = 0;  // largest bottom level over the systems (no launches below)
   int bottom_at[kMaxLevels] = {};  // some system's bottom kernel starts here
   int start_only = 0;  // cycle launches for newly prepared systems only
-  int any_mid = 0, any_plain = 1;  // systems with SysDev::lean 2, 0
-  // the host may rebuild the tables after this cycle: (r, z) of lean systems
-  // is summed up now (every cycle but those inside a captured sequence)
+  int any_mid = 0;  // systems with SysDev::lean 2
+  // the host may rebuild the tables after this cycle: (r, z) is summed up now
+  // (every cycle but those inside a captured sequence)
   int close = 1;
   int coarse_sweeps = kCoarseSweeps;
   int coarse_lds = 0;  // dynamic LDS bytes of the bottom-levels kernel

@@ -239,14 +239,14 @@ __device__ __forceinline__ Tile tile_of(const Rec& rc, const SysDev& s, int lb) 
 }
 
 // ===========================================================================
-// Lean systems (SysDev::lean: multigrid of two or more levels).  The kernel
-// after a reducing one sums its partials itself, every workgroup the same way,
-// and workgroup 0 stores what the iteration keeps; no field is stored by a
-// kernel whose other workgroups still need the value before (hence `end` beside
-// `done`: a workgroup of which only some wavefronts see `done` would sum up
-// what the others never wrote).  The operator also forms (r, r),
-// (r, q) and (q, q), so the update knows |r - alpha q|^2, and with it whether a
-// reliable update follows, before it touches r.  Six of an iteration's launches
+// Multigrid systems (SysDev::lean; two or more levels).  The kernel after a
+// reducing one sums its partials itself, every workgroup the same way, and
+// workgroup 0 stores what the iteration keeps; no field is stored by a kernel
+// whose other workgroups still need the value before (hence `end` beside `done`:
+// a workgroup of which only some wavefronts see `done` would sum up what the
+// others never wrote).  The operator also forms (r, r), (r, q) and (q, q), so the
+// update knows |r - alpha q|^2, and with it whether a reliable update follows,
+// before it touches r.  Six of an iteration's launches
 // fall away (four finalize kernels, an accumulation pass, (r, z)), which cost
 // ~4 us each while the kernels of a small system take 5 to 10 us: 64^3 63 -> 54
 // us per iteration of a solve, 32^3 46 -> 38.  The operator's and the update's
@@ -451,9 +451,9 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
   const Rec rc = en.rc;
   const SysDev& s = en.s;
   Scalars* sc = s.sc;
-  const bool lean = !SC && s.lean, dots = !SC && s.lean == 1;
-  // ru: a reliable update is pending (lean: the last one, done by now)
-  if (sc->done || (!lean && sc->ru) || s.pers) return;
+  const bool dots = !SC && s.lean == 1;
+  // ru: a reliable update is pending (multigrid: the last one, done by now)
+  if (sc->done || (SC && sc->ru) || s.pers) return;
   const int lb = b - rc.blk0;
   const Tile t = tile_of<VX>(rc, s, lb);
   const int nx = s.nx, ny = s.ny, nz = s.nz;
@@ -538,7 +538,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
       zv1 = ldv<T, VX>(r, i1);
       pv1 = ldv<T, VX>(pin, i1);
     }
-    if (lean) beta = lean_beta(s, sc, lb);
+    beta = lean_beta(s, sc, lb);
   }
   if (t.active) {
     if constexpr (SC) {
@@ -650,7 +650,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_spmv(const Ent* __restrict__ ent
 __global__ __launch_bounds__(kBlock) void k_fin_pcg_spmv(const SysDev* __restrict__ sds) {
   const SysDev& s = sds[blockIdx.x];
   Scalars* sc = s.sc;
-  if (s.lean || sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
+  if (sc->done || sc->ru || s.pers) return;  // ru: a reliable update is pending
   double acc[1];
   reduce_partials<1, 0u>(acc, s.partials, s.nblk_st);
   if (threadIdx.x == 0) {
@@ -800,11 +800,10 @@ __global__ __launch_bounds__(kBlock) void k_ru_accum(const Ent* __restrict__ ent
   block_partial<1, 0u>(acc, s.pacc, rc.nblk, lb);
 }
 
-__global__ __launch_bounds__(kBlock) void k_fin_ru_accum(const SysDev* __restrict__ sds, int so) {
+__global__ __launch_bounds__(kBlock) void k_fin_ru_accum(const SysDev* __restrict__ sds) {
   const SysDev& s = sds[blockIdx.x];
   Scalars* sc = s.sc;
-  if (s.lean || sc->done || !sc->ru) return;
-  if (so && sc->pc && !sc->first) return;
+  if (sc->done || !sc->ru) return;
   double acc[1] = {0.0};  // a zero start's sum (k_ru_accum wrote no partials)
   if (!sc->zero_start) reduce_partials<1, 0u>(acc, s.pacc, s.nblk_sm);
   if (threadIdx.x == 0) {
@@ -1052,11 +1051,10 @@ __global__ __launch_bounds__(kBlock) void k_ru_resid2(const Ent* __restrict__ en
   block_partial<3, 4u>(acc, s.pres, rc.nblk, lb);
 }
 
-__global__ __launch_bounds__(kBlock) void k_fin_ru_resid(const SysDev* __restrict__ sds, int so) {
+__global__ __launch_bounds__(kBlock) void k_fin_ru_resid(const SysDev* __restrict__ sds) {
   const SysDev& s = sds[blockIdx.x];
   Scalars* sc = s.sc;
-  if (s.lean || sc->done || !sc->ru) return;
-  if (so && sc->pc && !sc->first) return;
+  if (sc->done || !sc->ru) return;
   double acc[3];
   reduce_partials<3, 4u>(acc, s.pres, s.nblk_ru);
   if (threadIdx.x == 0) {
@@ -1265,7 +1263,7 @@ __global__ __launch_bounds__(kBlock) void k_mg_sweep(const Ent* __restrict__ ent
   // so: the start of newly prepared systems (first == 1); running ones skip
   if (so && !s.sc->first) return;
   if constexpr (MODE == 1 && L0) {
-    if (en.lv.post == 0 && s.lean && s.sc->ru && lean_verdict<kBlock>(s, s.sc, b - rc.blk0)) return;
+    if (en.lv.post == 0 && s.sc->ru && lean_verdict<kBlock>(s, s.sc, b - rc.blk0)) return;
   }
   const MgLevel& Lv = en.lv;
   // this system's level runs fused kernels (k_mg_pre, k_mg_post) instead
@@ -1529,7 +1527,7 @@ __global__ __launch_bounds__(kTileBlock) void k_mg_tile(const Ent* __restrict__ 
   if (wl >= 0 && wl >= s.mg_w) return;
   if (so && !s.sc->first) return;
   if constexpr (PRE) {
-    if (l == 0 && s.lean && s.sc->ru && lean_verdict<kTileBlock>(s, s.sc, b - rc.blk0)) return;
+    if (l == 0 && s.sc->ru && lean_verdict<kTileBlock>(s, s.sc, b - rc.blk0)) return;
   }
   const MgLevel& Lv = en.lv;
   const MgLevel& Lc = en.lc;
@@ -2121,7 +2119,7 @@ __global__ __launch_bounds__(NT, 4) void k_mg_pre(const Ent* __restrict__ ents,
   if (wl >= 0 && wl >= s.mg_w) return;
   if (so && !s.sc->first) return;
   if constexpr (L0) {
-    if (s.lean && s.sc->ru && lean_verdict<NT>(s, s.sc, b - rc.blk0)) return;
+    if (s.sc->ru && lean_verdict<NT>(s, s.sc, b - rc.blk0)) return;
   }
   const MgLevel Lv = cload(&en->lv);
   const MgLevel Lc = cload(&en->lc);
@@ -2319,7 +2317,7 @@ __global__ __launch_bounds__(NT, 4) void k_mg_pre4(const Ent* __restrict__ ents,
   if (wl >= 0 && wl >= s.mg_w) return;
   if (so && !s.sc->first) return;
   if constexpr (L0) {
-    if (s.lean && s.sc->ru && lean_verdict<NT>(s, s.sc, b - rc.blk0)) return;
+    if (s.sc->ru && lean_verdict<NT>(s, s.sc, b - rc.blk0)) return;
   }
   const MgLevel Lv = cload(&en->lv);
   const MgLevel Lc = cload(&en->lc);
@@ -3002,26 +3000,19 @@ __global__ __launch_bounds__(kBottomThreads) void k_mg_bottom(const SysDev* __re
   bottom_levels<T, NV, false>(s, l0, sweeps, a0, out);
 }
 
-// (r, z) of the preconditioned CG: beta = (r,z) / (r,z)_old (0 after a start)
+// (r, z) of the preconditioned CG
 __global__ __launch_bounds__(kBlock) void k_fin_precond(const SysDev* __restrict__ sds,
-                                                        int so, int close) {
+                                                        int so) {
   const SysDev& s = sds[blockIdx.x];
   Scalars* sc = s.sc;
   if (s.nlev <= 0 || sc->done) return;
   if (so && !sc->first) return;
-  if (s.lean && !close) return;
   double acc[1];
   reduce_partials<1, 0u>(acc, s.ppc, s.nblk_pc);
   if (threadIdx.x == 0) {
     const double rz = acc[0];
     sc->rz = rz;
-    if (s.lean) {
-      sc->rz_ok = 1;
-    } else {
-      sc->beta = sc->first ? 0.0 : rz / sc->rho;
-      sc->rho = rz;
-      sc->first = 0;
-    }
+    sc->rz_ok = 1;
     if (!isfinite(rz)) {
       sc->status = 6;
       sc->done = 1;
@@ -3844,7 +3835,7 @@ static int launch_vcycle(const LaunchSet& L, hipStream_t st, hipEvent_t* ev = nu
   };
   launch_cycle<T>(L, st, 0, -1, false, mark);
   mark(4);
-  if (L.any_plain || L.close) APH_LAUNCH(k_fin_precond, L.ns, st, L.sds, L.start_only, L.close);
+  if (L.close) APH_LAUNCH(k_fin_precond, L.ns, st, L.sds, L.start_only);
   if (ev) (void)hipEventRecord(ev[k], st);
   return k;
 }
@@ -3898,27 +3889,27 @@ static void launch_pcg_kernel(const LaunchSet& L, hipStream_t st, int j) {
       break;
     case 8: launch_vcycle<T>(L, st); break;
     case 1:
-      if (L.any_plain) APH_LAUNCH(k_fin_pcg_spmv, L.ns, st, L.sds);
+      if (!L.pc) APH_LAUNCH(k_fin_pcg_spmv, L.ns, st, L.sds);
       break;
     case 2:
       APH_LAUNCH((k_pcg_update<T, VX>), L.nsm, st, L.ent_sm, L.b2r_sm);
       break;
     case 3:
-      if (L.any_plain || L.any_mid) APH_LAUNCH(k_fin_pcg_update, L.ns, st, L.sds);
+      if (!L.pc || L.any_mid) APH_LAUNCH(k_fin_pcg_update, L.ns, st, L.sds);
       break;
     case 4:
-      if (L.any_plain || L.any_mid || L.start_only)
+      if (!L.pc || L.any_mid || L.start_only)
         APH_LAUNCH((k_ru_accum<T, VX>), L.nsm, st, L.ent_sm, L.b2r_sm, L.start_only);
       break;
     case 5:
-      if (L.any_plain) APH_LAUNCH(k_fin_ru_accum, L.ns, st, L.sds, L.start_only);
+      if (!L.pc) APH_LAUNCH(k_fin_ru_accum, L.ns, st, L.sds);
       break;
     case 6:
       if (L.vx_ru == 2) APH_LAUNCH(k_ru_resid2<T>, L.nru, st, L.ent_ru, L.b2r_ru, L.start_only);
       else APH_LAUNCH((k_ru_resid<T, 1>), L.nru, st, L.ent_ru, L.b2r_ru, L.start_only);
       break;
     default:
-      if (L.any_plain) APH_LAUNCH(k_fin_ru_resid, L.ns, st, L.sds, L.start_only);
+      if (!L.pc) APH_LAUNCH(k_fin_ru_resid, L.ns, st, L.sds);
       break;
   }
 }
