@@ -314,3 +314,30 @@ def test_launches_with_several_workgroups_per_unit(precision, mass):
             assert np.array_equal(x, xb)
         s.close()
     b.close()
+
+
+@pytest.mark.parametrize("method", [L.CONJUGATE, L.JACOBI, L.PCG])
+def test_guess_with_wide_strides(method):
+    """A guess whose strided range exceeds what set_system staged (the buffer moves
+    between the table's set-up and the solve), in place: as the dense guess, bit
+    for bit."""
+    shape = (6, 5, 7)
+    nz, ny, nx = shape
+    E = _system(shape, 12)
+    kw = dict(resmode=L.RES_REL_TRUE, tol=1e-10) if method == L.PCG else \
+        dict(resmode=L.RES_L2, tol=0.0, maxiter=6)
+    s = Poisson(shape, method=method, miniter=0, h3=1.0, **kw)
+    s.set_system(E)
+    x0 = np.random.default_rng(1).standard_normal(shape)
+    s.solve(None)
+    ly, lz, start = 130, 2600, 55
+    wide = np.full(start + nz * lz, 7.0)
+    inner = np.lib.stride_tricks.as_strided(wide[start:], shape, (8 * lz, 8 * ly, 8))
+    inner[...] = x0
+    info = L.Info()
+    L.check(L.lib().aphpois_solve(s.h, L.dptr(wide), L.dptr(wide), start, ly, lz, C.byref(info)))
+    x, dense = s.solve(x0)
+    s.close()
+    assert info.iter == dense["iter"] and np.array_equal(inner, x)
+    inner[...] = 7.0
+    assert np.all(wide == 7.0)
