@@ -22,12 +22,13 @@
 // gather that its readers reach after reading it.
 //
 // Microseconds per iteration, iteration kernels in graph replays -> resident:
-// reference CG 64^3 31.0 -> 7.2; reference Jacobi 60 x 45 x 52 16.4 -> 4.6;
-// PCG mixed 101 x 75 x 93 46 -> 11.6, FP64 128^3 52.9 -> 21.8 (mixed 128^3
-// 16.9).  What bounds an iteration now is its two gathers and the halo load
-// behind one of them (5 us with 16 workgroups, 8 us with 256), then the
-// stencil's LDS reads (0.35 us per cell and thread); at 16 cells per thread in
-// FP64 also the x and y conductances read from the caches.
+// reference CG 64^3 31.0 -> 6.4; reference Jacobi 60 x 45 x 52 16.4 -> 4.7;
+// PCG mixed 101 x 75 x 93 46 -> 10.5 (with a mass term 11.1), FP64 128^3 52.9 ->
+// 22 (mixed 128^3 14).  What bounds an iteration is waiting, 70 to 78 % of the
+// wavefronts' time by counters: its two gathers and the halo rows behind one of
+// them; then the stencil's LDS reads (0.35 us per cell and thread); at 16 cells
+// per thread in FP64 also the x and y conductances, read again in every
+// iteration (67 MB at 128^3, 3.4 TB/s).
 //
 // Every workgroup sums the partials in the same order, so all of them hold
 // the same scalars and take the same branches, and the result depends neither
