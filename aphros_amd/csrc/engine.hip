@@ -1096,8 +1096,11 @@ int Engine::build_tables() {
         // bound): short marches over more workgroups
         const long long ftgt = F.n >= (1LL << 21) ? std::min(1024LL, cdiv(F.n, 2048))
                                                   : std::max(1LL, cdiv(F.n, 512));
-        // level 0 follows the system's stencil tuning (autotuner / set_tile)
-        Rec f = make_stencil_rec(F.nx, F.ny, F.nz, vxl[l], ftgt, l == 0 ? tu : none, 64, 1024, true);
+        // level 0 follows the system's stencil tuning (autotuner / set_tile), with
+        // two rows or more: the fused restriction pairs rows inside one workgroup
+        Tuning tl = l == 0 ? tu : none;
+        tl.lx = std::min(tl.lx, kBlock / 2);
+        Rec f = make_stencil_rec(F.nx, F.ny, F.nz, vxl[l], ftgt, tl, 64, 1024, true);
         // the fused restriction sums plane pairs inside one workgroup: even
         // plane counts per tile (F.nz is even on every coarsened level)
         if (f.bz & 1) {

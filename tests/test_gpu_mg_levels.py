@@ -242,3 +242,24 @@ def test_row_tiles_of_the_jacobi_scaled_operator(shape, precision):
     err = np.linalg.norm((x - xk).ravel()) / np.linalg.norm(x.ravel())
     print(shape, precision, i, ik, err, flush=True)
     assert abs(i - ik) <= max(1, i // 50)
+
+
+@pytest.mark.parametrize("lx", [64, 128, 256])
+@pytest.mark.parametrize("precision,shape", [
+    (L.FP64, (8, 16, 264)),     # 132 columns: too long for the fused kernels
+    (L.MIXED, (16, 24, 130)),   # 65 columns of two cells
+])
+def test_tile_override_on_a_swept_level(precision, shape, lx):
+    """Rows of a tile as long as the workgroup: the restriction, which sums row
+    pairs inside a workgroup, still has two rows."""
+    e = _system(shape, 11, False)
+    s = Poisson(shape, method=L.PCG, precision=precision, resmode=L.RES_REL_TRUE, tol=1e-8,
+                maxiter=2000, precond=L.PRECOND_MG, mg_w=0)
+    s.set_system(e)
+    s.set_tile(lx=lx)
+    r = np.random.default_rng(12).standard_normal(shape)
+    r -= r.mean()
+    z = s.precond_apply(r)
+    s.close()
+    zo, nlev = O.mg_apply(e, r, bf16=precision == L.MIXED, w=0)
+    assert np.abs(z - zo).max() <= TOL[precision] * np.abs(zo).max()
