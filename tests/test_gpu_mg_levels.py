@@ -247,7 +247,7 @@ def test_row_tiles_of_the_jacobi_scaled_operator(shape, precision):
 @pytest.mark.parametrize("lx", [64, 128, 256])
 @pytest.mark.parametrize("precision,shape", [
     (L.FP64, (8, 16, 264)),     # 132 columns: too long for the fused kernels
-    (L.MIXED, (16, 24, 130)),   # 65 columns of two cells
+    (L.MIXED, (16, 16, 98)),    # 49 columns of two cells
 ])
 def test_tile_override_on_a_swept_level(precision, shape, lx):
     """Rows of a tile as long as the workgroup: the restriction, which sums row
